@@ -35,12 +35,6 @@ METRIC = "s/solve to residual 1e-6 + matvec HBM GB/s; mixed/learned vs plain FP6
 HBM_PEAK_GBPS = 8000.0
 
 
-def direct_sym(L: int, elem: int) -> bool:
-    """The direct tiles store the symmetric table layout up to order 5 (FP32)
-    / 4 (FP64) (mstm_amd/csrc/common.hpp, direct_sym)."""
-    return L <= (5 if elem == 4 else 4)
-
-
 def full_table_bytes_per_pair(L: int, elem: int) -> int:
     """Full rotation + axial table of one unordered pair (equal orders L):
     sum_{n<=L}(2n+1)^2 reals + 2 sum_{|m|<=L} (L-m1+1)^2 complex."""
@@ -50,20 +44,19 @@ def full_table_bytes_per_pair(L: int, elem: int) -> int:
 
 
 def sym_counts(L: int):
-    """(rotation reals, axial complex) of the symmetric layout: blocks m >= 0
-    only; half-sum/half-difference Wigner rows (n+1 values per degree for
-    m = 0, 2n+1 for m > 0) and one axial block per mode (one for m = 0)."""
-    rot = sum((n + 1) if m == 0 else (2 * n + 1) for m in range(0, L + 1) for n in range(max(1, m), L + 1))
-    ax = sum((1 if m == 0 else 2) * (L - max(1, m) + 1) ** 2 for m in range(0, L + 1))
+    """(rotation reals, axial complex) the direct tiles store per pair
+    (mstm_amd/csrc/common.hpp): triangles of the half-sum and half-difference
+    Wigner matrices, (n+1)^2 values of degree n, and of the axial blocks
+    m >= 0, one per mode (one for m = 0)."""
+    rot = sum((n + 1) ** 2 for n in range(1, L + 1))
+    ax = sum((1 if m == 0 else 2) * (L - max(1, m) + 1) * (L - max(1, m) + 2) // 2 for m in range(0, L + 1))
     return rot, ax
 
 
 def table_bytes_per_pair(L: int, elem: int) -> int:
     """Table bytes of one unordered pair as the direct tiles store them."""
-    if direct_sym(L, elem):
-        rot, ax = sym_counts(L)
-        return rot * elem + ax * 2 * elem
-    return full_table_bytes_per_pair(L, elem)
+    rot, ax = sym_counts(L)
+    return rot * elem + ax * 2 * elem
 
 
 def full_tile_flops_per_pair(L: int, nrhs: int = 2) -> int:
@@ -74,14 +67,11 @@ def full_tile_flops_per_pair(L: int, nrhs: int = 2) -> int:
     return 2 * nrhs * 16 * (s_rot + s_ax)
 
 
-def tile_flops_per_pair(L: int, nrhs: int = 2, elem: int = 4) -> int:
+def tile_flops_per_pair(L: int, nrhs: int = 2) -> int:
     """Flops the direct tiles execute for both directions of one pair and
-    nrhs columns: the symmetric rotations need R = sum of the stored row
-    lengths multiply-adds per rotation instead of S_rot; axial work is
-    unchanged: 16 (R + S_ax) per direction and column."""
-    if not direct_sym(L, elem):
-        return full_tile_flops_per_pair(L, nrhs)
-    rot, _ = sym_counts(L)
+    nrhs columns: the half-sum/half-difference rotations need (n+1)^2 + n^2
+    multiply-adds of degree n instead of (2n+1)^2; axial work is unchanged."""
+    rot = sum((n + 1) ** 2 + n ** 2 for n in range(1, L + 1))
     s_ax = sum((L - max(1, abs(m)) + 1) ** 2 for m in range(-L, L + 1))
     return 2 * nrhs * 16 * (rot + s_ax)
 
@@ -635,7 +625,7 @@ def main():
         rec = json.load(open(pmc)).get("by_columns", {}).get(str(ncol))
         traffic = rec["hbm_bytes_per_launch"] if rec else None
     fl32 = npairs * full_tile_flops_per_pair(L, ncol)
-    ex32 = npairs * tile_flops_per_pair(L, ncol, 4)
+    ex32 = npairs * tile_flops_per_pair(L, ncol)
     roof = dict(kernel=f"direct_tile_kernel<float,{L},{ncol}>", bound="hbm", achieved=round(ach32, 1),
                 peak=HBM_PEAK_GBPS, unit="GB/s", frac=round(ach32 / HBM_PEAK_GBPS, 4), traffic=traffic,
                 algorithmic_bytes=alg32, columns=ncol, avg_launch_ms=round(t32, 4),
@@ -646,8 +636,8 @@ def main():
                 note=("algorithmic bytes and flops per launch = the per-pair minimal table "
                       f"({full_table_bytes_per_pair(L, 4)} B at order {L} in FP32) and full-rotation flops "
                       "16 (S_rot + S_ax) per pair, direction and column, times the unordered pairs, plus the "
-                      "vectors; the kernel stores and reads the symmetric half-table (stored_bytes: blocks "
-                      "m >= 0, half-sum/half-difference Wigner rows, one axial block per mode), staged in LDS "
+                      "vectors; the kernel stores and reads triangles of symmetric matrices (stored_bytes: blocks "
+                      "m >= 0, half-sum/half-difference Wigner matrices, one axial block per mode), staged in LDS "
                       "once per tile step, and executes executed_flops; traffic is the measured HBM bytes; "
                       "packed FP32 is disabled, so the FP32 vector peak is 78.6 TF/s"))
     matvec = dict(fp32_tile_ms=round(t32, 4), fp32_columns=ncol, fp32_hbm_GBps=round(ach32, 1))

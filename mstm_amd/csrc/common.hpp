@@ -98,63 +98,83 @@ MSTM_HD constexpr int nmblocks(int LT, int LS) { return 2 * imn(LT, LS) + 1; }
 MSTM_HD constexpr int phi_off(int LT, int LS, int VW) { return sec_off(nmblocks(LT, LS), LT, LS, VW); }
 MSTM_HD constexpr int slot_len(int LT, int LS, int VW) { return phi_off(LT, LS, VW) + VW; }
 // ---------------------------------------------------------------------------
-// Symmetric pair-table layout of the direct tiles (LT = LS = L).  Two
-// symmetries halve the table:
-//   d^n(-m,-k) = (-1)^{m+k} d^n(m,k)      (Wigner d)
-//   A_{-m}(t,s) of mode p = A_m(t,s) of the other mode (axial coefficients;
-//   for m = 0 both modes coincide).
-// Only blocks m = 0..L are stored:
-//   ROT  degree by degree, n = 1..L; degree n holds the rows of blocks
-//        m = 0..n: the half-sum and half-difference rows
-//          E(n,0) = d^n(m,0),  E(n,k) = (d^n(m,k) + (-1)^k d^n(m,-k)) / 2,
-//          O(n,k) = (d^n(m,k) - (-1)^k d^n(m,-k)) / 2        (k = 1..n)
-//        stored E(n,0..n) then O(n,1..n); for m = 0 only E (= d^n(0,k));
-//        the section is padded once, to VW reals
-//   AX   per block m = 0..L: A_m(t,s), t fastest, for mode 0 and (m > 0)
-//        mode 1, each padded to VW reals
-// then PHI (cos, sin).  With u_k = x_k + (-1)^k x_{-k},
-// v_k = x_k - (-1)^k x_{-k} (k > 0), u_0 = x_0, the rotation
-// y_m = sum_k d(m,k) x_k of blocks m and -m becomes
-//   Y+ = sum_{k>=0} E_k u_k,  Y- = sum_{k>0} O_k v_k,
-//   y_m = Y+ + Y-,  y_{-m} = (-1)^m (Y+ - Y-)
-// and the back rotation accumulates P_k = sum E_k (z_m + (-1)^m z_{-m}),
-// Q_k = sum O_k (z_m - (-1)^m z_{-m}), from which U_k = P_k + Q_k,
-// U_{-k} = (-1)^k (P_k - Q_k), U_0 = P_0.  Both rotations of a degree read
-// the same contiguous rows, so a tile step runs degree by degree (forward),
-// block by block (axial), degree by degree (back).
+// Compact pair-table layout of the direct tiles (LT = LS = L).  Four
+// symmetries cut the full table to less than a third:
+//   d^n(-m,-k) = (-1)^{m+k} d^n(m,k),  d^n(k,m) = (-1)^{m+k} d^n(m,k)
+//   A_{-m}(t,s) of mode p = A_m(t,s) of the other mode (for m = 0 both modes
+//   coincide),  A_m(s,t) = (-1)^{t+s} A_m(t,s)
+// (d: Wigner d, A: axial coefficients).  Stored are, for n = 1..L,
+//   E_n(m,k) = (-1)^m (d(m,k) + (-1)^k d(m,-k)) / 2   (k = 0: (-1)^m d(m,0)),
+//   O_n(m,k) = (-1)^m (d(m,k) - (-1)^k d(m,-k)) / 2,
+// m, k = 0..n (E) and 1..n (O), and for m = 0..L the blocks
+//   B_m(t,s) = (-1)^t A_m(t,s), t, s = max(1,m)..L, of mode 0 and (m > 0) 1:
+// all symmetric matrices, so only their triangles (row <= column, column by
+// column).  With a_k = x_k + (-1)^k x_{-k}, b_k = x_k - (-1)^k x_{-k} (k > 0),
+// a_0 = x_0, a translation runs as
+//   u_k = cos(k phi) a_k + i sin(k phi) b_k,  v_k = cos b_k + i sin a_k,
+//   Y+ = E u, Y- = O v (degree by degree);  p_m = Y+ + Y-, q_m = Y+ - Y-,
+//   z_m = B_m p_m (own mode), z'_m = B_m q_m (other mode) (block by block);
+//   P = E (z + z'), Q = O (z - z') (degree by degree; the same matrices),
+//   (a_k, b_k of the result) / 2 = (-1)^t (cos P - i sin Q, cos Q - i sin P),
+// and for k = 0 a_0 = (-1)^t P_0.  The reverse direction (translation by -r)
+// is the same sequence on (-1)^n x with the two modes exchanged, its result
+// exchanged back and multiplied by (-1)^t.
 // ---------------------------------------------------------------------------
-MSTM_HD constexpr int sdeg_len(int n) { return (n + 1) + n * (2 * n + 1); }
-MSTM_HD constexpr int sdeg_off(int n)
+MSTM_HD constexpr int ctri(int i, int j) { return i <= j ? j * (j + 1) / 2 + i : i * (i + 1) / 2 + j; }
+// rotation section: degree n holds E_n then O_n
+MSTM_HD constexpr int crot_off(int n)
 {
     int s = 0;
-    for (int q = 1; q < n; q++) s += sdeg_len(q);
+    for (int q = 1; q < n; q++) s += (q + 1) * (q + 1);
     return s;
 }
-// row of block m (0 <= m <= n) of degree n inside the ROT section
-MSTM_HD constexpr int srow_off(int m, int n) { return sdeg_off(n) + (m == 0 ? 0 : (n + 1) + (m - 1) * (2 * n + 1)); }
-MSTM_HD constexpr int srow_len(int m, int n) { return m == 0 ? n + 1 : 2 * n + 1; }
-MSTM_HD constexpr int srot_tot(int L) { return sdeg_off(L + 1); }
-MSTM_HD constexpr int sax_len(int m, int L) { return 2 * (L - imx(1, m) + 1) * (L - imx(1, m) + 1); }  // one mode
-MSTM_HD constexpr int sax_modes(int m) { return m == 0 ? 1 : 2; }
-MSTM_HD constexpr int sax_off(int m, int L, int VW)
+MSTM_HD constexpr int crot_tot(int L) { return crot_off(L + 1); }
+MSTM_HD constexpr int crot_o(int n) { return (n + 1) * (n + 2) / 2; }  // O_n after E_n
+// axial section, in complex values: blocks m = L..0 (the small ones first),
+// mode 0 then mode 1; then one more complex value (cos phi, sin phi)
+MSTM_HD constexpr int cax_blk(int m, int L) { return (L - imx(1, m) + 1) * (L - imx(1, m) + 2) / 2; }
+MSTM_HD constexpr int cax_off(int m, int p, int L)
 {
-    int o = pad_to(srot_tot(L), VW);
-    for (int q = 0; q < m; q++) o += sax_modes(q) * pad_to(sax_len(q, L), VW);
-    return o;
+    int o = 0;
+    for (int q = L; q > m; q--) o += 2 * cax_blk(q, L);
+    return o + p * cax_blk(m, L);
 }
-MSTM_HD constexpr int sphi_off(int L, int VW) { return sax_off(L + 1, L, VW); }
-MSTM_HD constexpr int sslot_len(int L, int VW) { return sphi_off(L, VW) + VW; }
-// the direct tiles use the symmetric layout, staged in LDS, up to order 5
-// (FP32) / 4 (FP64); larger orders keep the full layout, whose unstaged form
-// folds the output phase into every term and so needs no P/Q accumulators
-MSTM_HD constexpr bool direct_sym(int L, int elem)
-{
-    return L <= (elem == 4 ? 5 : 4) && (int64_t)sslot_len(L, 16 / elem) * MSTM_SLOTS * elem <= 65536;
-}
+MSTM_HD constexpr int cax_tot(int L) { return cax_off(0, 1, L); }
+// sections as stored: padded to whole 16-byte chunks, the chunks of a group's
+// MSTM_SLOTS slots side by side (ilv), so that a slot's four lanes read one
+// chunk and a wave MSTM_SLOTS consecutive ones
+MSTM_HD constexpr int crot_pad(int L, int elem) { return pad_to(crot_tot(L), 16 / elem); }
 MSTM_HD constexpr int direct_slot_len(int L, int elem)
 {
-    return direct_sym(L, elem) ? sslot_len(L, 16 / elem) : slot_len(L, L, 16 / elem);
+    return crot_pad(L, elem) + pad_to(2 * (cax_tot(L) + 1), 16 / elem);
 }
+// element number of axial value c (real part) inside a slot
+MSTM_HD constexpr int cax_elem(int c, int L, int elem) { return crot_pad(L, elem) + 2 * c; }
+// order of the (a_k, b_k) values of one mode in the direct tiles' vectors:
+// even degrees first, so that the (-1)^n of the reverse direction is a
+// compare; per degree a_0, a_1, b_1, a_2, b_2, ...
+MSTM_HD constexpr int cvec_even(int L)
+{
+    int s = 0;
+    for (int q = 2; q <= L; q += 2) s += 2 * q + 1;
+    return s;
+}
+MSTM_HD constexpr int cvec_deg(int n, int L)
+{
+    int s = (n & 1) ? cvec_even(L) : 0;
+    for (int q = (n & 1) ? 1 : 2; q < n; q += 2) s += 2 * q + 1;
+    return s;
+}
+MSTM_HD constexpr int cvec(int n, int k, int b, int L) { return cvec_deg(n, L) + (k ? 2 * k - 1 + b : 0); }
+// complex values per unit of the direct tiles' vectors: 16 bytes (8 where a
+// column of an odd order's FP32 values is no whole number of 16-byte units)
+MSTM_HD constexpr int cvec_unit(int L, int elem) { return elem == 8 || (L & 1) ? 1 : 2; }
+
+// columns per workgroup of a four-column product of the direct tiles: all
+// four in one workgroup of four waves, or (FP64, and FP32 above order 4)
+// two workgroups of two, the staged sources of four columns leaving one
+// workgroup per CU
+MSTM_HD constexpr int tile_cols4(int L, int elem) { return elem == 4 && L <= 4 ? 4 : 2; }
 
 // interleaved position of element e (multiple-of-VW chunks) of slot k
 MSTM_HD constexpr int64_t ilv(int64_t e, int k, int VW) { return ((e / VW) * MSTM_SLOTS + k) * VW + e % VW; }

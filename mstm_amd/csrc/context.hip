@@ -591,7 +591,7 @@ static int direct_alloc(mstm_hip_ctx *c, int prec)
     DirectOp &d = c->dop[prec];
     const int L = c->Lmax;
     const size_t esz = prec == MSTM_HIP_FP64 ? sizeof(double) : sizeof(float);
-    size_t slot = (size_t)direct_slot_len(L, (int)esz);  // symmetric layout up to order 5 / 4
+    size_t slot = (size_t)direct_slot_len(L, (int)esz);
     d.tab_bytes = (size_t)c->ntiles * MSTM_SLOTS * MSTM_SLOTS * slot * esz;
     size_t nbp = (size_t)L * (L + 2);
     HIPCHK(dalloc(&d.tab, d.tab_bytes));
@@ -712,10 +712,9 @@ static int direct_matvec_buf(mstm_hip_ctx *c, int nrhs, const double *ain, doubl
     DirectOp &d = c->dop[prec];
     if (nrhs < 1 || nrhs > 4) return fail(c, MSTM_HIP_EARG, "direct product: %d columns", nrhs);
     const int L = c->Lmax, nr = nrhs > 2 ? 4 : 2;
-    // FP64 four-column products of order <= 4 run two workgroups per tile
-    // (step group): fewer step groups keep that launch within the same 512
-    // workgroups
-    if (prec == MSTM_HIP_FP64 && nr == 4 && L <= 4)
+    // four-column products that run two workgroups per tile (step group):
+    // fewer step groups keep the launch within the same 512 workgroups
+    if (nr == 4 && tile_cols4(L, prec == MSTM_HIP_FP64 ? 8 : 4) == 2)
         while (G > 1 && (int64_t)c->ntiles * G * 2 > 512) G /= 2;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (c->timing) {
@@ -724,22 +723,22 @@ static int direct_matvec_buf(mstm_hip_ctx *c, int nrhs, const double *ain, doubl
     }
     const int *gate = c->gate;
     if (prec == MSTM_HIP_FP64) {
-        HIPCHK(launch_prep<double>(ain, 2 * c->neqns, (double *)xin, nrhs, flags, c->nsph, c->npad, L, c->d_order,
+        HIPCHK(launch_prep_quad<double>(ain, 2 * c->neqns, (double *)xin, nrhs, flags, c->nsph, c->npad, L, c->d_order,
                                    c->d_offset, c->d_an, c->st, gate));
         if (e0) hipEventRecord(e0, c->st);
         HIPCHK(launch_direct_tiles<double>((const double *)d.tab, c->d_tiles, c->ntiles, L, (const double *)xin,
                                            (double *)part, c->npad, nr, G, c->st, gate));
         if (e1) hipEventRecord(e1, c->st);
-        HIPCHK(launch_reduce_post<double>((const double *)part, c->nblocks * G, aout, 2 * c->neqns, nrhs, flags, c->nsph,
+        HIPCHK(launch_reduce_quad<double>((const double *)part, c->nblocks * G, aout, 2 * c->neqns, nrhs, flags, c->nsph,
                                           c->npad, L, c->d_order, c->d_offset, c->d_an, c->st, gate));
     } else {
-        HIPCHK(launch_prep<float>(ain, 2 * c->neqns, (float *)xin, nrhs, flags, c->nsph, c->npad, L, c->d_order,
+        HIPCHK(launch_prep_quad<float>(ain, 2 * c->neqns, (float *)xin, nrhs, flags, c->nsph, c->npad, L, c->d_order,
                                   c->d_offset, c->d_an, c->st, gate));
         if (e0) hipEventRecord(e0, c->st);
         HIPCHK(launch_direct_tiles<float>((const float *)d.tab, c->d_tiles, c->ntiles, L, (const float *)xin,
                                           (float *)part, c->npad, nr, G, c->st, gate));
         if (e1) hipEventRecord(e1, c->st);
-        HIPCHK(launch_reduce_post<float>((const float *)part, c->nblocks * G, aout, 2 * c->neqns, nrhs, flags, c->nsph,
+        HIPCHK(launch_reduce_quad<float>((const float *)part, c->nblocks * G, aout, 2 * c->neqns, nrhs, flags, c->nsph,
                                          c->npad, L, c->d_order, c->d_offset, c->d_an, c->st, gate));
     }
     if (e0) c->ev_prec.push_back(prec + 2 * (nr == 4));

@@ -1230,7 +1230,7 @@ template <typename T> static int matvec_t(FftOp *f, int nrhs, const double *ain,
     hipLaunchKernelGGL(sphere_reduce_kernel<T>, dim3((unsigned)((ns4 + 255) / 256)), dim3(256), 0, st, far, nf, nr,
                        f->d_sstart, f->d_sent, n, f->npad, NBP, out);
     FCHK(hipGetLastError());
-    FCHK(launch_reduce_post<T>((const T *)out, 1, aout, 2 * f->g.neqns, nrhs, flags, n, f->npad, Lp, f->g.d_order,
+    FCHK(launch_post<T>((const T *)out, aout, 2 * f->g.neqns, nrhs, flags, n, f->npad, Lp, f->g.d_order,
                                f->g.d_offset, f->g.d_an, st));
     f->launches++;
     return 0;

@@ -14,8 +14,7 @@ hipError_t launch_direct_tables(T *tab, const int2 *tiles, int ntiles, int L, in
 template <typename T>
 hipError_t launch_list_tables(T *tab, const double *rtran, int nslots, int LT, int LS, int itype, double rimed,
                               const double *vcc, int LM, hipStream_t st);
-// the FP64 and FP32 direct tables in one pass: orders whose layout kind is
-// the same at both precisions (direct_tables_both_ok)
+// the FP64 and FP32 direct tables in one pass (orders where direct_tables_both_ok)
 bool direct_tables_both_ok(int L);
 hipError_t launch_direct_tables_both(double *tab64, float *tab32, const int2 *tiles, int ntiles, int L, int nsph,
                                      const double *pos, double rimed, const double *vcc, int LM, hipStream_t st);
@@ -25,19 +24,30 @@ hipError_t launch_direct_tables_both(double *tab64, float *tab32, const int2 *ti
 // when *gate == 0 (every system of the Krylov loop that issued the product
 // has stopped), so that products enqueued ahead of the host's next read of
 // the solver state cost little.
-template <typename T>
 // G (1, 2, 4, 8 or 16) workgroups per tile share its 16 steps; the partials
-// are then (partner block x G) per target
+// are then (partner block x G) per target.  Vectors in quad layout (tile.hpp).
+template <typename T>
 hipError_t launch_direct_tiles(const T *tab, const int2 *tiles, int ntiles, int L, const T *xin, T *partial, int npad,
                                int nr, int G, hipStream_t st, const int *gate = nullptr);
+template <> hipError_t launch_direct_tiles<float>(const float *, const int2 *, int, int, const float *, float *, int,
+                                                  int, int, hipStream_t, const int *);  // tile32.hip
+template <> hipError_t launch_direct_tiles<double>(const double *, const int2 *, int, int, const double *, double *,
+                                                   int, int, int, hipStream_t, const int *);  // tile64.hip
 template <typename T>
-hipError_t launch_prep(const double *ain, int ldain, T *xin, int nrhs, const int *flags, int nsph, int npad, int Lp,
-                       const int *order, const int *offset, const double *an, hipStream_t st,
-                       const int *gate = nullptr);
+hipError_t launch_prep_quad(const double *ain, int ldain, T *xin, int nrhs, const int *flags, int nsph, int npad,
+                            int Lp, const int *order, const int *offset, const double *an, hipStream_t st,
+                            const int *gate = nullptr);
 template <typename T>
-hipError_t launch_reduce_post(const T *partial, int nparts, double *aout, int ldaout, int nrhs, const int *flags,
+hipError_t launch_reduce_quad(const T *partial, int nparts, double *aout, int ldaout, int nrhs, const int *flags,
                               int nsph, int npad, int Lp, const int *order, const int *offset, const double *an,
                               hipStream_t st, const int *gate = nullptr);
+// FFT operator: up to two columns, [column][sphere][mode][packed (m,n)]
+template <typename T>
+hipError_t launch_prep(const double *ain, int ldain, T *xin, int nrhs, const int *flags, int nsph, int npad, int Lp,
+                       const int *order, const int *offset, const double *an, hipStream_t st);
+template <typename T>
+hipError_t launch_post(const T *res, double *aout, int ldaout, int nrhs, const int *flags, int nsph, int npad, int Lp,
+                       const int *order, const int *offset, const double *an, hipStream_t st);
 
 // mie.hip
 hipError_t launch_mie(const double *x, const double *mre, const double *mim, double mmed, int nsph, double qeps,

@@ -10,9 +10,10 @@
 #include "kernels.hpp"
 
 // Where build_slot's values go: one table of store type T, or the FP64 and
-// FP32 tables of the same slot at once (the same FP64 values, rounded for
-// the second).  off(VW) is an element's offset in a layout of VW elements
-// per 16 bytes; the slot is interleaved at k.
+// FP32 direct tables of the same slot at once (the same FP64 values, rounded
+// for the second).  Full layout: off(VW) is an element's offset in a layout
+// of VW elements per 16 bytes; the slot is interleaved at k.  Compact layout
+// of the direct tables (order L): rot(e, v) and ax(c, re, im).
 template <typename T> struct OneTable {
     T *__restrict__ grp;
     int k;
@@ -21,15 +22,31 @@ template <typename T> struct OneTable {
         constexpr int VW = 16 / (int)sizeof(T);
         grp[ilv(off(VW), k, VW)] = (T)v;
     }
+    __device__ __forceinline__ void rot(int e, double v, int) const { grp[ilv(e, k, 16 / (int)sizeof(T))] = (T)v; }
+    __device__ __forceinline__ void ax(int c, double re, double im, int L) const
+    {
+        T *p = grp + ilv(cax_elem(c, L, sizeof(T)), k, 16 / (int)sizeof(T));
+        p[0] = (T)re;
+        p[1] = (T)im;
+    }
 };
 struct BothTables {
-    double *__restrict__ g64;
-    float *__restrict__ g32;
-    int k;
+    OneTable<double> t64;
+    OneTable<float> t32;
     template <typename F> __device__ __forceinline__ void put(F off, double v) const
     {
-        g64[ilv(off(2), k, 2)] = v;
-        g32[ilv(off(4), k, 4)] = (float)v;
+        t64.put(off, v);
+        t32.put(off, v);
+    }
+    __device__ __forceinline__ void rot(int e, double v, int L) const
+    {
+        t64.rot(e, v, L);
+        t32.rot(e, v, L);
+    }
+    __device__ __forceinline__ void ax(int c, double re, double im, int L) const
+    {
+        t64.ax(c, re, im, L);
+        t32.ax(c, re, im, L);
     }
 };
 
@@ -90,14 +107,15 @@ __device__ __forceinline__ void build_slot(const Sink &out, int LT, int LS, int 
                 out.put([&](int VW) { return sec_off(b, LT, LS, VW) + r0 + kk + n; }, v);
             }
         };
-        // symmetric layout (LT = LS): half-sum / half-difference rows of block m >= 0
+        // compact layout (LT = LS): triangles of E_n and O_n, row m
         auto put_sym = [&](int m, const double *row) {
-            const int e0 = srow_off(m, n);
-            for (int kk = 0; kk <= n; kk++) {
-                double sg = (kk & 1) ? -1.0 : 1.0;
-                double e = (kk == 0) ? row[n] : 0.5 * (row[kk + n] + sg * row[-kk + n]);
-                out.put([&](int) { return e0 + kk; }, e);
-                if (m > 0 && kk > 0) out.put([&](int) { return e0 + n + kk; }, 0.5 * (row[kk + n] - sg * row[-kk + n]));
+            const int e0 = crot_off(n), o0 = e0 + crot_o(n);
+            const double sm = (m & 1) ? -1.0 : 1.0;
+            for (int kk = m; kk <= n; kk++) {
+                const double sg = (kk & 1) ? -sm : sm;
+                const double e = (kk == 0) ? row[n] : 0.5 * (sm * row[kk + n] + sg * row[-kk + n]);
+                out.rot(e0 + ctri(m, kk), e, LT);
+                if (m > 0) out.rot(o0 + ctri(m - 1, kk - 1), 0.5 * (sm * row[kk + n] - sg * row[-kk + n]), LT);
             }
         };
         if (sym) put_sym(0, rowp);
@@ -175,12 +193,19 @@ __device__ __forceinline__ void build_slot(const Sink &out, int LT, int LS, int 
                 }
             }
         }
+        if (sym) {  // triangles of B_m(t,s) = (-1)^t A_m(t,s)
+            for (int p = 0; p < (m ? 2 : 1); p++)
+                for (int l = m1; l <= LS; l++)
+                    for (int n = m1; n <= l; n++) {
+                        const cplx<double> v = cscale(ACT(n, l)[p], (n & 1) ? -1.0 : 1.0);
+                        out.ax(cax_off(m, p, LT) + ctri(n - m1, l - m1), v.re, v.im, LT);
+                    }
+            continue;
+        }
         // block start and mode stride in a layout of VW elements per 16 bytes
-        auto ax0 = [&](int VW) {
-            return sym ? sax_off(m, LT, VW) : sec_off(b, LT, LS, VW) + pad_to(rot_len(m, LT, LS), VW);
-        };
-        auto axp = [&](int VW) { return sym ? pad_to(sax_len(m, LT), VW) : pad_to(ax_len(m, LT, LS), VW); };
-        for (int p = 0; p < (sym ? sax_modes(m) : 2); p++)
+        auto ax0 = [&](int VW) { return sec_off(b, LT, LS, VW) + pad_to(rot_len(m, LT, LS), VW); };
+        auto axp = [&](int VW) { return pad_to(ax_len(m, LT, LS), VW); };
+        for (int p = 0; p < 2; p++)
             for (int l = m1; l <= LS; l++)
                 for (int n = m1; n <= LT; n++) {
                     const int e = 2 * ((n - m1) + (LT - m1 + 1) * (l - m1));
@@ -189,9 +214,19 @@ __device__ __forceinline__ void build_slot(const Sink &out, int LT, int LS, int 
                 }
     }
 #undef ACT
-    auto ep = [&](int VW) { return sym ? sphi_off(LT, VW) : phi_off(LT, LS, VW); };
-    out.put(ep, cph);
-    out.put([&](int VW) { return ep(VW) + 1; }, sph);
+    if (sym) {
+        out.ax(cax_tot(LT), cph, sph, LT);
+    } else {
+        out.put([&](int VW) { return phi_off(LT, LS, VW); }, cph);
+        out.put([&](int VW) { return phi_off(LT, LS, VW) + 1; }, sph);
+    }
+}
+
+// self pairs and padding spheres
+template <typename Sink> __device__ __forceinline__ void zero_slot(const Sink &out, int L, int elem)
+{
+    for (int e = 0; e < crot_pad(L, elem); e++) out.rot(e, 0.0, L);
+    for (int c = 0; c <= cax_tot(L); c++) out.ax(c, 0.0, 0.0, L);
 }
 
 // Direct-path tables: slot q = (tile*S + step)*S + k (S = MSTM_SLOTS) holds
@@ -214,19 +249,17 @@ __global__ void direct_tables_kernel(T *__restrict__ tab, const int2 *__restrict
     int2 bt = tiles[tile];
     int it = bt.x * MSTM_SLOTS + k;
     int is = bt.y * MSTM_SLOTS + (k + step) % MSTM_SLOTS;
-    T *grp = tab + g * slot_elems * MSTM_SLOTS;
-    const int VW = 16 / (int)sizeof(T);
+    const OneTable<T> out{tab + g * slot_elems * MSTM_SLOTS, k};
     if (it >= nsph || is >= nsph || it == is) {
-        for (int e = 0; e < slot_elems; e++) grp[ilv(e, k, VW)] = (T)0;
+        zero_slot(out, L, (int)sizeof(T));
         return;
     }
     double rt[3] = {pos[3 * it] - pos[3 * is], pos[3 * it + 1] - pos[3 * is + 1], pos[3 * it + 2] - pos[3 * is + 2]};
-    build_slot<LMX>(OneTable<T>{grp, k}, L, L, 3, rt, rimed, vcc, LM, direct_sym(L, (int)sizeof(T)));
+    build_slot<LMX>(out, L, L, 3, rt, rimed, vcc, LM, true);
 }
 
-// Both direct tables, FP64 and FP32, in one pass (orders with the same
-// layout kind at both precisions: symmetric up to 4, full from 6): each
-// slot's FP64 values are worked out once and stored twice.
+// Both direct tables, FP64 and FP32, in one pass: each slot's FP64 values are
+// worked out once and stored twice.
 template <int LMX>
 __global__ void direct_tables_both_kernel(double *__restrict__ tab64, float *__restrict__ tab32,
                                           const int2 *__restrict__ tiles, int ntiles, int L_, int nsph,
@@ -243,15 +276,14 @@ __global__ void direct_tables_both_kernel(double *__restrict__ tab64, float *__r
     int2 bt = tiles[tile];
     int it = bt.x * MSTM_SLOTS + k;
     int is = bt.y * MSTM_SLOTS + (k + step) % MSTM_SLOTS;
-    double *g64 = tab64 + g * se64 * MSTM_SLOTS;
-    float *g32 = tab32 + g * se32 * MSTM_SLOTS;
+    const BothTables out{{tab64 + g * se64 * MSTM_SLOTS, k}, {tab32 + g * se32 * MSTM_SLOTS, k}};
     if (it >= nsph || is >= nsph || it == is) {
-        for (int e = 0; e < se64; e++) g64[ilv(e, k, 2)] = 0.0;
-        for (int e = 0; e < se32; e++) g32[ilv(e, k, 4)] = 0.0f;
+        zero_slot(out.t64, L, 8);
+        zero_slot(out.t32, L, 4);
         return;
     }
     double rt[3] = {pos[3 * it] - pos[3 * is], pos[3 * it + 1] - pos[3 * is + 1], pos[3 * it + 2] - pos[3 * is + 2]};
-    build_slot<LMX>(BothTables{g64, g32, k}, L, L, 3, rt, rimed, vcc, LM, direct_sym(L, 8));
+    build_slot<LMX>(out, L, L, 3, rt, rimed, vcc, LM, true);
 }
 
 template <typename T>
@@ -282,7 +314,10 @@ template hipError_t launch_direct_tables<float>(float *, const int2 *, int, int,
 template hipError_t launch_direct_tables<double>(double *, const int2 *, int, int, int, const double *, double,
                                                  const double *, int, hipStream_t);
 
-bool direct_tables_both_ok(int L) { return L >= 1 && L <= MSTM_TAB_L && direct_sym(L, 8) == direct_sym(L, 4); }
+// order 5 takes two passes: compiled for both stores at once, its recurrences
+// contract to other fused multiply-adds than in the separate builds, and the
+// two ways must give the same bits
+bool direct_tables_both_ok(int L) { return L >= 1 && L <= MSTM_TAB_L && L != 5; }
 
 hipError_t launch_direct_tables_both(double *tab64, float *tab32, const int2 *tiles, int ntiles, int L, int nsph,
                                      const double *pos, double rimed, const double *vcc, int LM, hipStream_t st)
