@@ -107,8 +107,11 @@ struct mstm_hip_ctx {
     size_t fg_bytes = 0;
     double *d_gm = nullptr;  // GMRES basis of the inner solver, two systems interleaved
     size_t gm_bytes = 0;
-    double *d_gh = nullptr;  // GMRES projections on the device (2 passes x 2 systems)
-    double *d_gp = nullptr;  // block partials of the GMRES projections (krylov grid x basis size)
+    GmSys *d_gsys = nullptr;  // small quantities of two GMRES systems
+    GmStat *h_gstat = nullptr;  // pinned: their state after the last two steps
+    hipEvent_t gm_ev[2] = {nullptr, nullptr};
+    double *d_gp = nullptr;  // block sums of the GMRES projections
+    size_t gp_bytes = 0;
     int inner = 1;           // inner solver of the mixed refinement: 0 BiCG, 1 GMRES
     int max_ref = 6;         // FP64 refinement cycles of the mixed solvers
     // Krylov work vectors (complex FP64, neqns each)
@@ -419,8 +422,11 @@ int mstm_hip_destroy(mstm_hip_ctx *c)
     release_spheres(c);
     release_observables(c);
     dfree(c->lig.params);
-    dfree(c->d_gh);
+    dfree(c->d_gsys);
     dfree(c->d_gp);
+    for (auto &e : c->gm_ev)
+        if (e) hipEventDestroy(e);
+    if (c->h_gstat) hipHostFree(c->h_gstat);
     dfree(c->d_vcc);
     dfree(c->d_partials);
     dfree(c->d_bscal);
@@ -767,13 +773,25 @@ static int matvec(mstm_hip_ctx *c, int nrhs, const double *ain, double *aout, co
         const size_t V = 2 * (size_t)c->neqns;
         for (int r0 = 0; r0 < nrhs; r0 += 2) {  // the node-grid operator takes two columns per call
             const int nr = std::min(2, nrhs - r0);
-            int rc = fft_matvec(c->fft, nr, ain + V * r0, aout + V * r0, flags + r0, prec, c->st);
+            int rc = fft_matvec(c->fft, nr, ain + V * r0, aout + V * r0, flags + r0, prec, c->st, c->gate);
             if (rc) return fail(c, rc, "fft matvec: %s", fft_last_error(c->fft));
             c->stats.matvecs[prec]++;
         }
         return 0;
     }
     return direct_matvec(c, nrhs, ain, aout, flags, prec);
+}
+
+// take the last product out of the counts (it was enqueued ahead and its
+// gate was closed)
+static void drop_product(mstm_hip_ctx *c, int prec, int use_fft)
+{
+    c->stats.matvecs[prec]--;
+    if (use_fft) fft_drop_product(c->fft);
+    else if (!c->ev_prec.empty() && c->ev_used >= 2) {
+        c->ev_used -= 2;
+        c->ev_prec.pop_back();
+    }
 }
 
 static void collect_events(mstm_hip_ctx *c)
@@ -1090,33 +1108,39 @@ static int oos2_dev(mstm_hip_ctx *c, int ns, int nord, const double *eps, const 
 
 // GMRES(m) (Saad & Schultz, SIAM J. Sci. Stat. Comput. 7, 856 (1986)) for
 // ns = 1 or 2 systems A d_s = b_s at once, from d_s = 0.  Arnoldi vectors
-// are FP64 and orthogonalised by classical Gram-Schmidt applied twice (one
-// projection kernel and one update kernel per pass, no host round trip);
-// the products run at precision prec, one column per system (both systems
-// in one launch while both iterate) -- half the columns of a BiCG step.  A
+// are FP64 and orthogonalised by classical Gram-Schmidt applied twice; the
+// products run at precision prec, one column per system (both systems in one launch) -- half the columns of a BiCG step.  A
 // system stops when its residual estimate |g_{j+1}|^2/|b|^2 < eps[s];
 // restarts every m steps from the residual b - A d.  it[s]: Arnoldi steps.
+// Projections, rotations and the stop test stay on the device (launch_gm_step);
+// the host enqueues one step ahead of the state it has read, and a step of
+// systems that have all stopped returns at once (gate).
 static int scaled_copy(mstm_hip_ctx *c, double *dst, const double *src, double sr, double si);
-static const int GM_M = 120;
 static int gmres2_dev(mstm_hip_ctx *c, int ns, int niter, const double *eps, const double *b, double *x, int prec,
                       int use_fft, int *it, double *err)
 {
-    typedef std::complex<double> zc;
-    const int m = std::min(GM_M, multi_vec_max() - 2);
     const int n = c->neqns;
     const size_t V = 2 * c->kv_n;
-    const size_t need = sizeof(double) * V * 2 * (m + 1);
+    const size_t need = sizeof(double) * V * 2 * (GM_M + 1), npart = sizeof(double) * 2 * gm_partials(n);
     if (c->gm_bytes < need) {
         dfree(c->d_gm);
+        c->gm_bytes = 0;
         HIPCHK(dalloc(&c->d_gm, need));
         c->gm_bytes = need;
     }
-    if (!c->d_gh) HIPCHK(dalloc(&c->d_gh, sizeof(double) * 2 * 4 * (GM_M + 2)));
-    if (!c->d_gp) HIPCHK(dalloc(&c->d_gp, sizeof(double) * 2 * (size_t)krylov_grid() * (GM_M + 2)));
+    if (c->gp_bytes < npart) {
+        dfree(c->d_gp);
+        c->gp_bytes = 0;
+        HIPCHK(dalloc(&c->d_gp, npart));
+        c->gp_bytes = npart;
+    }
+    if (!c->d_gsys) HIPCHK(dalloc(&c->d_gsys, sizeof(GmSys) * 2));
+    if (!c->h_gstat) HIPCHK(hipHostMalloc((void **)&c->h_gstat, sizeof(GmStat) * 4, hipHostMallocDefault));
+    for (auto &e : c->gm_ev)
+        if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     auto basis = [&](int j, int sys) { return c->d_gm + V * (2 * (size_t)j + sys); };
-    double *W = c->d_kv + V * KV_CAPS;  // w_s at W + s V
+    double *W = c->d_kv + V * KV_CAPS;  // products
     double *T = c->d_kv + V * KV_ST;    // temporaries t_s at T + s V
-    auto hdev = [&](int pass, int sys) { return c->d_gh + 2 * (size_t)(GM_M + 2) * (2 * sys + pass); };
     double bb[2] = {0, 0};
     bool open[2] = {false, false};
     for (int q = 0; q < ns; q++) {
@@ -1135,16 +1159,13 @@ static int gmres2_dev(mstm_hip_ctx *c, int ns, int niter, const double *eps, con
         err[q] = open[q] ? 1.0 : 0.0;
     }
     int f2[2] = {2, 2};
-    std::vector<zc> H[2], g[2], sn[2];
-    std::vector<double> cs[2];
     for (int cycle = 0; open[0] || (ns == 2 && open[1]); cycle++) {
         double beta[2] = {0, 0};
         if (cycle == 0) {
             for (int q = 0; q < ns; q++)
                 if (open[q]) {
                     beta[q] = std::sqrt(bb[q]);
-                    rc = scaled_copy(c, basis(0, q), b + V * q, 1.0 / beta[q], 0.0);
-                    if (rc) return rc;
+                    HIPCHK(hipMemcpyAsync(basis(0, q), b + V * q, sizeof(double) * V, hipMemcpyDeviceToDevice, c->st));
                 }
         } else {
             // r = b - A x = b - x + T H x
@@ -1171,106 +1192,60 @@ static int gmres2_dev(mstm_hip_ctx *c, int ns, int niter, const double *eps, con
                 err[q] = v[0] / bb[q];
                 if (err[q] < eps[q] || it[q] >= niter || beta[q] == 0.0) {
                     open[q] = false;
+                    beta[q] = 0.0;
                     continue;
                 }
-                rc = scaled_copy(c, basis(0, q), T + V * q, 1.0 / beta[q], 0.0);
+                HIPCHK(hipMemcpyAsync(basis(0, q), T + V * q, sizeof(double) * V, hipMemcpyDeviceToDevice, c->st));
+            }
+            if (!open[0] && !(ns == 2 && open[1])) break;
+        }
+        // the systems of this cycle: both, or the one that is open
+        const int q0 = open[0] ? 0 : 1, nq = (open[0] ? 1 : 0) + (ns == 2 && open[1] ? 1 : 0);
+        GmStart st[2];
+        for (int q = 0; q < nq; q++) st[q] = {bb[q0 + q], eps[q0 + q], beta[q0 + q], it[q0 + q], niter, GM_M};
+        HIPCHK(launch_gm_begin(c->d_gsys, nq, st, basis(0, q0), (int64_t)V, n, c->d_gate, c->st));
+        struct GateScope {  // products outside this loop are never gated
+            mstm_hip_ctx *c;
+            ~GateScope() { c->gate = nullptr; }
+        } gate_scope{c};
+        c->gate = c->d_gate;
+        // enqueue step j, then read the state after step j - 1
+        auto stat = [&](int j) { return c->h_gstat + 2 * (j & 1); };
+        auto enqueue = [&](int j) -> int {
+            int r = matvec(c, nq, basis(j, q0), W, f2, prec, use_fft);
+            if (r) return r;
+            HIPCHK(launch_gm_step(c->d_gsys, nq, basis(0, q0), (int64_t)(2 * V), (int64_t)V, j + 1, W, (int64_t)V, n,
+                                  c->d_gp, c->d_gate, stat(j), c->st));
+            HIPCHK(hipEventRecord(c->gm_ev[j & 1], c->st));
+            return 0;
+        };
+        rc = enqueue(0);
+        if (rc) return rc;
+        int last = 0;  // steps enqueued - 1
+        for (int j = 0;; j++) {
+            if (j + 1 < GM_M) {
+                rc = enqueue(j + 1);
                 if (rc) return rc;
+                last = j + 1;
+            }
+            HIPCHK(hipEventSynchronize(c->gm_ev[j & 1]));
+            bool any = false;
+            for (int q = 0; q < nq; q++) any = any || stat(j)[q].active;
+            if (!any) {
+                if (last > j) drop_product(c, prec, use_fft);  // the step enqueued ahead did nothing
+                for (int q = 0; q < nq; q++) {
+                    const GmStat *s = stat(j) + q;
+                    it[q0 + q] += s->k;
+                    err[q0 + q] = s->err;
+                    if (s->done) open[q0 + q] = false;
+                    if (prec == MSTM_HIP_FP64) c->stats.iters_fp64 += s->k;
+                    else c->stats.iters_fp32 += s->k;
+                }
+                break;
             }
         }
-        bool run[2] = {open[0], ns == 2 && open[1]};
-        int k[2] = {0, 0};
-        for (int q = 0; q < ns; q++) {
-            H[q].assign((size_t)(m + 1) * m, zc(0.0));
-            g[q].assign(m + 1, zc(0.0));
-            sn[q].assign(m, zc(0.0));
-            cs[q].assign(m, 0.0);
-            g[q][0] = beta[q];
-        }
-        for (int j = 0; j < m && (run[0] || run[1]); j++) {
-            // w = A v_j = v_j - T H v_j
-            if (run[0] && run[1]) rc = matvec(c, 2, basis(j, 0), W, f2, prec, use_fft);
-            else rc = matvec(c, 1, basis(j, run[0] ? 0 : 1), W + V * (run[0] ? 0 : 1), f2, prec, use_fft);
-            if (rc) return rc;
-            for (int q = 0; q < ns; q++) {
-                if (!run[q]) continue;
-                double *w = W + V * q;
-                HIPCHK(launch_zaxpby(1.0, 0.0, basis(j, q), -1.0, 0.0, w, n, c->st));
-                // two passes of classical Gram-Schmidt against v_0..v_j
-                for (int pass = 0; pass < 2; pass++) {
-                    HIPCHK(launch_multi_zdot(basis(0, q), (int64_t)(2 * V), j + 1, w, n, c->d_gp, hdev(pass, q),
-                                             c->st));
-                    HIPCHK(launch_multi_axpy(basis(0, q), (int64_t)(2 * V), j + 1, hdev(pass, q), -1.0, w, n,
-                                             c->st));
-                }
-            }
-            // |w|^2 of each system (separate partial regions), then one host round trip
-            for (int q = 0; q < ns; q++)
-                if (run[q]) HIPCHK(launch_zdot(W + V * q, W + V * q, n, 1, pregion(c, 2 + q), nullptr, c->st));
-            std::vector<zc> hh[2][2];
-            for (int q = 0; q < ns; q++) {
-                if (!run[q]) continue;
-                for (int pass = 0; pass < 2; pass++) {
-                    hh[q][pass].resize(j + 1);
-                    HIPCHK(hipMemcpyAsync(hh[q][pass].data(), hdev(pass, q), sizeof(zc) * (j + 1),
-                                          hipMemcpyDeviceToHost, c->st));
-                }
-            }
-            rc = fetch_partials(c, 2 * krylov_grid() * 4);
-            if (rc) return rc;
-            for (int q = 0; q < ns; q++) {
-                if (!run[q]) continue;
-                double v[2];
-                reduce_region(c, pregion_off(2 + q), 1, v);
-                const double hn = std::sqrt(std::max(v[0], 0.0));
-                auto h = [&](int r, int col) -> zc & { return H[q][(size_t)r * m + col]; };
-                for (int r = 0; r <= j; r++) h(r, j) = hh[q][0][r] + hh[q][1][r];
-                h(j + 1, j) = hn;
-                for (int r = 0; r < j; r++) {  // earlier rotations on column j
-                    const zc a = h(r, j), bq = h(r + 1, j);
-                    h(r, j) = cs[q][r] * a + sn[q][r] * bq;
-                    h(r + 1, j) = -std::conj(sn[q][r]) * a + cs[q][r] * bq;
-                }
-                const zc a = h(j, j), bq = h(j + 1, j);
-                const double nu = std::sqrt(std::norm(a) + std::norm(bq));
-                if (std::abs(a) == 0.0) {
-                    cs[q][j] = 0.0;
-                    sn[q][j] = 1.0;
-                } else {
-                    cs[q][j] = std::abs(a) / nu;
-                    sn[q][j] = (a / std::abs(a)) * std::conj(bq) / nu;
-                }
-                h(j, j) = cs[q][j] * a + sn[q][j] * bq;
-                h(j + 1, j) = 0.0;
-                g[q][j + 1] = -std::conj(sn[q][j]) * g[q][j];
-                g[q][j] = cs[q][j] * g[q][j];
-                k[q] = j + 1;
-                it[q]++;
-                if (prec == MSTM_HIP_FP64) c->stats.iters_fp64++;
-                else c->stats.iters_fp32++;
-                err[q] = std::norm(g[q][j + 1]) / bb[q];
-                if (err[q] < eps[q] || it[q] >= niter || hn == 0.0 || nu == 0.0) {
-                    run[q] = false;
-                    if (err[q] < eps[q] || it[q] >= niter) open[q] = false;
-                } else {
-                    rc = scaled_copy(c, basis(j + 1, q), W + V * q, 1.0 / hn, 0.0);
-                    if (rc) return rc;
-                }
-            }
-        }
-        // x += sum_i y_i v_i with R y = g
-        for (int q = 0; q < ns; q++) {
-            if (!k[q]) continue;
-            auto h = [&](int r, int col) -> zc & { return H[q][(size_t)r * m + col]; };
-            std::vector<zc> y(k[q]);
-            for (int r = k[q] - 1; r >= 0; r--) {
-                zc sum = g[q][r];
-                for (int t = r + 1; t < k[q]; t++) sum -= h(r, t) * y[t];
-                y[r] = h(r, r) != zc(0.0) ? sum / h(r, r) : zc(0.0);
-            }
-            HIPCHK(hipMemcpyAsync(hdev(0, q), y.data(), sizeof(zc) * k[q], hipMemcpyHostToDevice, c->st));
-            HIPCHK(launch_multi_axpy(basis(0, q), (int64_t)(2 * V), k[q], hdev(0, q), 1.0, x + V * q, n, c->st));
-            HIPCHK(hipStreamSynchronize(c->st));  // y lives on the host stack
-        }
+        HIPCHK(launch_gm_update(c->d_gsys, nq, basis(0, q0), (int64_t)(2 * V), (int64_t)V, x + V * q0, (int64_t)V, n,
+                                c->st));
     }
     return 0;
 }

@@ -82,8 +82,10 @@ static int4 flags4(const int *flags, int nrhs)
 template <typename T>
 __global__ void prep_kernel(const cplx<double> *__restrict__ ain, int ldain, cplx<T> *__restrict__ xin, int nrhs,
                             int4 flags, int nsph, int npad, int Lp, const int *__restrict__ order,
-                            const int *__restrict__ offset, const cplx<double> *__restrict__ an)
+                            const int *__restrict__ offset, const cplx<double> *__restrict__ an,
+                            const int *__restrict__ gate)
 {
+    if (gate && !*gate) return;
     const int NBP = Lp * (Lp + 2);
     int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= (int64_t)2 * npad * NBP) return;
@@ -104,7 +106,7 @@ __global__ void prep_kernel(const cplx<double> *__restrict__ ain, int ldain, cpl
 
 template <typename T>
 hipError_t launch_prep(const double *ain, int ldain, T *xin, int nrhs, const int *flags, int nsph, int npad, int Lp,
-                       const int *order, const int *offset, const double *an, hipStream_t st)
+                       const int *order, const int *offset, const double *an, hipStream_t st, const int *gate)
 {
     if (nrhs < 1 || nrhs > 2) return hipErrorInvalidValue;
     const int64_t n = (int64_t)2 * npad * Lp * (Lp + 2);
@@ -112,13 +114,13 @@ hipError_t launch_prep(const double *ain, int ldain, T *xin, int nrhs, const int
     hipLaunchKernelGGL(prep_kernel<T>, dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0, st,
                        reinterpret_cast<const cplx<double> *>(ain), ldain / 2, reinterpret_cast<cplx<T> *>(xin), nrhs,
                        flags4(flags, nrhs), nsph, npad, Lp, order, offset,
-                       reinterpret_cast<const cplx<double> *>(an));
+                       reinterpret_cast<const cplx<double> *>(an), gate);
     return hipGetLastError();
 }
 template hipError_t launch_prep<float>(const double *, int, float *, int, const int *, int, int, int, const int *,
-                                       const int *, const double *, hipStream_t);
+                                       const int *, const double *, hipStream_t, const int *);
 template hipError_t launch_prep<double>(const double *, int, double *, int, const int *, int, int, int, const int *,
-                                        const int *, const double *, hipStream_t);
+                                        const int *, const double *, hipStream_t, const int *);
 
 // Direct tiles: quad layout (tile.hpp).  Position, in T, of complex value idx
 // of (column r, mode p) of a sphere.
@@ -193,8 +195,10 @@ template hipError_t launch_prep_quad<double>(const double *, int, double *, int,
 template <typename T>
 __global__ void post_kernel(const cplx<T> *__restrict__ res, cplx<double> *__restrict__ aout, int ldaout, int nrhs,
                             int4 flags, int nsph, int npad, int Lp, const int *__restrict__ order,
-                            const int *__restrict__ offset, const cplx<double> *__restrict__ an)
+                            const int *__restrict__ offset, const cplx<double> *__restrict__ an,
+                            const int *__restrict__ gate)
 {
+    if (gate && !*gate) return;
     const int NBP = Lp * (Lp + 2);
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= (int64_t)nrhs * nsph * NBP) return;
@@ -212,7 +216,7 @@ __global__ void post_kernel(const cplx<T> *__restrict__ res, cplx<double> *__res
 
 template <typename T>
 hipError_t launch_post(const T *res, double *aout, int ldaout, int nrhs, const int *flags, int nsph, int npad, int Lp,
-                       const int *order, const int *offset, const double *an, hipStream_t st)
+                       const int *order, const int *offset, const double *an, hipStream_t st, const int *gate)
 {
     if (nrhs < 1 || nrhs > 2) return hipErrorInvalidValue;
     const int64_t n = (int64_t)nrhs * nsph * Lp * (Lp + 2);
@@ -220,13 +224,13 @@ hipError_t launch_post(const T *res, double *aout, int ldaout, int nrhs, const i
     hipLaunchKernelGGL(post_kernel<T>, dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0, st,
                        reinterpret_cast<const cplx<T> *>(res), reinterpret_cast<cplx<double> *>(aout), ldaout / 2,
                        nrhs, flags4(flags, nrhs), nsph, npad, Lp, order, offset,
-                       reinterpret_cast<const cplx<double> *>(an));
+                       reinterpret_cast<const cplx<double> *>(an), gate);
     return hipGetLastError();
 }
 template hipError_t launch_post<float>(const float *, double *, int, int, const int *, int, int, int, const int *,
-                                       const int *, const double *, hipStream_t);
+                                       const int *, const double *, hipStream_t, const int *);
 template hipError_t launch_post<double>(const double *, double *, int, int, const int *, int, int, int, const int *,
-                                        const int *, const double *, hipStream_t);
+                                        const int *, const double *, hipStream_t, const int *);
 
 // Direct tiles: the sum over the partials (quad layout) in FP64, then the
 // post-op.  A workgroup owns SP spheres of one column pair: U units (16 bytes;

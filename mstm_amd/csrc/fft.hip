@@ -49,8 +49,10 @@ __global__ __launch_bounds__(NT) void list_translate_kernel(const T *__restrict_
                                                                     const int64_t *__restrict__ src_off, int64_t rs,
                                                                     int64_t ms, int64_t es,
                                                                     const unsigned char *__restrict__ ident,
-                                                                    cplx<T> *__restrict__ dst)
+                                                                    cplx<T> *__restrict__ dst,
+                                                                    const int *__restrict__ gate)
 {
+    if (gate && !*gate) return;
     constexpr int VW = 16 / sizeof(T);
     const int q = blockIdx.x, tid = threadIdx.x;
     if (q >= nslots) return;
@@ -191,14 +193,14 @@ static int list_translate_threads(int LT, int LS)
 template <typename T, int DIR>
 static hipError_t launch_list_translate(dim3 g, size_t lds, hipStream_t st, const T *tab, int nslots, int LT, int LS,
                                         const cplx<T> *src, const int64_t *off, int64_t rs, int64_t ms, int64_t es,
-                                        const unsigned char *ident, cplx<T> *dst)
+                                        const unsigned char *ident, cplx<T> *dst, const int *gate)
 {
     if (list_translate_threads(LT, LS) == 256)
         hipLaunchKernelGGL((list_translate_kernel<T, DIR, 256>), g, dim3(256), lds, st, tab, nslots, LT, LS, src, off,
-                           rs, ms, es, ident, dst);
+                           rs, ms, es, ident, dst, gate);
     else
         hipLaunchKernelGGL((list_translate_kernel<T, DIR, 128>), g, dim3(128), lds, st, tab, nslots, LT, LS, src, off,
-                           rs, ms, es, ident, dst);
+                           rs, ms, es, ident, dst, gate);
     return hipGetLastError();
 }
 
@@ -213,8 +215,10 @@ template <typename T> static size_t list_translate_lds(int LT, int LS)
 // anode[r][p][n][cell] = sum over spheres of the cell of asph[i][r][p][n]
 template <typename T>
 __global__ void node_reduce_kernel(const cplx<T> *__restrict__ asph, const int *__restrict__ cstart,
-                                   const int *__restrict__ cmem, int ncells, int nblk, cplx<T> *__restrict__ anode)
+                                   const int *__restrict__ cmem, int ncells, int nblk, cplx<T> *__restrict__ anode,
+                                   const int *__restrict__ gate)
 {
+    if (gate && !*gate) return;
     int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= (int64_t)4 * nblk * ncells) return;
     int cell = (int)(q % ncells);
@@ -230,8 +234,9 @@ template <typename T>
 __global__ void sphere_reduce_kernel(const cplx<T> *__restrict__ far, const cplx<T> *__restrict__ nf,
                                      const cplx<T> *__restrict__ nr, const int *__restrict__ sstart,
                                      const int *__restrict__ sent, int nsph, int npad, int NBP,
-                                     cplx<T> *__restrict__ out)
+                                     cplx<T> *__restrict__ out, const int *__restrict__ gate)
 {
+    if (gate && !*gate) return;
     int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= (int64_t)nsph * 4 * NBP) return;
     int e = (int)(q % NBP);
@@ -292,8 +297,10 @@ __device__ __forceinline__ void stage_radix(const cplx<T> *__restrict__ A, cplx<
 
 template <typename T>
 __global__ void fft_pass_kernel(const cplx<T> *__restrict__ in, cplx<T> *__restrict__ out, int3 din, int3 dout,
-                                int axis, FftPlan plan, int nin, int nout, int sign, int P)
+                                int axis, FftPlan plan, int nin, int nout, int sign, int P,
+                                const int *__restrict__ gate)
 {
+    if (gate && !*gate) return;
     extern __shared__ unsigned char smem[];
     cplx<T> *A = reinterpret_cast<cplx<T> *>(smem);
     const int n = plan.n;
@@ -410,7 +417,7 @@ static FftPlan make_plan(int n)
 
 template <typename T>
 static hipError_t fft_axis(const cplx<T> *in, cplx<T> *out, int batch, int3 din, int3 dout, int axis, int n, int nin,
-                           int nout, int sign, hipStream_t st)
+                           int nout, int sign, hipStream_t st, const int *gate = nullptr)
 {
     FftPlan pl = make_plan(n);
     if (pl.n < 0) return hipErrorInvalidValue;
@@ -424,7 +431,8 @@ static hipError_t fft_axis(const cplx<T> *in, cplx<T> *out, int batch, int3 din,
     int a0 = axis == 0 ? 1 : 0, a1 = axis == 2 ? 1 : 2;
     int npen = d[a0] * d[a1];
     dim3 g((npen + P - 1) / P, batch);
-    hipLaunchKernelGGL(fft_pass_kernel<T>, g, dim3(256), sh, st, in, out, din, dout, axis, pl, nin, nout, sign, P);
+    hipLaunchKernelGGL(fft_pass_kernel<T>, g, dim3(256), sh, st, in, out, din, dout, axis, pl, nin, nout, sign, P,
+                       gate);
     return hipGetLastError();
 }
 
@@ -469,8 +477,9 @@ __device__ __forceinline__ void contract_degrees(const cplx<float> *__restrict__
 
 template <typename T>
 __global__ void contract_kernel(const cplx<float> *__restrict__ K, const cplx<T> *__restrict__ a,
-                                cplx<T> *__restrict__ g, int M, int nblk)
+                                cplx<T> *__restrict__ g, int M, int nblk, const int *__restrict__ gate)
 {
+    if (gate && !*gate) return;
     constexpr int LC = CONTRACT_LC;
     static_assert(LC == 4, "the degree-count switch below covers 1..4");
     // workgroup -> (frequency block x, mode p, degree block z): the Z degree
@@ -894,6 +903,13 @@ void fft_reset_stats(FftOp *f)
     f->launches = 0;
 }
 
+void fft_drop_product(FftOp *f)
+{
+    if (!f) return;
+    f->launches--;
+    if (f->cev_used >= 2) f->cev_used -= 2;
+}
+
 static void free_prec(FftOp *f, int p)
 {
     ffree(f->jtab[p]);
@@ -1165,7 +1181,7 @@ int fft_setup(FftOp *f, int prec, hipStream_t st)
 }
 
 template <typename T> static int matvec_t(FftOp *f, int nrhs, const double *ain, double *aout, const int *flags,
-                                          hipStream_t st)
+                                          hipStream_t st, const int *gate)
 {
     const int prec = sizeof(T) == 8 ? 0 : 1;
     const int n = f->nsph, Lp = f->Lp, LG = f->LG, nblk = f->nblk;
@@ -1176,24 +1192,24 @@ template <typename T> static int matvec_t(FftOp *f, int nrhs, const double *ain,
             *nr = (cplx<T> *)f->nr[prec], *out = (cplx<T> *)f->out[prec];
     const T *jt = (const T *)f->jtab[prec], *ht = (const T *)f->htab[prec];
     FCHK(launch_prep<T>(ain, 2 * f->g.neqns, (T *)xin, nrhs, flags, n, f->npad, Lp, f->g.d_order, f->g.d_offset,
-                        f->g.d_an, st));
+                        f->g.d_an, st, gate));
     const int64_t rs_sph = (int64_t)f->npad * 2 * NBP;
     // sphere -> node (J translation, :573-626)
     dim3 lg(n);
     const size_t ljb = list_translate_lds<T>(LG, Lp), lhb = list_translate_lds<T>(Lp, Lp);
     FCHK((launch_list_translate<T, 0>)(lg, ljb, st, jt, n, LG, Lp, xin, f->d_off_sph, rs_sph, (int64_t)NBP, (int64_t)1,
-                                     f->d_ident_j, asph));
+                                     f->d_ident_j, asph, gate));
     int64_t nn4 = (int64_t)4 * nblk * f->ncells;
     hipLaunchKernelGGL(node_reduce_kernel<T>, dim3((unsigned)((nn4 + 255) / 256)), dim3(256), 0, st, asph, f->d_cstart,
-                       f->d_cmem, f->ncells, nblk, B);
+                       f->d_cmem, f->ncells, nblk, B, gate);
     FCHK(hipGetLastError());
     // forward zero-padded 3-D FFT: z, y, x
     const int batch = 4 * nblk;
     int3 d0 = N, d1 = make_int3(N.x, N.y, 2 * N.z), d2 = make_int3(N.x, 2 * N.y, 2 * N.z),
          d3 = make_int3(2 * N.x, 2 * N.y, 2 * N.z);
-    FCHK(fft_axis<T>(B, A, batch, d0, d1, 2, 2 * N.z, N.z, 2 * N.z, -1, st));
-    FCHK(fft_axis<T>(A, B, batch, d1, d2, 1, 2 * N.y, N.y, 2 * N.y, -1, st));
-    FCHK(fft_axis<T>(B, A, batch, d2, d3, 0, 2 * N.x, N.x, 2 * N.x, -1, st));
+    FCHK(fft_axis<T>(B, A, batch, d0, d1, 2, 2 * N.z, N.z, 2 * N.z, -1, st, gate));
+    FCHK(fft_axis<T>(A, B, batch, d1, d2, 1, 2 * N.y, N.y, 2 * N.y, -1, st, gate));
+    FCHK(fft_axis<T>(B, A, batch, d2, d3, 0, 2 * N.x, N.x, 2 * N.x, -1, st, gate));
     // per-frequency contraction with the node kernel spectrum
     const int cX = (f->M + 127) / 128, cZ = (nblk + CONTRACT_LC - 1) / CONTRACT_LC;
     dim3 cg_((unsigned)((2 * cX + 7) / 8 * 8 * cZ));
@@ -1206,42 +1222,42 @@ template <typename T> static int matvec_t(FftOp *f, int nrhs, const double *ain,
     f->cev_prec.resize(f->cev.size() / 2 + 1);
     f->cev_prec[f->cev_used / 2] = prec;
     FCHK(hipEventRecord(f->cev[f->cev_used], st));
-    hipLaunchKernelGGL(contract_kernel<T>, cg_, dim3(128), 0, st, f->K, A, B, f->M, nblk);
+    hipLaunchKernelGGL(contract_kernel<T>, cg_, dim3(128), 0, st, f->K, A, B, f->M, nblk, gate);
     FCHK(hipGetLastError());
     FCHK(hipEventRecord(f->cev[f->cev_used + 1], st));
     f->cev_used += 2;
     // inverse: x, y, z keeping the first N per axis
-    FCHK(fft_axis<T>(B, A, batch, d3, d2, 0, 2 * N.x, 2 * N.x, N.x, 1, st));
-    FCHK(fft_axis<T>(A, B, batch, d2, d1, 1, 2 * N.y, 2 * N.y, N.y, 1, st));
-    FCHK(fft_axis<T>(B, A, batch, d1, d0, 2, 2 * N.z, 2 * N.z, N.z, 1, st));
+    FCHK(fft_axis<T>(B, A, batch, d3, d2, 0, 2 * N.x, 2 * N.x, N.x, 1, st, gate));
+    FCHK(fft_axis<T>(A, B, batch, d2, d1, 1, 2 * N.y, 2 * N.y, N.y, 1, st, gate));
+    FCHK(fft_axis<T>(B, A, batch, d1, d0, 2, 2 * N.z, 2 * N.z, N.z, 1, st, gate));
     // node -> sphere (reverse J translation) from gnode[r][p][l][cell] in A
     const int64_t nc = f->ncells;
     FCHK((launch_list_translate<T, 1>)(lg, ljb, st, jt, n, LG, Lp, A, f->d_off_node, 2 * nblk * nc, nblk * nc, nc,
-                                     f->d_ident_j, far));
+                                     f->d_ident_j, far, gate));
     // near-field pairs, both directions (local_sphere_to_sphere_expansion)
     if (f->npairs) {
         dim3 pg(f->npairs);
         FCHK((launch_list_translate<T, 0>)(pg, lhb, st, ht, f->npairs, Lp, Lp, xin, f->d_off_pj, rs_sph, (int64_t)NBP,
-                                         (int64_t)1, f->d_ident_h, nf));
+                                         (int64_t)1, f->d_ident_h, nf, gate));
         FCHK((launch_list_translate<T, 1>)(pg, lhb, st, ht, f->npairs, Lp, Lp, xin, f->d_off_pi, rs_sph, (int64_t)NBP,
-                                         (int64_t)1, f->d_ident_h, nr));
+                                         (int64_t)1, f->d_ident_h, nr, gate));
     }
     int64_t ns4 = (int64_t)n * 4 * NBP;
     hipLaunchKernelGGL(sphere_reduce_kernel<T>, dim3((unsigned)((ns4 + 255) / 256)), dim3(256), 0, st, far, nf, nr,
-                       f->d_sstart, f->d_sent, n, f->npad, NBP, out);
+                       f->d_sstart, f->d_sent, n, f->npad, NBP, out, gate);
     FCHK(hipGetLastError());
     FCHK(launch_post<T>((const T *)out, aout, 2 * f->g.neqns, nrhs, flags, n, f->npad, Lp, f->g.d_order,
-                               f->g.d_offset, f->g.d_an, st));
+                               f->g.d_offset, f->g.d_an, st, gate));
     f->launches++;
     return 0;
 }
 
-int fft_matvec(FftOp *f, int nrhs, const double *ain, double *aout, const int *flags, int prec, hipStream_t st)
+int fft_matvec(FftOp *f, int nrhs, const double *ain, double *aout, const int *flags, int prec, hipStream_t st, const int *gate)
 {
     if (!f) return 3;
     if (!f->ready[prec]) {  // the context sets the operator up (fft_setup after binding its tables)
         f->err = "FFT operator of this precision not set up";
         return 3;
     }
-    return prec == 0 ? matvec_t<double>(f, nrhs, ain, aout, flags, st) : matvec_t<float>(f, nrhs, ain, aout, flags, st);
+    return prec == 0 ? matvec_t<double>(f, nrhs, ain, aout, flags, st, gate) : matvec_t<float>(f, nrhs, ain, aout, flags, st, gate);
 }

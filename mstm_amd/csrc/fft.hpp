@@ -34,7 +34,9 @@ void fft_grid(const FftOp *f, double *cell_boundary, int *sphere_node, int *numb
 // (re)binds the context's device pointers (vcc may have been regrown)
 void fft_bind(FftOp *f, const FftGeometry &g);
 int fft_setup(FftOp *f, int prec, hipStream_t st);
-int fft_matvec(FftOp *f, int nrhs, const double *ain, double *aout, const int *flags, int prec, hipStream_t st);
+int fft_matvec(FftOp *f, int nrhs, const double *ain, double *aout, const int *flags, int prec, hipStream_t st,
+               const int *gate);  // gate: as for the direct product
+void fft_drop_product(FftOp *f);  // the last product did nothing (its gate was closed): not counted
 void fft_clear(FftOp *f);
 void fft_destroy(FftOp *f);
 const char *fft_last_error(const FftOp *f);

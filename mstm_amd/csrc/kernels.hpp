@@ -44,10 +44,10 @@ hipError_t launch_reduce_quad(const T *partial, int nparts, double *aout, int ld
 // FFT operator: up to two columns, [column][sphere][mode][packed (m,n)]
 template <typename T>
 hipError_t launch_prep(const double *ain, int ldain, T *xin, int nrhs, const int *flags, int nsph, int npad, int Lp,
-                       const int *order, const int *offset, const double *an, hipStream_t st);
+                       const int *order, const int *offset, const double *an, hipStream_t st, const int *gate);
 template <typename T>
 hipError_t launch_post(const T *res, double *aout, int ldaout, int nrhs, const int *flags, int nsph, int npad, int Lp,
-                       const int *order, const int *offset, const double *an, hipStream_t st);
+                       const int *order, const int *offset, const double *an, hipStream_t st, const int *gate);
 
 // mie.hip
 hipError_t launch_mie(const double *x, const double *mre, const double *mim, double mmed, int nsph, double qeps,
@@ -103,12 +103,37 @@ hipError_t launch_bicg_c(double *cp, double *cw, const double *cr, const double 
 hipError_t launch_bicg_init(double *cr, double *cq, double *cw, double *cp, const double *pnp, const double *anp, int n,
                             double *partials, hipStream_t st);
 hipError_t launch_zaxpby(double ar, double ai, const double *x, double br, double bi, double *y, int n, hipStream_t st);
-// block Gram-Schmidt (GMRES): V_j at V + j*stride (doubles), out/h device arrays of nvec complex
-int multi_vec_max();
-hipError_t launch_multi_zdot(const double *V, int64_t stride, int nvec, const double *w, int n, double *partials,
-                             double *out, hipStream_t st);
-hipError_t launch_multi_axpy(const double *V, int64_t stride, int nvec, const double *h, double sign, double *w, int n,
-                             hipStream_t st);
+// GMRES (restart length GM_M at most) with its small quantities on the device,
+// one or two systems; see krylov.hip
+#define GM_M 120
+struct GmSys {
+    double bb, eps, err, scale;  // |b|^2, stop test |g|^2 / bb < eps, its last value; 1 / norm of the next vector
+    int active, done;            // iterating; stopped on eps or niter
+    int k, it0, niter, m;        // steps of this cycle, steps before it, step limits
+    double cs[GM_M];
+    cplx<double> sn[GM_M], g[GM_M + 1], h[2][GM_M + 1];
+    cplx<double> R[GM_M * (GM_M + 1) / 2];  // columns of the triangular factor
+};
+struct GmStart {
+    double bb, eps, beta;  // beta = |v_0| as given, 0: not in this cycle
+    int it0, niter, m;
+};
+struct GmStat {  // what the host reads after a step
+    double err;
+    int active, done, k;
+};
+size_t gm_partials(int n);  // complex values of block sums two systems need
+// start of a cycle, v_0 at V (+ vs for the second system), normalized here
+hipError_t launch_gm_begin(GmSys *sys, int ns, const GmStart *st, double *V, int64_t vs, int n, int *gate,
+                           hipStream_t str);
+// step nv = 1, 2, ...: basis vectors v_i at V + i * stride (+ vs), the product
+// of v_{nv-1} at p (+ ps); v_nv is written.  stat: two values of
+// device-visible pinned host memory
+hipError_t launch_gm_step(GmSys *sys, int ns, double *V, int64_t stride, int64_t vs, int nv, const double *p,
+                          int64_t ps, int n, double *partials, int *gate, GmStat *stat, hipStream_t str);
+// x (+ xs) += the cycle's correction
+hipError_t launch_gm_update(GmSys *sys, int ns, const double *U, int64_t stride, int64_t vs, double *x, int64_t xs,
+                            int n, hipStream_t str);
 
 // observe.hip (complex FP64 throughout)
 hipError_t launch_merge(const double *amnp, int64_t ldc, const int *order, const int *offset, const int *torder,

@@ -370,86 +370,310 @@ hipError_t launch_zaxpby(double ar, double ai, const double *x, double br, doubl
 }
 
 // ---------------------------------------------------------------------------
-// Block Gram-Schmidt pieces of the GMRES inner solver: nvec vectors V_j at
-// V + j*stride (complex), one vector w.
-// multi_zdot: partial[b*nvec + j] = sum over the block's share of conj(V_j) w
-// reduce_cols: out[j] = sum_b partial[b*nvec + j] (fixed order)
-// multi_axpy: w -= sum_j h_j V_j (sign = -1) or w += ... (sign = +1)
+// One Arnoldi step of GMRES for one or two systems, without the host: the
+// kernels of a step take both systems in one launch (blockIdx.z), and the
+// projections, the Givens rotations and the stop test stay on the device
+// (GmSys).  After the product p = T H v_j:
+//   dots   w = v_j - p, written to v_{j+1}; <v_i, w>, i <= j
+//   reduce h_i;   axpy  w -= sum_i h_i v_i
+//   dots, reduce, axpy once more (with the block sums of |w|^2)
+//   final  |w|, the column of H, its rotations, g, the stop test
+//   scale  v_{j+1} = w / |w|
+// Bound by reading the basis, twice per projection.  Four waves of a workgroup
+// take four basis vectors each of a chunk of 256 rows, a lane the rows of four
+// threads of a 256-wide reduction tree, so a sum needs no barrier and a step
+// has thousands of waves: 38 us on average over a cycle of 120 steps for the two
+// systems of a 1000-sphere cylinder, axpy 30 us, reduce + final + scale 30 us per
+// step (one workgroup per chunk and system going through the vectors with a tree
+// for each: 142 us the dots of both, and the host decided each step).  Sums run in
+// the order of that tree over the 512 chunks, whatever the launch, so an
+// Arnoldi vector's bits depend on the vectors before it only.
 // ---------------------------------------------------------------------------
-#define MV_MAX 128
-__global__ __launch_bounds__(KB) void multi_zdot_kernel(const cplx<double> *__restrict__ V, int64_t stride, int nvec,
-                                                        const cplx<double> *__restrict__ w, int n,
-                                                        cplx<double> *__restrict__ partials)
+#define GM_SPAN (KGRID * KB)  // rows i, i + GM_SPAN, ... belong to one thread of the tree
+static_assert(KB == 256, "gm kernels: 256-row chunks, four rows per lane");
+
+// the tree over a chunk's 256 threads, lane t holding threads t, t+64, t+128, t+192
+__device__ __forceinline__ cplx<double> tree256(const cplx<double> (&s)[4])
 {
-    __shared__ cplx<double> red[KB];
-    for (int j = 0; j < nvec; j++) {
-        cplx<double> s = cmk(0.0, 0.0);
-        const cplx<double> *v = V + (int64_t)j * stride;
-        for (int i = blockIdx.x * KB + threadIdx.x; i < n; i += gridDim.x * KB) cfma(s, cconj(v[i]), w[i]);
-        red[threadIdx.x] = s;
-        __syncthreads();
-        for (int h = KB / 2; h > 0; h >>= 1) {
-            if (threadIdx.x < h) red[threadIdx.x] = cadd(red[threadIdx.x], red[threadIdx.x + h]);
-            __syncthreads();
+    cplx<double> v = cadd(cadd(s[0], s[2]), cadd(s[1], s[3]));
+#pragma unroll
+    for (int d = 32; d; d >>= 1) v = cadd(v, cmk(__shfl_xor(v.re, d), __shfl_xor(v.im, d)));
+    return v;  // lane 0
+}
+
+__global__ __launch_bounds__(KB) void gm_dots_kernel(cplx<double> *__restrict__ V, int64_t stride, int64_t vs, int nv,
+                                                     const cplx<double> *__restrict__ P, int64_t ps, int n,
+                                                     const GmSys *__restrict__ sys, int pass,
+                                                     cplx<double> *__restrict__ part, int64_t region)
+{
+    if (!sys[blockIdx.z].active) return;
+    V += blockIdx.z * vs;
+    P += blockIdx.z * ps;
+    part += blockIdx.z * region;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int v0 = (blockIdx.y * 4 + wave) * 4;
+    if (v0 >= nv) return;
+    const cplx<double> *vj = V + (int64_t)(nv - 1) * stride;
+    cplx<double> *wn = V + (int64_t)nv * stride;
+    const bool first = v0 == 0 && !pass;
+    cplx<double> s[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) s[q][r] = cmk(0.0, 0.0);
+    for (int k0 = blockIdx.x * KB; k0 < n; k0 += GM_SPAN) {
+        cplx<double> w[4], v[4][4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int i = k0 + lane + 64 * r;
+            w[r] = cmk(0.0, 0.0);
+            if (i < n) w[r] = pass ? wn[i] : csub(vj[i], P[i]);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                v[q][r] = cmk(0.0, 0.0);
+                if (v0 + q < nv && i < n) v[q][r] = V[(int64_t)(v0 + q) * stride + i];
+            }
         }
-        if (threadIdx.x == 0) partials[(int64_t)j * gridDim.x + blockIdx.x] = red[0];
-        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int i = k0 + lane + 64 * r;
+            if (first && i < n) wn[i] = w[r];
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (i < n) cfma(s[q][r], cconj(v[q][r]), w[r]);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const cplx<double> t = tree256(s[q]);
+        if (lane == 0 && v0 + q < nv) part[(int64_t)(v0 + q) * gridDim.x + blockIdx.x] = t;
     }
 }
 
-// out[j] = sum over the nblk block partials of vector j (stored j-major);
-// one workgroup per vector, fixed reduction order
-__global__ __launch_bounds__(KB) void reduce_cols_kernel(const cplx<double> *__restrict__ partials, int nblk,
-                                                         cplx<double> *__restrict__ out)
+// h_i = sum over the chunks, one wave per i (chunks beyond the last are zero)
+__global__ __launch_bounds__(KB) void gm_reduce_kernel(int nv, int nch, GmSys *__restrict__ sys, int pass,
+                                                       const cplx<double> *__restrict__ part, int64_t region)
 {
-    __shared__ cplx<double> red[KB];
-    const int j = blockIdx.x;
+    GmSys &S = sys[blockIdx.z];
+    const int j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (!S.active || j >= nv) return;
+    part += blockIdx.z * region + (int64_t)j * nch;
+    cplx<double> s[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int b = lane + 64 * r;
+        s[r] = b < nch ? part[b] : cmk(0.0, 0.0);
+        if (b + KB < nch) s[r] = cadd(s[r], part[b + KB]);
+    }
+    const cplx<double> t = tree256(s);
+    if (lane == 0) S.h[pass][j] = t;
+}
+
+// w -= sum_i h_i v_i; second pass: block sums of |w|^2
+__global__ __launch_bounds__(KB) void gm_axpy_kernel(cplx<double> *__restrict__ V, int64_t stride, int64_t vs, int nv,
+                                                     int n, const GmSys *__restrict__ sys, int pass,
+                                                     cplx<double> *__restrict__ part, int64_t region)
+{
+    const GmSys &S = sys[blockIdx.z];
+    if (!S.active) return;
+    __shared__ cplx<double> hs[GM_M + 2], sh[KB];
+    V += blockIdx.z * vs;
+    for (int j = threadIdx.x; j < nv; j += KB) hs[j] = cscale(S.h[pass][j], -1.0);
+    __syncthreads();
     cplx<double> s = cmk(0.0, 0.0);
-    for (int b = threadIdx.x; b < nblk; b += KB) s = cadd(s, partials[(int64_t)j * nblk + b]);
-    red[threadIdx.x] = s;
+    for (int i = blockIdx.x * KB + threadIdx.x; i < n; i += GM_SPAN) {
+        cplx<double> a = V[(int64_t)nv * stride + i];
+#pragma unroll 8
+        for (int j = 0; j < nv; j++) cfma(a, hs[j], V[(int64_t)j * stride + i]);
+        V[(int64_t)nv * stride + i] = a;
+        cfma(s, cconj(a), a);
+    }
+    if (!pass) return;
+    sh[threadIdx.x] = s;
     __syncthreads();
-    for (int h = KB / 2; h > 0; h >>= 1) {
-        if (threadIdx.x < h) red[threadIdx.x] = cadd(red[threadIdx.x], red[threadIdx.x + h]);
+    if (threadIdx.x >= 64) return;
+    cplx<double> f[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) f[r] = sh[threadIdx.x + 64 * r];
+    s = tree256(f);
+    if (threadIdx.x == 0) part[blockIdx.z * region + blockIdx.x] = s;
+}
+
+__global__ __launch_bounds__(KB) void gm_scale_kernel(cplx<double> *__restrict__ v, int64_t vs, int n,
+                                                      const GmSys *__restrict__ sys)
+{
+    if (!sys[blockIdx.z].active) return;
+    const double f = sys[blockIdx.z].scale;
+    const int i = blockIdx.x * KB + threadIdx.x;
+    if (i < n) v[blockIdx.z * vs + i] = cscale(v[blockIdx.z * vs + i], f);
+}
+
+// |w|, column j of H through the earlier rotations and its own, g, and
+// the stop test (one workgroup per system); gate = any system active
+__global__ __launch_bounds__(KB) void gm_final_kernel(int nv, int nb, GmSys *__restrict__ sys, int ns,
+                                                      const cplx<double> *__restrict__ part, int64_t region,
+                                                      int *__restrict__ gate, GmStat *__restrict__ stat)
+{
+    typedef cplx<double> Z;
+    __shared__ Z col[GM_M + 1], sn[GM_M];
+    __shared__ double cs[GM_M], sq[KGRID];
+    int any = 0;
+    for (int q = 0; q < ns; q++) {
+        GmSys &S = sys[q];
+        if (!S.active) continue;  // uniform
+        const int j = nv - 1;
+        for (int b = threadIdx.x; b < nb; b += KB) sq[b] = part[q * region + b].re;
+        for (int i = threadIdx.x; i < nv; i += KB) {
+            col[i] = cadd(S.h[0][i], S.h[1][i]);
+            if (i < j) {
+                sn[i] = S.sn[i];
+                cs[i] = S.cs[i];
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double ww = 0.0;
+            for (int b = 0; b < nb; b++) ww += sq[b];
+            const double hn = sqrt(ww > 0.0 ? ww : 0.0);
+            Z *R = S.R + (j * (j + 1)) / 2;
+            Z cur = col[0];
+            for (int r = 0; r < j; r++) {  // earlier rotations on column j
+                const Z b = col[r + 1];
+                R[r] = cadd(cscale(cur, cs[r]), cmul(sn[r], b));
+                cur = csub(cscale(b, cs[r]), cmul(cconj(sn[r]), cur));
+            }
+            const double ca = sqrt(cur.re * cur.re + cur.im * cur.im), nu = sqrt(ca * ca + hn * hn);
+            double c = 0.0;
+            Z s = cmk(1.0, 0.0);
+            if (ca != 0.0) {
+                c = ca / nu;
+                s = cscale(cur, hn / (ca * nu));
+            }
+            R[j] = cadd(cscale(cur, c), cscale(s, hn));
+            S.cs[j] = c;
+            S.sn[j] = s;
+            const Z gj = S.g[j], gn = cmul(cmk(-s.re, s.im), gj);
+            S.g[j + 1] = gn;
+            S.g[j] = cscale(gj, c);
+            S.k = nv;
+            S.scale = 1.0 / hn;
+            S.err = (gn.re * gn.re + gn.im * gn.im) / S.bb;
+            S.done = S.err < S.eps || S.it0 + nv >= S.niter;
+            if (S.done || hn == 0.0 || nu == 0.0 || nv == S.m) S.active = 0;
+        }
+        __syncthreads();
+        any |= S.active;
+    }
+    if (threadIdx.x == 0) {
+        *gate = any;
+        for (int q = 0; q < ns; q++) stat[q] = {sys[q].err, sys[q].active, sys[q].done, sys[q].k};
+        __threadfence_system();  // stat is pinned host memory
+    }
+}
+
+// R y = g, back substitution (one workgroup per system), y in h[0]
+__global__ __launch_bounds__(128) void gm_solve_kernel(GmSys *__restrict__ sys)
+{
+    typedef cplx<double> Z;
+    GmSys &S = sys[blockIdx.x];
+    const int k = S.k, t = threadIdx.x;
+    __shared__ Z piv;
+    Z g = t < k ? S.g[t] : cmk(0.0, 0.0);
+    for (int r = k - 1; r >= 0; r--) {
+        const Z *R = S.R + (r * (r + 1)) / 2;
+        if (t == r) {
+            const Z d = R[r];
+            piv = d.re != 0.0 || d.im != 0.0 ? cdiv(g, d) : cmk(0.0, 0.0);
+            S.h[0][r] = piv;
+        }
+        __syncthreads();
+        if (t < r) g = csub(g, cmul(R[t], piv));
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[j] = red[0];
 }
 
-__global__ void multi_axpy_kernel(const cplx<double> *__restrict__ V, int64_t stride, int nvec,
-                                  const cplx<double> *__restrict__ h, double sign, cplx<double> *__restrict__ w, int n)
+// x += sum_{i < k} y_i v_i
+__global__ __launch_bounds__(KB) void gm_update_kernel(const cplx<double> *__restrict__ U, int64_t stride, int64_t vs,
+                                                       cplx<double> *__restrict__ x, int64_t xs, int n,
+                                                       const GmSys *__restrict__ sys)
 {
-    __shared__ cplx<double> hs[MV_MAX];
-    for (int j = threadIdx.x; j < nvec; j += blockDim.x) hs[j] = cscale(h[j], sign);
+    const GmSys &S = sys[blockIdx.z];
+    const int k = S.k;
+    __shared__ cplx<double> hs[GM_M + 2];
+    U += blockIdx.z * vs;
+    x += blockIdx.z * xs;
+    for (int j = threadIdx.x; j < k; j += KB) hs[j] = S.h[0][j];
     __syncthreads();
-    for (int i = blockIdx.x * KB + threadIdx.x; i < n; i += gridDim.x * KB) {
-        cplx<double> a = w[i];
-        for (int j = 0; j < nvec; j++) cfma(a, hs[j], V[(int64_t)j * stride + i]);
-        w[i] = a;
-    }
+    const int i = blockIdx.x * KB + threadIdx.x;
+    if (i >= n) return;
+    cplx<double> a = x[i];
+#pragma unroll 8
+    for (int j = 0; j < k; j++) cfma(a, hs[j], U[(int64_t)j * stride + i]);
+    x[i] = a;
 }
 
-int multi_vec_max() { return MV_MAX; }
-
-// out (device, nvec complex) = V^H w; partials needs KGRID*nvec complex
-hipError_t launch_multi_zdot(const double *V, int64_t stride, int nvec, const double *w, int n, double *partials,
-                             double *out, hipStream_t st)
+// start of a cycle (beta = 0: not a system of it)
+__global__ void gm_begin_kernel(GmSys *__restrict__ sys, int ns, GmStart a, GmStart b, int *__restrict__ gate)
 {
-    if (nvec <= 0) return hipSuccess;
-    hipLaunchKernelGGL(multi_zdot_kernel, dim3(KGRID), dim3(KB), 0, st, reinterpret_cast<const cplx<double> *>(V),
-                       stride / 2, nvec, reinterpret_cast<const cplx<double> *>(w), n,
-                       reinterpret_cast<cplx<double> *>(partials));
-    hipLaunchKernelGGL(reduce_cols_kernel, dim3(nvec), dim3(KB), 0, st, reinterpret_cast<const cplx<double> *>(partials),
-                       KGRID, reinterpret_cast<cplx<double> *>(out));
+    const int q = threadIdx.x;
+    if (q == 0) *gate = 1;
+    if (q >= ns) return;
+    const GmStart &st = q ? b : a;
+    GmSys &S = sys[q];
+    S.bb = st.bb;
+    S.eps = st.eps;
+    S.err = 0.0;
+    S.active = st.beta > 0.0;
+    S.done = 0;
+    S.k = 0;
+    S.it0 = st.it0;
+    S.niter = st.niter;
+    S.m = st.m;
+    S.scale = 1.0 / st.beta;
+    S.g[0] = cmk(st.beta, 0.0);
+}
+
+static int gm_chunks(int n) { return imn(KGRID, (n + KB - 1) / KB); }
+size_t gm_partials(int n) { return (size_t)2 * (GM_M + 1) * gm_chunks(n); }
+
+hipError_t launch_gm_begin(GmSys *sys, int ns, const GmStart *st, double *V, int64_t vs, int n, int *gate,
+                           hipStream_t str)
+{
+    if (ns < 1 || ns > 2) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(gm_begin_kernel, dim3(1), dim3(64), 0, str, sys, ns, st[0], st[ns - 1], gate);
+    hipLaunchKernelGGL(gm_scale_kernel, dim3((n + KB - 1) / KB, 1, ns), dim3(KB), 0, str, (cplx<double> *)V, vs / 2, n,
+                       sys);
     return hipGetLastError();
 }
 
-hipError_t launch_multi_axpy(const double *V, int64_t stride, int nvec, const double *h, double sign, double *w, int n,
-                             hipStream_t st)
+hipError_t launch_gm_step(GmSys *sys, int ns, double *V, int64_t stride, int64_t vs, int nv, const double *p,
+                          int64_t ps, int n, double *partials, int *gate, GmStat *stat, hipStream_t str)
 {
-    if (nvec <= 0) return hipSuccess;
-    if (nvec > MV_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(multi_axpy_kernel, dim3(KGRID), dim3(KB), 0, st, reinterpret_cast<const cplx<double> *>(V),
-                       stride / 2, nvec, reinterpret_cast<const cplx<double> *>(h), sign,
-                       reinterpret_cast<cplx<double> *>(w), n);
+    typedef cplx<double> Z;
+    if (ns < 1 || ns > 2 || nv < 1 || nv > GM_M) return hipErrorInvalidValue;
+    const int nch = gm_chunks(n);
+    const int64_t region = (int64_t)gm_partials(n) / 2;
+    Z *v = (Z *)V, *part = (Z *)partials;
+    for (int pass = 0; pass < 2; pass++) {
+        hipLaunchKernelGGL(gm_dots_kernel, dim3(nch, (nv + 15) / 16, ns), dim3(KB), 0, str, v, stride / 2, vs / 2, nv,
+                           (const Z *)p, ps / 2, n, sys, pass, part, region);
+        hipLaunchKernelGGL(gm_reduce_kernel, dim3((nv + 3) / 4, 1, ns), dim3(KB), 0, str, nv, nch, sys, pass, part,
+                           region);
+        hipLaunchKernelGGL(gm_axpy_kernel, dim3(nch, 1, ns), dim3(KB), 0, str, v, stride / 2, vs / 2, nv, n, sys, pass,
+                           part, region);
+    }
+    hipLaunchKernelGGL(gm_final_kernel, dim3(1), dim3(KB), 0, str, nv, nch, sys, ns, part, region, gate, stat);
+    hipLaunchKernelGGL(gm_scale_kernel, dim3((n + KB - 1) / KB, 1, ns), dim3(KB), 0, str, v + nv * (stride / 2), vs / 2,
+                       n, sys);
+    return hipGetLastError();
+}
+
+hipError_t launch_gm_update(GmSys *sys, int ns, const double *U, int64_t stride, int64_t vs, double *x, int64_t xs,
+                            int n, hipStream_t str)
+{
+    typedef cplx<double> Z;
+    hipLaunchKernelGGL(gm_solve_kernel, dim3(ns), dim3(128), 0, str, sys);
+    hipLaunchKernelGGL(gm_update_kernel, dim3((n + KB - 1) / KB, 1, ns), dim3(KB), 0, str, (const Z *)U, stride / 2,
+                       vs / 2, (Z *)x, xs / 2, n, sys);
     return hipGetLastError();
 }
