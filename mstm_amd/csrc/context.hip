@@ -82,6 +82,9 @@ enum {
 
 }  // namespace
 
+// a block of BiCG systems takes at most this much work space
+#define BICG_BLOCK_BYTES ((size_t)512 << 20)
+
 struct mstm_hip_ctx {
     int device = 0;
     hipStream_t st = nullptr;
@@ -166,6 +169,8 @@ struct mstm_hip_ctx {
         int vccd_T = 0, vccd_LS = 0;
         double *d_dist = nullptr, *d_dq = nullptr;
         size_t dist_bytes = 0, dq_bytes = 0;
+        unsigned char *d_blk = nullptr;  // work space of a block of column pairs (BicgBlock)
+        size_t blk_bytes = 0;
         double tmatrix_ms = 0;
         int tm_solves = 0;
         double *h_pin = nullptr;  // pinned host copies of each column pair's efficiencies and merge
@@ -381,6 +386,8 @@ static void release_observables(mstm_hip_ctx *c)
     dfree(c->obs.d_vccd);
     dfree(c->obs.d_dist);
     dfree(c->obs.d_dq);
+    dfree(c->obs.d_blk);
+    c->obs.blk_bytes = 0;
     if (c->obs.h_pin) hipHostFree(c->obs.h_pin);
     c->obs.h_pin = nullptr;
     c->obs.pin_bytes = 0;
@@ -730,22 +737,22 @@ static int direct_matvec_buf(mstm_hip_ctx *c, int nrhs, const double *ain, doubl
     const int *gate = c->gate;
     if (prec == MSTM_HIP_FP64) {
         HIPCHK(launch_prep_quad<double>(ain, 2 * c->neqns, (double *)xin, nrhs, flags, c->nsph, c->npad, L, c->d_order,
-                                   c->d_offset, c->d_an, c->st, gate));
+                                   c->d_offset, c->d_an, 1, c->st, gate));
         if (e0) hipEventRecord(e0, c->st);
         HIPCHK(launch_direct_tiles<double>((const double *)d.tab, c->d_tiles, c->ntiles, L, (const double *)xin,
-                                           (double *)part, c->npad, nr, G, c->st, gate));
+                                           (double *)part, c->npad, nr, G, 1, c->st, gate));
         if (e1) hipEventRecord(e1, c->st);
         HIPCHK(launch_reduce_quad<double>((const double *)part, c->nblocks * G, aout, 2 * c->neqns, nrhs, flags, c->nsph,
-                                          c->npad, L, c->d_order, c->d_offset, c->d_an, c->st, gate));
+                                          c->npad, L, c->d_order, c->d_offset, c->d_an, 1, c->st, gate));
     } else {
         HIPCHK(launch_prep_quad<float>(ain, 2 * c->neqns, (float *)xin, nrhs, flags, c->nsph, c->npad, L, c->d_order,
-                                  c->d_offset, c->d_an, c->st, gate));
+                                  c->d_offset, c->d_an, 1, c->st, gate));
         if (e0) hipEventRecord(e0, c->st);
         HIPCHK(launch_direct_tiles<float>((const float *)d.tab, c->d_tiles, c->ntiles, L, (const float *)xin,
-                                          (float *)part, c->npad, nr, G, c->st, gate));
+                                          (float *)part, c->npad, nr, G, 1, c->st, gate));
         if (e1) hipEventRecord(e1, c->st);
         HIPCHK(launch_reduce_quad<float>((const float *)part, c->nblocks * G, aout, 2 * c->neqns, nrhs, flags, c->nsph,
-                                         c->npad, L, c->d_order, c->d_offset, c->d_an, c->st, gate));
+                                         c->npad, L, c->d_order, c->d_offset, c->d_an, 1, c->st, gate));
     }
     if (e0) c->ev_prec.push_back(prec + 2 * (nr == 4));
     c->stats.matvecs[prec]++;
@@ -961,8 +968,8 @@ static int bicg2_dev(mstm_hip_ctx *c, int ns, int niter, const double *eps, cons
     c->gate = gate;
     HIPCHK(hipMemcpyAsync(S, hS, sizeof(BicgScal) * ns, hipMemcpyHostToDevice, c->st));
     // |b|^2
-    for (int s = 0; s < ns; s++) HIPCHK(launch_zdot(B[s], B[s], n, 1, pregion(c, s), nullptr, c->st));
-    HIPCHK(launch_bicg_scal(0, c->d_partials, region, S, ns, c->st, gate));
+    HIPCHK(launch_bicg_norm(B[0], (int64_t)V, n, c->d_partials, region, ns, c->st));
+    HIPCHK(launch_bicg_scal(0, c->d_partials, region, S, ns, n, c->st, gate));
     int rc = 0;
     bool act[2] = {true, ns == 2};
     if (!lazy) {
@@ -982,9 +989,12 @@ static int bicg2_dev(mstm_hip_ctx *c, int ns, int niter, const double *eps, cons
                 if (act[s]) rc = matvec(c, 1, X[s], Rr[s], f, prec, use_fft);
         if (rc) return rc;
     }
-    for (int s = 0; s < ns; s++)
-        if (act[s]) HIPCHK(launch_bicg_init(Rr[s], Q[s], W[s], P[s], B[s], X[s], n, pregion(c, s), c->st));
-    HIPCHK(launch_bicg_scal(1, c->d_partials, region, S, ns, c->st, gate));
+    {
+        const int s0 = act[0] ? 0 : 1, nact = act[0] && act[1] ? 2 : 1;
+        HIPCHK(launch_bicg_init(Rr[s0], Q[s0], W[s0], P[s0], B[s0], X[s0], (int64_t)V, 2 * (int64_t)V, n,
+                                pregion(c, s0), region, nact, c->st));
+    }
+    HIPCHK(launch_bicg_scal(1, c->d_partials, region, S, ns, n, c->st, gate));
     if (!lazy) {
         rc = sync_state();
         if (rc) return rc;
@@ -1001,10 +1011,10 @@ static int bicg2_dev(mstm_hip_ctx *c, int ns, int niter, const double *eps, cons
         else rc_ = matvec(c, 2, act[0] ? P[0] : P[1], act[0] ? AP[0] : AP[1], f4, prec, use_fft);
         if (rc_) return rc_;
         HIPCHK(launch_bicg_a_dev(AP[0], AW[0], P[0], W[0], 2 * (int64_t)V, n, pregion(c, 0), region, S, ns, c->st));
-        HIPCHK(launch_bicg_scal(2, c->d_partials, region, S, ns, c->st, gate));
+        HIPCHK(launch_bicg_scal(2, c->d_partials, region, S, ns, n, c->st, gate));
         HIPCHK(launch_bicg_b_dev(X[0], Rr[0], Q[0], P[0], AP[0], AW[0], (int64_t)V, 2 * (int64_t)V, S, n, pregion(c, 0),
                                  region, ns, c->st));
-        HIPCHK(launch_bicg_scal(3, c->d_partials, region, S, ns, c->st, gate));
+        HIPCHK(launch_bicg_scal(3, c->d_partials, region, S, ns, n, c->st, gate));
         HIPCHK(launch_bicg_c_dev(P[0], W[0], Rr[0], Q[0], (int64_t)V, 2 * (int64_t)V, S, n, ns, c->st));
         return 0;
     };
@@ -1039,6 +1049,119 @@ static int bicg2_dev(mstm_hip_ctx *c, int ns, int niter, const double *eps, cons
     for (int s = 0; s < ns; s++) {
         it[s] = act[s] ? iter : hS[s].it;  // ran out: niter + 1
         err[s] = hS[s].err;
+    }
+    return 0;
+}
+
+// ---------------------------------------------------------------------------
+// cbicg for a block of np column pairs (2 np systems, FP64, direct operator):
+// the T-matrix's columns of one degree share their operator, and a pair alone
+// leaves most of the chip idle on a small cluster (200 spheres of order 4: 67 us
+// per iteration, 31 of them the tiles; in blocks of up to 33 pairs 23 us per pair
+// and iteration, 19 of them the tiles, which then run at the rate of a full
+// chip: 335 -> 94 ms for the T-matrix of order 16).  Every system keeps its own recurrences, scalars, stop and count;
+// the kernels of a step take all systems, and a pair whose two systems have
+// stopped closes its gate.
+// ---------------------------------------------------------------------------
+struct BicgBlock {
+    int np = 0, G = 1;  // pairs, workgroups per tile of the product
+    double *x, *b, *pw, *cap, *r, *q, *partials, *xin, *part;
+    BicgScal *sc;
+    int *gate;
+};
+
+// the parts of a work space at base (null: sizes only); returns its bytes
+static size_t bicg_block_layout(const mstm_hip_ctx *c, unsigned char *base, BicgBlock &k)
+{
+    size_t o = 0;
+    const size_t V = sizeof(double) * 2 * c->kv_n, np = (size_t)k.np;
+    const size_t col = sizeof(double) * 2 * 4 * 2 * (size_t)c->npad * c->Lmax * (c->Lmax + 2);  // four product columns
+    auto put = [&](auto *&p, size_t bytes) {
+        p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + o);
+        o += (bytes + 255) / 256 * 256;
+    };
+    put(k.x, 2 * V * np);
+    put(k.b, 2 * V * np);
+    put(k.pw, 4 * V * np);
+    put(k.cap, 4 * V * np);
+    put(k.r, 2 * V * np);
+    put(k.q, 2 * V * np);
+    put(k.partials, sizeof(double) * 4 * (size_t)krylov_grid() * 2 * np);
+    put(k.xin, col * np);
+    put(k.part, col * np * c->nblocks * k.G);
+    put(k.sc, sizeof(BicgScal) * 2 * np);
+    put(k.gate, sizeof(int) * np);
+    return o;
+}
+
+// the block for np of the columns of one degree: as many pairs as the work
+// space may hold, split evenly, and workgroups per tile while the tiles of all
+// pairs are fewer than 2048.  Work space of 96 / 256 / 512 / 1024 MB, T-matrix:
+// 200 spheres 114 / 97 / 94 / 94 ms, 500 spheres 510 / 337 / 302 / 292 ms, 900
+// spheres 1492 (pairs alone) / 1492 / 1306 / 1291 ms.
+static BicgBlock bicg_block_plan(const mstm_hip_ctx *c, int np)
+{
+    const size_t limit = (size_t)BICG_BLOCK_BYTES;
+    BicgBlock k;
+    k.np = np;
+    while (k.np > 1 && bicg_block_layout(c, nullptr, k) > limit) {
+        const int parts = (np + k.np - 1) / k.np + 1;
+        k.np = std::min(k.np - 1, (np + parts - 1) / parts);
+    }
+    k.G = c->tgroups;
+    while (k.G > 1 && ((int64_t)c->ntiles * k.G * k.np > 2048 || bicg_block_layout(c, nullptr, k) > limit)) k.G /= 2;
+    return k;
+}
+
+// b in k.b; x in k.x = b at the start, the solutions at the end; hS: 2 np scalars
+static int bicg_block(mstm_hip_ctx *c, const BicgBlock &k, int niter, double eps, BicgScal *hS, int *it, double *err)
+{
+    const int n = c->neqns, np = k.np, ns = 2 * np, L = c->Lmax, K = 4;
+    const int64_t V = 2 * (int64_t)c->kv_n, region = 2 * (int64_t)krylov_grid();
+    const DirectOp &d = c->dop[MSTM_HIP_FP64];
+    auto product = [&](int ncol, const double *in, double *out, const int *f, const int *gate) -> int {
+        HIPCHK(launch_prep_quad<double>(in, (int)V, k.xin, ncol, f, c->nsph, c->npad, L, c->d_order, c->d_offset,
+                                        c->d_an, np, c->st, gate));
+        HIPCHK(launch_direct_tiles<double>((const double *)d.tab, c->d_tiles, c->ntiles, L, k.xin, k.part, c->npad,
+                                           ncol, k.G, np, c->st, gate));
+        HIPCHK(launch_reduce_quad<double>(k.part, c->nblocks * k.G, out, (int)V, ncol, f, c->nsph, c->npad, L,
+                                          c->d_order, c->d_offset, c->d_an, np, c->st, gate));
+        c->stats.matvecs[MSTM_HIP_FP64] += np;
+        return 0;
+    };
+    for (int s = 0; s < ns; s++) {
+        hS[s] = BicgScal{};
+        hS[s].eps = eps;
+    }
+    HIPCHK(hipMemcpyAsync(k.sc, hS, sizeof(BicgScal) * ns, hipMemcpyHostToDevice, c->st));
+    HIPCHK(launch_bicg_norm(k.b, V, n, k.partials, region, ns, c->st));
+    HIPCHK(launch_bicg_scal(0, k.partials, region, k.sc, ns, n, c->st, k.gate));
+    const int f2[2] = {2, 2}, f4[4] = {2, 3, 2, 3};
+    if (int rc = product(2, k.x, k.r, f2, k.gate)) return rc;
+    HIPCHK(launch_bicg_init(k.r, k.q, k.pw + V, k.pw, k.b, k.x, V, 2 * V, n, k.partials, region, ns, c->st));
+    HIPCHK(launch_bicg_scal(1, k.partials, region, k.sc, ns, n, c->st, k.gate));
+    bool any = true;
+    for (int iter = 0; iter < niter && any;) {
+        const int nst = std::min(K, niter - iter);
+        for (int q = 0; q < nst; q++) {
+            if (int rc = product(4, k.pw, k.cap, f4, k.gate)) return rc;
+            HIPCHK(launch_bicg_a_dev(k.cap, k.cap + V, k.pw, k.pw + V, 2 * V, n, k.partials, region, k.sc, ns, c->st));
+            HIPCHK(launch_bicg_scal(2, k.partials, region, k.sc, ns, n, c->st, k.gate));
+            HIPCHK(launch_bicg_b_dev(k.x, k.r, k.q, k.pw, k.cap, k.cap + V, V, 2 * V, k.sc, n, k.partials, region, ns,
+                                     c->st));
+            HIPCHK(launch_bicg_scal(3, k.partials, region, k.sc, ns, n, c->st, k.gate));
+            HIPCHK(launch_bicg_c_dev(k.pw, k.pw + V, k.r, k.q, V, 2 * V, k.sc, n, ns, c->st));
+        }
+        iter += nst;
+        HIPCHK(hipMemcpyAsync(hS, k.sc, sizeof(BicgScal) * ns, hipMemcpyDeviceToHost, c->st));
+        HIPCHK(hipStreamSynchronize(c->st));
+        any = false;
+        for (int s = 0; s < ns; s++) any |= hS[s].active != 0;
+    }
+    for (int s = 0; s < ns; s++) {
+        it[s] = hS[s].active ? niter + 1 : hS[s].it;  // ran out: niter + 1
+        err[s] = hS[s].err;
+        c->stats.iters_fp64 += hS[s].active ? niter : hS[s].it - hS[s].brk;
     }
     return 0;
 }
@@ -2594,20 +2717,45 @@ int mstm_hip_tmatrix_solution(mstm_hip_ctx *c, double eps, int niter, double con
     if (int rc = ensure_vccm(c, T, c->Lmax)) return rc;
     if (int rc = ensure_vccd(c, T, c->Lmax)) return rc;
     if (int rc = grow(c, &c->obs.d_dist, c->obs.dist_bytes, sizeof(double) * V * 2 * (2 * T + 1))) return rc;
-    if (int rc = grow(c, &c->obs.d_dq, c->obs.dq_bytes, sizeof(double) * 9 * nsph)) return rc;
     const size_t per_group = sizeof(double) * 8 * (size_t)bT;
+    // Column pairs solved together (plain solver): the widest block of any
+    // degree; without room for it the pairs go one by one.
+    int np = 1;
+    if (solver == MSTM_HIP_SOLVE_PLAIN) {
+        size_t need_blk = 0;
+        for (int l = 1; l <= T; l++) {
+            BicgBlock k = bicg_block_plan(c, 2 * l + 1);
+            need_blk = std::max(need_blk, bicg_block_layout(c, nullptr, k));
+            np = std::max(np, k.np);
+        }
+        if (np > 1 && (!c->obs.d_blk || c->obs.blk_bytes < need_blk)) {
+            dfree(c->obs.d_blk);
+            c->obs.blk_bytes = 0;
+            if (dalloc(&c->obs.d_blk, need_blk) == hipSuccess) c->obs.blk_bytes = need_blk;
+            else {
+                (void)hipGetLastError();
+                c->obs.d_blk = nullptr;
+                np = 1;
+            }
+        }
+        if (np > 1 && !c->dop[MSTM_HIP_FP64].ready)
+            if (int rc = mstm_hip_setup_direct(c, MSTM_HIP_FP64)) return rc;
+    }
     int G = std::min(nsph, 1024);
     G = (int)std::max<size_t>(1, std::min<size_t>((size_t)G, ((size_t)1 << 30) / per_group));
-    if (int rc = grow(c, &c->obs.d_part, c->obs.part_bytes, per_group * G)) return rc;
-    if (int rc = grow(c, &c->obs.d_a0, c->obs.a0_bytes, per_group)) return rc;
+    const int npm = (int)std::max<size_t>(1, std::min<size_t>((size_t)np, ((size_t)1 << 28) / (per_group * G)));  // merged together
+    if (int rc = grow(c, &c->obs.d_part, c->obs.part_bytes, per_group * G * npm)) return rc;
+    if (int rc = grow(c, &c->obs.d_a0, c->obs.a0_bytes, per_group * np)) return rc;
+    if (int rc = grow(c, &c->obs.d_dq, c->obs.dq_bytes, sizeof(double) * 9 * nsph * np)) return rc;
     // vol_radius (mstm-input-37.f90:1205-1211): real(4) exponent .333333
     double vr = 0.0;
     for (int i = 0; i < nsph; i++) vr += c->radius[i] * c->radius[i] * c->radius[i];
     vr = std::pow(vr, (double).333333f);
     const double vr2 = vr * vr;
-    // the per-pair copies land in pinned memory, so that they are
-    // asynchronous and the pair waits for the device only once
-    const size_t pin_need = sizeof(double) * ((size_t)9 * nsph + (size_t)8 * bT);
+    // the copies of a block land in pinned memory, so that they are
+    // asynchronous and the block waits for them only once
+    const size_t nq = (size_t)9 * nsph * np, na0 = (size_t)8 * bT * np;
+    const size_t pin_need = sizeof(double) * (nq + na0) + sizeof(BicgScal) * 2 * np;
     if (c->obs.pin_bytes < pin_need) {
         if (c->obs.h_pin) hipHostFree(c->obs.h_pin);
         c->obs.h_pin = nullptr;
@@ -2615,7 +2763,10 @@ int mstm_hip_tmatrix_solution(mstm_hip_ctx *c, double eps, int niter, double con
         HIPCHK(hipHostMalloc((void **)&c->obs.h_pin, pin_need, hipHostMallocDefault));
         c->obs.pin_bytes = pin_need;
     }
-    double *hq = c->obs.h_pin, *ha0 = c->obs.h_pin + (size_t)9 * nsph;
+    double *hq = c->obs.h_pin, *ha0 = c->obs.h_pin + nq;
+    BicgScal *hS = reinterpret_cast<BicgScal *>(ha0 + na0);
+    std::vector<int> it(2 * (size_t)np);
+    std::vector<double> err(2 * (size_t)np);
     std::vector<double> sq((size_t)3 * nsph, 0.0);
     double qt[3] = {0.0, 0.0, 0.0}, qeffold = 0.0;
     int64_t nt = 0;
@@ -2628,68 +2779,87 @@ int mstm_hip_tmatrix_solution(mstm_hip_ctx *c, double eps, int niter, double con
         const int b0 = l * (l + 2);
         HIPCHK(launch_distribute(l, c->d_order, c->d_offset, c->d_pos, nsph, c->Lmax, c->obs.r0, c->rimed,
                                  c->obs.d_vccd, c->obs.d_dist, n, std::min(nsph, 1024), c->st));
-        for (int k0 = -l; k0 <= l; k0++) {
-            // columns (k0, q = 1) and (k0, q = 2): two independent systems solved together
-            double *dp = c->obs.d_dist + V * 2 * (k0 + l);
-            for (int q = 0; q < 2; q++)
-                HIPCHK(launch_mie_mult(dp + V * q, b + V * q, nsph, c->d_order, c->d_offset, c->d_mieoff, c->d_an, 1,
-                                       0, c->Lmax, c->st));
-            int it[2] = {0, 0}, rc = 0;
-            double err[2] = {0.0, 0.0};
-            const double eps2[2] = {eps, eps};
-            if (solver == MSTM_HIP_SOLVE_PLAIN) {
-                HIPCHK(hipMemcpyAsync(x, b, sizeof(double) * 2 * V, hipMemcpyDeviceToDevice, c->st));
-                rc = bicg2_dev(c, 2, niter, eps2, b, x, MSTM_HIP_FP64, 0, it, err);
+        // columns (k0, q = 1) and (k0, q = 2): pairs of independent systems,
+        // one or a block of them solved together
+        const BicgBlock plan = np > 1 ? bicg_block_plan(c, 2 * l + 1) : BicgBlock{};
+        for (int k0 = -l; k0 <= l;) {
+            const int nk = np > 1 ? std::min(plan.np, l + 1 - k0) : 1;
+            const double *dp = c->obs.d_dist + V * 2 * (k0 + l);
+            const double *xs = x;
+            std::fill(it.begin(), it.end(), 0);
+            std::fill(err.begin(), err.end(), 0.0);
+            int rc = 0;
+            if (np > 1) {
+                BicgBlock k = plan;
+                k.np = nk;
+                bicg_block_layout(c, c->obs.d_blk, k);
+                HIPCHK(launch_mie_mult(dp, k.b, nsph, c->d_order, c->d_offset, c->d_mieoff, c->d_an, 1, 0, c->Lmax,
+                                       c->st, 2 * nk, (int64_t)V));
+                HIPCHK(hipMemcpyAsync(k.x, k.b, sizeof(double) * 2 * V * nk, hipMemcpyDeviceToDevice, c->st));
+                rc = bicg_block(c, k, niter, eps, hS, it.data(), err.data());
+                xs = k.x;
             } else {
-                HIPCHK(hipMemsetAsync(x, 0, sizeof(double) * 2 * V, c->st));
-                rc = refine2_dev(c, 2, niter, eps, b, x, 0, it, err, b);
-                for (int p = 0; p < 2 && !rc; p++)
-                    if (err[p] >= eps && it[p] < niter) {
-                        c->stats.lig_fallbacks++;
-                        HIPCHK(hipMemcpyAsync(x + V * p, b + V * p, sizeof(double) * V, hipMemcpyDeviceToDevice,
-                                              c->st));
-                        int it2 = 0;
-                        rc = bicg2_dev(c, 1, niter - it[p], &eps, b + V * p, x + V * p, MSTM_HIP_FP64, 0, &it2,
-                                       &err[p]);
-                        it[p] += it2;
-                    }
+                HIPCHK(launch_mie_mult(dp, b, nsph, c->d_order, c->d_offset, c->d_mieoff, c->d_an, 1, 0, c->Lmax,
+                                       c->st, 2, (int64_t)V));
+                const double eps2[2] = {eps, eps};
+                if (solver == MSTM_HIP_SOLVE_PLAIN) {
+                    HIPCHK(hipMemcpyAsync(x, b, sizeof(double) * 2 * V, hipMemcpyDeviceToDevice, c->st));
+                    rc = bicg2_dev(c, 2, niter, eps2, b, x, MSTM_HIP_FP64, 0, it.data(), err.data());
+                } else {
+                    HIPCHK(hipMemsetAsync(x, 0, sizeof(double) * 2 * V, c->st));
+                    rc = refine2_dev(c, 2, niter, eps, b, x, 0, it.data(), err.data(), b);
+                    for (int p = 0; p < 2 && !rc; p++)
+                        if (err[p] >= eps && it[p] < niter) {
+                            c->stats.lig_fallbacks++;
+                            HIPCHK(hipMemcpyAsync(x + V * p, b + V * p, sizeof(double) * V, hipMemcpyDeviceToDevice,
+                                                  c->st));
+                            int it2 = 0;
+                            rc = bicg2_dev(c, 1, niter - it[p], &eps, b + V * p, x + V * p, MSTM_HIP_FP64, 0, &it2,
+                                           &err[p]);
+                            it[p] += it2;
+                        }
+                }
             }
             if (rc) return rc;
-            c->obs.tm_solves += 2;
-            for (int q = 0; q < 2; q++) {
+            c->obs.tm_solves += 2 * nk;
+            for (int q = 0; q < 2 * nk; q++) {
                 *maxiter = std::max(*maxiter, it[q]);
                 *maxerr = std::max(*maxerr, err[q]);
                 if (it[q] > niter || err[q] > eps) *istat = 1;
             }
             // per-sphere efficiencies of each column (qefficiencyfactors, npol = 1)
-            HIPCHK(launch_qeff(x, dp, 2 * n, nsph, c->d_radius, c->d_order, c->d_offset, c->d_mieoff, c->d_an,
-                               c->rimed, c->obs.d_dq, c->st));
-            HIPCHK(hipMemcpyAsync(hq, c->obs.d_dq, sizeof(double) * 9 * nsph, hipMemcpyDeviceToHost, c->st));
-            // both columns merged to the origin at order l (target orders min(l, torder_i))
-            HIPCHK(launch_merge(x, n, c->d_order, c->d_offset, c->obs.d_torder, c->d_pos, nsph, l, c->Lmax,
-                                c->obs.r0, c->rimed, c->obs.d_vccm, c->obs.d_part, G, c->obs.d_a0, c->st));
-            HIPCHK(hipMemcpyAsync(ha0, c->obs.d_a0, sizeof(double) * 8 * b0, hipMemcpyDeviceToHost, c->st));
+            HIPCHK(launch_qeff(xs, dp, 2 * n, nsph, c->d_radius, c->d_order, c->d_offset, c->d_mieoff, c->d_an,
+                               c->rimed, c->obs.d_dq, c->st, nk));
+            HIPCHK(hipMemcpyAsync(hq, c->obs.d_dq, sizeof(double) * 9 * nsph * nk, hipMemcpyDeviceToHost, c->st));
+            // the columns merged to the origin at order l (target orders min(l, torder_i))
+            for (int p = 0; p < nk; p += npm)
+                HIPCHK(launch_merge(xs + 2 * V * p, n, c->d_order, c->d_offset, c->obs.d_torder, c->d_pos, nsph, l,
+                                    c->Lmax, c->obs.r0, c->rimed, c->obs.d_vccm, c->obs.d_part, G,
+                                    c->obs.d_a0 + (size_t)8 * b0 * p, c->st, std::min(npm, nk - p)));
+            HIPCHK(hipMemcpyAsync(ha0, c->obs.d_a0, sizeof(double) * 8 * b0 * nk, hipMemcpyDeviceToHost, c->st));
             HIPCHK(hipStreamSynchronize(c->st));
-            for (int q = 0; q < 2; q++) {
-                for (int i = 0; i < nsph; i++)
-                    for (int e = 0; e < 3; e++) sq[3 * i + e] += hq[9 * i + 3 * (q + 1) + e];
-                const double *a0 = ha0 + 4 * (size_t)b0 * q;  // [mode][b0] complex
-                const double d1 = -2.0 / vr2 * a0[2 * ((size_t)q * b0 + amn(k0, l, l))];
-                double d3 = 0.0;
-                for (int e = 0; e < 2 * b0; e++) d3 += a0[2 * e] * a0[2 * e] + a0[2 * e + 1] * a0[2 * e + 1];
-                d3 *= 2.0 / vr2;
-                qt[0] += d1;
-                qt[1] += d1 - d3;
-                qt[2] += d3;
-                for (int nn = 1; nn <= l; nn++)
-                    for (int m = -nn; m <= nn; m++)
-                        for (int p = 0; p < 2; p++) {
-                            const size_t e = (size_t)p * b0 + amn(m, nn, l);
-                            tmat[2 * nt] = a0[2 * e];
-                            tmat[2 * nt + 1] = a0[2 * e + 1];
-                            nt++;
-                        }
-            }
+            for (int p = 0; p < nk; p++, k0++)
+                for (int q = 0; q < 2; q++) {
+                    const double *hqp = hq + (size_t)9 * nsph * p;
+                    for (int i = 0; i < nsph; i++)
+                        for (int e = 0; e < 3; e++) sq[3 * i + e] += hqp[9 * i + 3 * (q + 1) + e];
+                    const double *a0 = ha0 + 4 * (size_t)b0 * (2 * p + q);  // [mode][b0] complex
+                    const double d1 = -2.0 / vr2 * a0[2 * ((size_t)q * b0 + amn(k0, l, l))];
+                    double d3 = 0.0;
+                    for (int e = 0; e < 2 * b0; e++) d3 += a0[2 * e] * a0[2 * e] + a0[2 * e + 1] * a0[2 * e + 1];
+                    d3 *= 2.0 / vr2;
+                    qt[0] += d1;
+                    qt[1] += d1 - d3;
+                    qt[2] += d3;
+                    for (int nn = 1; nn <= l; nn++)
+                        for (int m = -nn; m <= nn; m++)
+                            for (int h = 0; h < 2; h++) {
+                                const size_t e = (size_t)h * b0 + amn(m, nn, l);
+                                tmat[2 * nt] = a0[2 * e];
+                                tmat[2 * nt + 1] = a0[2 * e + 1];
+                                nt++;
+                            }
+                }
         }
         double qe[2] = {0.0, 0.0};
         for (int i = 0; i < nsph; i++)

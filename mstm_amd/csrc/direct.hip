@@ -138,8 +138,10 @@ __global__ void prep_quad_kernel(const cplx<double> *__restrict__ ain, int ldain
                                  const int *__restrict__ offset, const cplx<double> *__restrict__ an,
                                  const int *__restrict__ gate)
 {
-    if (gate && !*gate) return;
+    if (gate && !gate[blockIdx.y]) return;
     const int NK = Lp * (Lp + 3) / 2;
+    ain += (int64_t)blockIdx.y * nrhs * ldain;
+    xin += (int64_t)blockIdx.y * nr * npad * 4 * Lp * (Lp + 2);
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= (int64_t)nr * npad * NK) return;
     const int e = (int)(q % NK);
@@ -172,21 +174,22 @@ __global__ void prep_quad_kernel(const cplx<double> *__restrict__ ain, int ldain
 
 template <typename T>
 hipError_t launch_prep_quad(const double *ain, int ldain, T *xin, int nrhs, const int *flags, int nsph, int npad,
-                            int Lp, const int *order, const int *offset, const double *an, hipStream_t st,
+                            int Lp, const int *order, const int *offset, const double *an, int nq, hipStream_t st,
                             const int *gate)
 {
-    if (nrhs < 1 || nrhs > 4) return hipErrorInvalidValue;
+    if (nrhs < 1 || nrhs > 4 || nq < 1 || nq > 65535) return hipErrorInvalidValue;
     const int nr = nrhs > 2 ? 4 : 2, bs = 256;
     const int64_t n = (int64_t)nr * npad * (Lp * (Lp + 3) / 2);
-    hipLaunchKernelGGL(prep_quad_kernel<T>, dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0, st,
+    hipLaunchKernelGGL(prep_quad_kernel<T>, dim3((unsigned)((n + bs - 1) / bs), nq), dim3(bs), 0, st,
                        reinterpret_cast<const cplx<double> *>(ain), ldain / 2, xin, nrhs, flags4(flags, nrhs), nr,
                        nsph, npad, Lp, order, offset, reinterpret_cast<const cplx<double> *>(an), gate);
     return hipGetLastError();
 }
 template hipError_t launch_prep_quad<float>(const double *, int, float *, int, const int *, int, int, int, const int *,
-                                            const int *, const double *, hipStream_t, const int *);
+                                            const int *, const double *, int, hipStream_t, const int *);
 template hipError_t launch_prep_quad<double>(const double *, int, double *, int, const int *, int, int, int,
-                                             const int *, const int *, const double *, hipStream_t, const int *);
+                                             const int *, const int *, const double *, int, hipStream_t,
+                                             const int *);
 
 // ---------------------------------------------------------------------------
 // Post-op (sphereinteraction :158-168).  FFT operator: the result of one
@@ -250,13 +253,15 @@ __global__ __launch_bounds__(1024) void reduce_quad_kernel(const T *__restrict__
                                                           const cplx<double> *__restrict__ an,
                                                           const int *__restrict__ gate)
 {
-    if (gate && !*gate) return;  // uniform over the grid
+    if (gate && !gate[blockIdx.z]) return;  // uniform over the workgroup
     extern __shared__ double red[];  // [KS][SP][8 NB]
     typedef T vec __attribute__((ext_vector_type(VC)));
     const int NB = Lp * (Lp + 2), NK = Lp * (Lp + 3) / 2, U = 8 * NB / VC;
     const int sph0 = blockIdx.x * SP, rp = blockIdx.y;
     const int64_t stride = (int64_t)(nr / 2) * npad * U;  // one partial
-    const vec *p0 = reinterpret_cast<const vec *>(part) + ((int64_t)rp * npad + sph0) * U;
+    aout += (int64_t)blockIdx.z * nrhs * ldaout;
+    const vec *p0 = reinterpret_cast<const vec *>(part) + blockIdx.z * nparts * stride +
+                    ((int64_t)rp * npad + sph0) * U;
     const int nsp = imn(SP, npad - sph0);
     for (int e = threadIdx.x; e < KS * nsp * U; e += blockDim.x) {
         const int un = e % (nsp * U), j = e / (nsp * U);
@@ -310,28 +315,30 @@ __global__ __launch_bounds__(1024) void reduce_quad_kernel(const T *__restrict__
 template <typename T>
 hipError_t launch_reduce_quad(const T *partial, int nparts, double *aout, int ldaout, int nrhs, const int *flags,
                               int nsph, int npad, int Lp, const int *order, const int *offset, const double *an,
-                              hipStream_t st, const int *gate)
+                              int nq, hipStream_t st, const int *gate)
 {
-    if (nrhs < 1 || nrhs > 4) return hipErrorInvalidValue;
+    if (nrhs < 1 || nrhs > 4 || nq < 1 || nq > 65535) return hipErrorInvalidValue;
     const int nr = nrhs > 2 ? 4 : 2, NB = Lp * (Lp + 2);
     const int VC = 2 * cvec_unit(Lp, sizeof(T)), U = 8 * NB / VC;
     // about one unit per thread of 256; fewer than two workgroups per CU: one
     // sphere and 1024 threads each, and chains of about four loads
     int SP = imx(1, 256 / U), threads = 256;
-    if ((int64_t)nsph * (nr / 2) / SP < 512) {
+    if ((int64_t)nsph * (nr / 2) * nq / SP < 512) {
         SP = 1;
         threads = 1024;
     }
     const int KS = imx(1, imn(threads / (SP * U), (nparts + 3) / 4));
-    const dim3 g((nsph + SP - 1) / SP, nr / 2);
+    const dim3 g((nsph + SP - 1) / SP, nr / 2, nq);
     const size_t lds = sizeof(double) * (size_t)KS * SP * 8 * NB;
-#define RQ(V)                                                                                                              hipLaunchKernelGGL((reduce_quad_kernel<T, V>), g, dim3(threads), lds, st, partial, nparts,                                                    reinterpret_cast<cplx<double> *>(aout), ldaout / 2, nrhs, flags4(flags, nrhs), nr, nsph, npad,                         Lp, SP, KS, order, offset, reinterpret_cast<const cplx<double> *>(an), gate)
+#define RQ(V) \
+    hipLaunchKernelGGL((reduce_quad_kernel<T, V>), g, dim3(threads), lds, st, partial, nparts,                                                    reinterpret_cast<cplx<double> *>(aout), ldaout / 2, nrhs, flags4(flags, nrhs), nr, nsph, npad,                         Lp, SP, KS, order, offset, reinterpret_cast<const cplx<double> *>(an), gate)
     if (VC == 2) RQ(2);
     else RQ((sizeof(T) == 8 ? 2 : 4));
 #undef RQ
     return hipGetLastError();
 }
 template hipError_t launch_reduce_quad<float>(const float *, int, double *, int, int, const int *, int, int, int,
-                                              const int *, const int *, const double *, hipStream_t, const int *);
+                                              const int *, const int *, const double *, int, hipStream_t,
+                                              const int *);
 template hipError_t launch_reduce_quad<double>(const double *, int, double *, int, int, const int *, int, int, int,
-                                               const int *, const int *, const double *, hipStream_t, const int *);
+                                               const int *, const int *, const double *, int, hipStream_t, const int *);

@@ -26,21 +26,23 @@ hipError_t launch_direct_tables_both(double *tab64, float *tab32, const int2 *ti
 // the solver state cost little.
 // G (1, 2, 4, 8 or 16) workgroups per tile share its 16 steps; the partials
 // are then (partner block x G) per target.  Vectors in quad layout (tile.hpp).
+// nq > 1: that many sets of nr columns in one launch, each set's columns, sources
+// and partials behind those of the set before, set q gated by gate[q].
 template <typename T>
 hipError_t launch_direct_tiles(const T *tab, const int2 *tiles, int ntiles, int L, const T *xin, T *partial, int npad,
-                               int nr, int G, hipStream_t st, const int *gate = nullptr);
+                               int nr, int G, int nq, hipStream_t st, const int *gate = nullptr);
 template <> hipError_t launch_direct_tiles<float>(const float *, const int2 *, int, int, const float *, float *, int,
-                                                  int, int, hipStream_t, const int *);  // tile32.hip
+                                                  int, int, int, hipStream_t, const int *);  // tile32.hip
 template <> hipError_t launch_direct_tiles<double>(const double *, const int2 *, int, int, const double *, double *,
-                                                   int, int, int, hipStream_t, const int *);  // tile64.hip
+                                                   int, int, int, int, hipStream_t, const int *);  // tile64.hip
 template <typename T>
 hipError_t launch_prep_quad(const double *ain, int ldain, T *xin, int nrhs, const int *flags, int nsph, int npad,
-                            int Lp, const int *order, const int *offset, const double *an, hipStream_t st,
+                            int Lp, const int *order, const int *offset, const double *an, int nq, hipStream_t st,
                             const int *gate = nullptr);
 template <typename T>
 hipError_t launch_reduce_quad(const T *partial, int nparts, double *aout, int ldaout, int nrhs, const int *flags,
                               int nsph, int npad, int Lp, const int *order, const int *offset, const double *an,
-                              hipStream_t st, const int *gate = nullptr);
+                              int nq, hipStream_t st, const int *gate = nullptr);
 // FFT operator: up to two columns, [column][sphere][mode][packed (m,n)]
 template <typename T>
 hipError_t launch_prep(const double *ain, int ldain, T *xin, int nrhs, const int *flags, int nsph, int npad, int Lp,
@@ -53,13 +55,14 @@ hipError_t launch_post(const T *res, double *aout, int ldaout, int nrhs, const i
 hipError_t launch_mie(const double *x, const double *mre, const double *mim, double mmed, int nsph, double qeps,
                       int *order, double *an, int ldan, hipStream_t st);
 hipError_t launch_mie_mult(const double *ain, double *aout, int nsph, const int *order, const int *offset,
-                           const int *mieoff, const double *an, int idir, int inverse, int Lmax, hipStream_t st);
+                           const int *mieoff, const double *an, int idir, int inverse, int Lmax, hipStream_t st,
+                           int ncol = 1, int64_t ld = 0);  // ncol columns, ld doubles apart
 hipError_t launch_planewave(double *pmnp, int ld, int nsph, const double *pos, const int *order, const int *offset,
                             double alpha, double sinc, int dir, double rimed, hipStream_t st,
                             const int *excited = nullptr);
 hipError_t launch_qeff(const double *amnp, const double *pmnp, int ld, int nsph, const double *radius, const int *order,
                        const int *offset, const int *mieoff, const double *an, double rimed, double *qeff,
-                       hipStream_t st);
+                       hipStream_t st, int npair = 1);  // npair column pairs behind each other
 
 // krylov.hip (all vectors complex FP64, lengths in complex elements)
 int krylov_grid();
@@ -78,13 +81,17 @@ struct BicgScal {
 // cbk, csk.  The iteration number is counted on the device, so the launches
 // of an iteration are the same every time (they can be replayed from a
 // graph).  partials: region s of the system s at partials + s * region
-// (complex), one or two values per block.  gate (optional): set to 1 while
-// any system is active, else 0.
-hipError_t launch_bicg_scal(int step, const double *partials, int64_t region, BicgScal *st, int ns, hipStream_t st_,
-                            int *gate = nullptr);
+// (complex), one or two values per block of a vector of n elements.  gate
+// (optional): gate[q] set to 1 while system 2 q or 2 q + 1 is active, else 0.
+hipError_t launch_bicg_scal(int step, const double *partials, int64_t region, BicgScal *st, int ns, int n,
+                            hipStream_t st_, int *gate = nullptr);
 // the vector steps of ns systems in one launch: system s's vectors at the
 // given pointers plus s * sv (x, r, q) or s * sp (p, w, Ap, A^H w) doubles,
 // its partial sums at partials + s * region complex values
+hipError_t launch_bicg_norm(const double *b, int64_t sv, int n, double *partials, int64_t region, int ns,
+                            hipStream_t st);  // |b|^2
+hipError_t launch_bicg_init(double *cr, double *cq, double *cw, double *cp, const double *pnp, const double *anp,
+                            int64_t sv, int64_t sp, int n, double *partials, int64_t region, int ns, hipStream_t st);
 hipError_t launch_bicg_a_dev(double *cap, double *caw, const double *cp, const double *cw, int64_t sp, int n,
                              double *partials, int64_t region, const BicgScal *sc, int ns, hipStream_t st);
 hipError_t launch_bicg_b_dev(double *anp, double *cr, double *cq, const double *cp, const double *cap,
@@ -94,14 +101,6 @@ hipError_t launch_bicg_c_dev(double *cp, double *cw, const double *cr, const dou
                              const BicgScal *sc, int n, int ns, hipStream_t st);
 hipError_t launch_zdot(const double *a, const double *b, int n, int conj_a, double *partials, double *result,
                        hipStream_t st);
-hipError_t launch_bicg_a(double *cap, double *caw, const double *cp, const double *cw, int n, double *partials,
-                         hipStream_t st);
-hipError_t launch_bicg_b(double *anp, double *cr, double *cq, const double *cp, const double *cap, const double *caw,
-                         double cakr, double caki, int n, double *partials, hipStream_t st);
-hipError_t launch_bicg_c(double *cp, double *cw, const double *cr, const double *cq, double cbkr, double cbki, int n,
-                         hipStream_t st);
-hipError_t launch_bicg_init(double *cr, double *cq, double *cw, double *cp, const double *pnp, const double *anp, int n,
-                            double *partials, hipStream_t st);
 hipError_t launch_zaxpby(double ar, double ai, const double *x, double br, double bi, double *y, int n, hipStream_t st);
 // GMRES (restart length GM_M at most) with its small quantities on the device,
 // one or two systems; see krylov.hip
@@ -138,7 +137,8 @@ hipError_t launch_gm_update(GmSys *sys, int ns, const double *U, int64_t stride,
 // observe.hip (complex FP64 throughout)
 hipError_t launch_merge(const double *amnp, int64_t ldc, const int *order, const int *offset, const int *torder,
                         const double *pos, int nsph, int T, int LS, const double *r0, double rimed, const double *vccm,
-                        double *part, int G, double *a0, hipStream_t st);
+                        double *part, int G, double *a0, hipStream_t st,
+                        int npair = 1);  // npair column pairs behind each other
 hipError_t launch_scatmat(const double *a0, int T, int nang, const double *ct, const double *phi, double rimed,
                           double *sm, hipStream_t st);
 hipError_t launch_distribute(int l, const int *order, const int *offset, const double *pos, int nsph, int LS,

@@ -42,87 +42,6 @@ hipError_t launch_zdot(const double *a, const double *b, int n, int conj_a, doub
     return hipGetLastError();
 }
 
-// cap = cp - cap ; caw = cw - caw ; partial <cw, cap>   (:897-903)
-__global__ void bicg_a_kernel(cplx<double> *__restrict__ cap, cplx<double> *__restrict__ caw,
-                              const cplx<double> *__restrict__ cp, const cplx<double> *__restrict__ cw, int n,
-                              cplx<double> *__restrict__ partials)
-{
-    cplx<double> s = cmk(0.0, 0.0);
-    for (int i = blockIdx.x * KB + threadIdx.x; i < n; i += gridDim.x * KB) {
-        cplx<double> a = csub(cp[i], cap[i]);
-        cap[i] = a;
-        caw[i] = csub(cw[i], caw[i]);
-        cfma(s, cconj(cw[i]), a);
-    }
-    block_sum3(&s, 1);
-    if (threadIdx.x == 0) partials[blockIdx.x] = s;
-}
-
-// anp += cak cp ; cr -= cak cap ; cq -= conj(cak) caw ;
-// partials <cq, cr>, <cr, cr>   (:912-920)
-__global__ void bicg_b_kernel(cplx<double> *__restrict__ anp, cplx<double> *__restrict__ cr,
-                              cplx<double> *__restrict__ cq, const cplx<double> *__restrict__ cp,
-                              const cplx<double> *__restrict__ cap, const cplx<double> *__restrict__ caw,
-                              cplx<double> cak, int n, cplx<double> *__restrict__ partials)
-{
-    cplx<double> s[2] = {cmk(0.0, 0.0), cmk(0.0, 0.0)};
-    cplx<double> cakc = cconj(cak);
-    for (int i = blockIdx.x * KB + threadIdx.x; i < n; i += gridDim.x * KB) {
-        cplx<double> a = anp[i];
-        cfma(a, cak, cp[i]);
-        anp[i] = a;
-        cplx<double> r = cr[i];
-        cfma(r, cscale(cak, -1.0), cap[i]);
-        cr[i] = r;
-        cplx<double> q = cq[i];
-        cfma(q, cscale(cakc, -1.0), caw[i]);
-        cq[i] = q;
-        cfma(s[0], cconj(q), r);
-        cfma(s[1], cconj(r), r);
-    }
-    block_sum3(s, 2);
-    if (threadIdx.x == 0) {
-        partials[2 * blockIdx.x] = s[0];
-        partials[2 * blockIdx.x + 1] = s[1];
-    }
-}
-
-// cp = cr + cbk cp ; cw = cq + conj(cbk) cw   (:928-929)
-__global__ void bicg_c_kernel(cplx<double> *__restrict__ cp, cplx<double> *__restrict__ cw,
-                              const cplx<double> *__restrict__ cr, const cplx<double> *__restrict__ cq,
-                              cplx<double> cbk, int n)
-{
-    cplx<double> cbkc = cconj(cbk);
-    for (int i = blockIdx.x * KB + threadIdx.x; i < n; i += gridDim.x * KB) {
-        cplx<double> p = cr[i];
-        cfma(p, cbk, cp[i]);
-        cp[i] = p;
-        cplx<double> w = cq[i];
-        cfma(w, cbkc, cw[i]);
-        cw[i] = w;
-    }
-}
-
-// cr = pnp - anp + cr ; cq = cw = conj(cr) ; cp = cr ; partial sum cr*cr
-// (bilinear, :828-834)
-__global__ void bicg_init_kernel(cplx<double> *__restrict__ cr, cplx<double> *__restrict__ cq,
-                                 cplx<double> *__restrict__ cw, cplx<double> *__restrict__ cp,
-                                 const cplx<double> *__restrict__ pnp, const cplx<double> *__restrict__ anp, int n,
-                                 cplx<double> *__restrict__ partials)
-{
-    cplx<double> s = cmk(0.0, 0.0);
-    for (int i = blockIdx.x * KB + threadIdx.x; i < n; i += gridDim.x * KB) {
-        cplx<double> r = cadd(csub(pnp[i], anp[i]), cr[i]);
-        cr[i] = r;
-        cq[i] = cconj(r);
-        cw[i] = cconj(r);
-        cp[i] = r;
-        cfma(s, r, r);
-    }
-    block_sum3(&s, 1);
-    if (threadIdx.x == 0) partials[blockIdx.x] = s;
-}
-
 // y = a*x + b*y (complex scalars a, b)
 __global__ void zaxpby_kernel(cplx<double> a, const cplx<double> *__restrict__ x, cplx<double> b,
                               cplx<double> *__restrict__ y, int n)
@@ -135,6 +54,9 @@ __global__ void zaxpby_kernel(cplx<double> a, const cplx<double> *__restrict__ x
 }
 
 int krylov_grid() { return KGRID; }
+// blocks of the BiCG kernels: those of the full grid that have rows (the others'
+// partial sums would be zeros)
+static int bicg_grid(int n) { return imn(KGRID, (n + KB - 1) / KB); }
 
 // ---------------------------------------------------------------------------
 // Device-resident BiCG scalars (see BicgScal in kernels.hpp).  The vector
@@ -142,20 +64,21 @@ int krylov_grid() { return KGRID; }
 // may launch one iteration for both systems and learn only afterwards which
 // of them stopped.
 // ---------------------------------------------------------------------------
+// one workgroup per pair of systems
 __global__ __launch_bounds__(KB) void bicg_scal_kernel(int step, const cplx<double> *__restrict__ partials,
                                                        int64_t region, BicgScal *__restrict__ sc, int ns,
-                                                       int *__restrict__ gate)
+                                                       int nb, int *__restrict__ gate)
 {
     __shared__ cplx<double> red[2][KB];
-    const int nv = step == 3 ? 2 : 1;
-    for (int s = 0; s < ns; s++) {
+    const int nv = step == 3 ? 2 : 1, sa = 2 * blockIdx.x, se = imn(ns, sa + 2);
+    for (int s = sa; s < se; s++) {
         BicgScal &S = sc[s];
         const bool skip = step >= 1 && !S.active;  // uniform: read by all threads
         if (!skip) {
             const cplx<double> *p = partials + region * s;
             for (int q = 0; q < nv; q++) {
                 cplx<double> v = cmk(0.0, 0.0);
-                for (int b = threadIdx.x; b < KGRID; b += KB) v = cadd(v, p[(int64_t)nv * b + q]);
+                for (int b = threadIdx.x; b < nb; b += KB) v = cadd(v, p[(int64_t)nv * b + q]);
                 red[q][threadIdx.x] = v;
             }
             __syncthreads();
@@ -207,8 +130,8 @@ __global__ __launch_bounds__(KB) void bicg_scal_kernel(int step, const cplx<doub
     }
     if (gate && threadIdx.x == 0) {
         int any = 0;
-        for (int s = 0; s < ns; s++) any |= sc[s].active != 0;
-        *gate = any;
+        for (int s = sa; s < se; s++) any |= sc[s].active != 0;
+        gate[blockIdx.x] = any;
     }
 }
 
@@ -216,6 +139,39 @@ __global__ __launch_bounds__(KB) void bicg_scal_kernel(int step, const cplx<doub
 // its vectors at the base pointers plus s times a stride (complex elements:
 // sv for x, r, q; sp for p, w, Ap, A^H w), its scalars at sc[s] and its
 // partial sums at partials + s * region; a stopped system returns at once.
+// |b|^2
+__global__ void bicg_norm_kernel(const cplx<double> *__restrict__ b, int64_t sv, int n, cplx<double> *__restrict__ partials,
+                                 int64_t region)
+{
+    b += blockIdx.y * sv;
+    cplx<double> s = cmk(0.0, 0.0);
+    for (int i = blockIdx.x * KB + threadIdx.x; i < n; i += gridDim.x * KB) cfma(s, cconj(b[i]), b[i]);
+    block_sum3(&s, 1);
+    if (threadIdx.x == 0) partials[blockIdx.y * region + blockIdx.x] = s;
+}
+
+// cr = pnp - anp + cr ; cq = cw = conj(cr) ; cp = cr ; partial sum cr*cr
+// (bilinear, :828-834)
+__global__ void bicg_init_kernel(cplx<double> *__restrict__ cr, cplx<double> *__restrict__ cq,
+                                 cplx<double> *__restrict__ cw, cplx<double> *__restrict__ cp,
+                                 const cplx<double> *__restrict__ pnp, const cplx<double> *__restrict__ anp, int64_t sv,
+                                 int64_t sp, int n, cplx<double> *__restrict__ partials, int64_t region)
+{
+    const int64_t v = blockIdx.y * sv, p = blockIdx.y * sp;
+    cplx<double> s = cmk(0.0, 0.0);
+    for (int i = blockIdx.x * KB + threadIdx.x; i < n; i += gridDim.x * KB) {
+        cplx<double> r = cadd(csub(pnp[v + i], anp[v + i]), cr[v + i]);
+        cr[v + i] = r;
+        cq[v + i] = cconj(r);
+        cw[p + i] = cconj(r);
+        cp[p + i] = r;
+        cfma(s, r, r);
+    }
+    block_sum3(&s, 1);
+    if (threadIdx.x == 0) partials[blockIdx.y * region + blockIdx.x] = s;
+}
+
+// cap = cp - cap ; caw = cw - caw ; partial <cw, cap>   (:897-903)
 __global__ void bicg_a_dev_kernel(cplx<double> *__restrict__ cap, cplx<double> *__restrict__ caw,
                                   const cplx<double> *__restrict__ cp, const cplx<double> *__restrict__ cw, int64_t sp,
                                   int n, cplx<double> *__restrict__ partials, int64_t region,
@@ -239,6 +195,8 @@ __global__ void bicg_a_dev_kernel(cplx<double> *__restrict__ cap, cplx<double> *
     if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
+// anp += cak cp ; cr -= cak cap ; cq -= conj(cak) caw ;
+// partials <cq, cr>, <cr, cr>   (:912-920)
 __global__ void bicg_b_dev_kernel(cplx<double> *__restrict__ anp, cplx<double> *__restrict__ cr,
                                   cplx<double> *__restrict__ cq, const cplx<double> *__restrict__ cp,
                                   const cplx<double> *__restrict__ cap, const cplx<double> *__restrict__ caw,
@@ -276,6 +234,7 @@ __global__ void bicg_b_dev_kernel(cplx<double> *__restrict__ anp, cplx<double> *
     }
 }
 
+// cp = cr + cbk cp ; cw = cq + conj(cbk) cw   (:928-929)
 __global__ void bicg_c_dev_kernel(cplx<double> *__restrict__ cp, cplx<double> *__restrict__ cw,
                                   const cplx<double> *__restrict__ cr, const cplx<double> *__restrict__ cq, int64_t sv,
                                   int64_t sp, const BicgScal *__restrict__ sc, int n)
@@ -297,19 +256,35 @@ __global__ void bicg_c_dev_kernel(cplx<double> *__restrict__ cp, cplx<double> *_
     }
 }
 
-hipError_t launch_bicg_scal(int step, const double *partials, int64_t region, BicgScal *sc, int ns, hipStream_t st,
-                            int *gate)
+hipError_t launch_bicg_scal(int step, const double *partials, int64_t region, BicgScal *sc, int ns, int n,
+                            hipStream_t st, int *gate)
 {
-    if (ns < 1 || ns > 2 || step < 0 || step > 3) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(bicg_scal_kernel, dim3(1), dim3(KB), 0, st, step,
-                       reinterpret_cast<const cplx<double> *>(partials), region, sc, ns, gate);
+    if (ns < 1 || step < 0 || step > 3) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(bicg_scal_kernel, dim3((ns + 1) / 2), dim3(KB), 0, st, step,
+                       reinterpret_cast<const cplx<double> *>(partials), region, sc, ns, bicg_grid(n), gate);
+    return hipGetLastError();
+}
+hipError_t launch_bicg_norm(const double *b, int64_t sv, int n, double *partials, int64_t region, int ns,
+                            hipStream_t st)
+{
+    typedef cplx<double> Z;
+    hipLaunchKernelGGL(bicg_norm_kernel, dim3(bicg_grid(n), ns), dim3(KB), 0, st, (const Z *)b, sv / 2, n,
+                       (Z *)partials, region);
+    return hipGetLastError();
+}
+hipError_t launch_bicg_init(double *cr, double *cq, double *cw, double *cp, const double *pnp, const double *anp,
+                            int64_t sv, int64_t sp, int n, double *partials, int64_t region, int ns, hipStream_t st)
+{
+    typedef cplx<double> Z;
+    hipLaunchKernelGGL(bicg_init_kernel, dim3(bicg_grid(n), ns), dim3(KB), 0, st, (Z *)cr, (Z *)cq, (Z *)cw, (Z *)cp,
+                       (const Z *)pnp, (const Z *)anp, sv / 2, sp / 2, n, (Z *)partials, region);
     return hipGetLastError();
 }
 hipError_t launch_bicg_a_dev(double *cap, double *caw, const double *cp, const double *cw, int64_t sp, int n,
                              double *partials, int64_t region, const BicgScal *sc, int ns, hipStream_t st)
 {
     typedef cplx<double> Z;
-    hipLaunchKernelGGL(bicg_a_dev_kernel, dim3(KGRID, ns), dim3(KB), 0, st, (Z *)cap, (Z *)caw, (const Z *)cp,
+    hipLaunchKernelGGL(bicg_a_dev_kernel, dim3(bicg_grid(n), ns), dim3(KB), 0, st, (Z *)cap, (Z *)caw, (const Z *)cp,
                        (const Z *)cw, sp / 2, n, (Z *)partials, region, sc);
     return hipGetLastError();
 }
@@ -318,7 +293,7 @@ hipError_t launch_bicg_b_dev(double *anp, double *cr, double *cq, const double *
                              int64_t region, int ns, hipStream_t st)
 {
     typedef cplx<double> Z;
-    hipLaunchKernelGGL(bicg_b_dev_kernel, dim3(KGRID, ns), dim3(KB), 0, st, (Z *)anp, (Z *)cr, (Z *)cq, (const Z *)cp,
+    hipLaunchKernelGGL(bicg_b_dev_kernel, dim3(bicg_grid(n), ns), dim3(KB), 0, st, (Z *)anp, (Z *)cr, (Z *)cq, (const Z *)cp,
                        (const Z *)cap, (const Z *)caw, sv / 2, sp / 2, sc, n, (Z *)partials, region);
     return hipGetLastError();
 }
@@ -326,40 +301,8 @@ hipError_t launch_bicg_c_dev(double *cp, double *cw, const double *cr, const dou
                              const BicgScal *sc, int n, int ns, hipStream_t st)
 {
     typedef cplx<double> Z;
-    hipLaunchKernelGGL(bicg_c_dev_kernel, dim3(KGRID, ns), dim3(KB), 0, st, (Z *)cp, (Z *)cw, (const Z *)cr,
+    hipLaunchKernelGGL(bicg_c_dev_kernel, dim3(bicg_grid(n), ns), dim3(KB), 0, st, (Z *)cp, (Z *)cw, (const Z *)cr,
                        (const Z *)cq, sv / 2, sp / 2, sc, n);
-    return hipGetLastError();
-}
-hipError_t launch_bicg_a(double *cap, double *caw, const double *cp, const double *cw, int n, double *partials,
-                         hipStream_t st)
-{
-    typedef cplx<double> Z;
-    hipLaunchKernelGGL(bicg_a_kernel, dim3(KGRID), dim3(KB), 0, st, (Z *)cap, (Z *)caw, (const Z *)cp, (const Z *)cw, n,
-                       (Z *)partials);
-    return hipGetLastError();
-}
-hipError_t launch_bicg_b(double *anp, double *cr, double *cq, const double *cp, const double *cap, const double *caw,
-                         double cakr, double caki, int n, double *partials, hipStream_t st)
-{
-    typedef cplx<double> Z;
-    hipLaunchKernelGGL(bicg_b_kernel, dim3(KGRID), dim3(KB), 0, st, (Z *)anp, (Z *)cr, (Z *)cq, (const Z *)cp,
-                       (const Z *)cap, (const Z *)caw, cmk(cakr, caki), n, (Z *)partials);
-    return hipGetLastError();
-}
-hipError_t launch_bicg_c(double *cp, double *cw, const double *cr, const double *cq, double cbkr, double cbki, int n,
-                         hipStream_t st)
-{
-    typedef cplx<double> Z;
-    hipLaunchKernelGGL(bicg_c_kernel, dim3(KGRID), dim3(KB), 0, st, (Z *)cp, (Z *)cw, (const Z *)cr, (const Z *)cq,
-                       cmk(cbkr, cbki), n);
-    return hipGetLastError();
-}
-hipError_t launch_bicg_init(double *cr, double *cq, double *cw, double *cp, const double *pnp, const double *anp, int n,
-                            double *partials, hipStream_t st)
-{
-    typedef cplx<double> Z;
-    hipLaunchKernelGGL(bicg_init_kernel, dim3(KGRID), dim3(KB), 0, st, (Z *)cr, (Z *)cq, (Z *)cw, (Z *)cp,
-                       (const Z *)pnp, (const Z *)anp, n, (Z *)partials);
     return hipGetLastError();
 }
 hipError_t launch_zaxpby(double ar, double ai, const double *x, double br, double bi, double *y, int n, hipStream_t st)

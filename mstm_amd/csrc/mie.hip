@@ -127,11 +127,13 @@ hipError_t launch_mie(const double *x, const double *mre, const double *mim, dou
 __global__ void mie_mult_kernel(const cplx<double> *__restrict__ ain, cplx<double> *__restrict__ aout, int nsph,
                                 const int *__restrict__ order, const int *__restrict__ offset,
                                 const int *__restrict__ mieoff, const cplx<double> *__restrict__ an, int idir,
-                                int inverse, int Lmax)
+                                int inverse, int Lmax, int64_t ld)
 {
     int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int NBM = Lmax * (Lmax + 2);
     if (q >= (int64_t)nsph * NBM) return;
+    ain += blockIdx.y * ld;
+    aout += blockIdx.y * ld;
     int i = (int)(q / NBM), e = (int)(q % NBM);
     int L = order[i], NB = L * (L + 2);
     if (e >= NB) return;
@@ -159,13 +161,14 @@ __global__ void mie_mult_kernel(const cplx<double> *__restrict__ ain, cplx<doubl
 }
 
 hipError_t launch_mie_mult(const double *ain, double *aout, int nsph, const int *order, const int *offset,
-                           const int *mieoff, const double *an, int idir, int inverse, int Lmax, hipStream_t st)
+                           const int *mieoff, const double *an, int idir, int inverse, int Lmax, hipStream_t st,
+                           int ncol, int64_t ld)
 {
     int64_t n = (int64_t)nsph * Lmax * (Lmax + 2);
     int bs = 256;
-    hipLaunchKernelGGL(mie_mult_kernel, dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0, st,
+    hipLaunchKernelGGL(mie_mult_kernel, dim3((unsigned)((n + bs - 1) / bs), ncol), dim3(bs), 0, st,
                        reinterpret_cast<const cplx<double> *>(ain), reinterpret_cast<cplx<double> *>(aout), nsph, order,
-                       offset, mieoff, reinterpret_cast<const cplx<double> *>(an), idir, inverse, Lmax);
+                       offset, mieoff, reinterpret_cast<const cplx<double> *>(an), idir, inverse, Lmax, ld / 2);
     return hipGetLastError();
 }
 
@@ -274,6 +277,9 @@ __global__ void qeff_kernel(const cplx<double> *__restrict__ amnp, const cplx<do
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nsph) return;
+    amnp += (int64_t)blockIdx.y * 2 * ld;
+    pmnp += (int64_t)blockIdx.y * 2 * ld;
+    qeff += (int64_t)blockIdx.y * 9 * nsph;
     int L = order[i], NB = L * (L + 2);
     double xs = radius[i], xr = xs * rim;
     double psi[MIE_NMAX + 2];
@@ -351,10 +357,10 @@ __global__ void qeff_kernel(const cplx<double> *__restrict__ amnp, const cplx<do
 
 hipError_t launch_qeff(const double *amnp, const double *pmnp, int ld, int nsph, const double *radius, const int *order,
                        const int *offset, const int *mieoff, const double *an, double rimed, double *qeff,
-                       hipStream_t st)
+                       hipStream_t st, int npair)
 {
     int bs = 64;
-    hipLaunchKernelGGL(qeff_kernel, dim3((nsph + bs - 1) / bs), dim3(bs), 0, st,
+    hipLaunchKernelGGL(qeff_kernel, dim3((nsph + bs - 1) / bs, npair), dim3(bs), 0, st,
                        reinterpret_cast<const cplx<double> *>(amnp), reinterpret_cast<const cplx<double> *>(pmnp),
                        ld / 2, nsph, radius, order, offset, mieoff, reinterpret_cast<const cplx<double> *>(an), rimed,
                        qeff);

@@ -104,7 +104,7 @@ __global__ __launch_bounds__(OBS_THREADS) void merge_kernel(MergeArgs a)
 {
     const int g = blockIdx.x, G = gridDim.x, j = threadIdx.x, k = j - OBS_KOFF;
     const int T = a.T, b0 = T * (T + 2);
-    cplx<double> *P = reinterpret_cast<cplx<double> *>(a.part) + (int64_t)g * 4 * b0;
+    cplx<double> *P = reinterpret_cast<cplx<double> *>(a.part) + ((int64_t)blockIdx.y * G + g) * 4 * b0;
     for (int e = j; e < 4 * b0; e += OBS_THREADS) P[e] = cmk(0.0, 0.0);
 
     __shared__ double jw[128 + MSTM_MAX_L + 2];
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(OBS_THREADS) void merge_kernel(MergeArgs a)
     __shared__ cplx<double> act[OBS_NCH][3][MSTM_MAX_L + 1];
     __syncthreads();
 
-    const cplx<double> *A = reinterpret_cast<const cplx<double> *>(a.amnp);
+    const cplx<double> *A = reinterpret_cast<const cplx<double> *>(a.amnp) + (int64_t)blockIdx.y * 2 * a.ldc;
     for (int i = g; i < a.nsph; i += G) {
         const int L = a.order[i], bl = L * (L + 2);
         const int Ti = imn(T, a.torder[i]);
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(256) void merge_reduce_kernel(const double *part, i
     const int e = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / KS), j = threadIdx.x % KS;
     const bool live = e < 2 * b0;
     const int col = live ? e / b0 : 0, q = live ? e - col * b0 : 0;
-    const cplx<double> *P = reinterpret_cast<const cplx<double> *>(part);
+    const cplx<double> *P = reinterpret_cast<const cplx<double> *>(part) + (int64_t)blockIdx.y * G * 4 * b0;
     cplx<double> s0 = cmk(0.0, 0.0), s1 = cmk(0.0, 0.0);
     if (live) {
 #pragma unroll 4
@@ -293,23 +293,27 @@ __global__ __launch_bounds__(256) void merge_reduce_kernel(const double *part, i
         s1.im += __shfl_xor(s1.im, w, KS);
     }
     if (!live || j) return;
-    cplx<double> *O = reinterpret_cast<cplx<double> *>(a0) + (int64_t)col * 2 * b0;
+    cplx<double> *O = reinterpret_cast<cplx<double> *>(a0) + ((int64_t)blockIdx.y * 2 + col) * 2 * b0;
     O[q] = cadd(s0, s1);
     O[b0 + q] = csub(s0, s1);
 }
 
 hipError_t launch_merge(const double *amnp, int64_t ldc, const int *order, const int *offset, const int *torder,
                         const double *pos, int nsph, int T, int LS, const double *r0, double rimed, const double *vccm,
-                        double *part, int G, double *a0, hipStream_t st)
+                        double *part, int G, double *a0, hipStream_t st, int npair)
 {
-    if (T < 1 || T > OBS_KOFF || LS < 1 || LS > MSTM_MAX_L || G < 1) return hipErrorInvalidValue;
+    if (npair < 1 || npair > 65535 || T < 1 || T > OBS_KOFF || LS < 1 || LS > MSTM_MAX_L || G < 1) return hipErrorInvalidValue;
     MergeArgs a{amnp, ldc, order, offset, torder, pos, nsph, T, LS, r0[0], r0[1], r0[2], rimed, vccm, part};
-    hipLaunchKernelGGL(merge_kernel, dim3(G), dim3(OBS_THREADS), 0, st, a);
+    hipLaunchKernelGGL(merge_kernel, dim3(G, npair), dim3(OBS_THREADS), 0, st, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const int64_t n = 2 * T * (T + 2);
-    if (G >= 64) hipLaunchKernelGGL(merge_reduce_kernel<16>, dim3((unsigned)((n * 16 + 255) / 256)), dim3(256), 0, st, part, G, T, a0);
-    else hipLaunchKernelGGL(merge_reduce_kernel<4>, dim3((unsigned)((n * 4 + 255) / 256)), dim3(256), 0, st, part, G, T, a0);
+    if (G >= 64)
+        hipLaunchKernelGGL(merge_reduce_kernel<16>, dim3((unsigned)((n * 16 + 255) / 256), npair), dim3(256), 0, st,
+                           part, G, T, a0);
+    else
+        hipLaunchKernelGGL(merge_reduce_kernel<4>, dim3((unsigned)((n * 4 + 255) / 256), npair), dim3(256), 0, st,
+                           part, G, T, a0);
     return hipGetLastError();
 }
 

@@ -367,24 +367,32 @@ template <typename T, int L> constexpr int tile_waves() { return sizeof(T) == 4 
 // two workgroups of two (NRL = 2) where the staged sources of four columns
 // would leave one workgroup per CU.  The two are numbered 8 apart: workgroups
 // are dealt to MI355X's 8 XCDs round robin, so they run on one XCD and the
-// second reads the table group from its L2.
+// second reads the table group from its L2.  nq sets of columns (a block
+// of BiCG systems; sources, partials and gates one set after the other) are
+// further workgroups of that kind: all sets of a unit run side by side.
 template <typename T, int L, int NR, int NRL>
 __global__ __launch_bounds__(64 * NRL) __attribute__((amdgpu_waves_per_eu(tile_waves<T, L>()))) void tile_kernel(
     const T *__restrict__ tab, const int2 *__restrict__ tiles, int nunits, const T *__restrict__ xin,
-    T *__restrict__ part, int npad, int G, const int *__restrict__ gate)
+    T *__restrict__ part, int npad, int G, int nq, const int *__restrict__ gate)
 {
-    if (gate && !*gate) return;  // the issuing solver has stopped every system
     typedef cplx<T> Z;
     typedef TileShape<T, L, NRL> H;
     typedef typename vec16<T>::type V;
     constexpr int S = H::S, RP = H::RP;
     constexpr int NH = NR / NRL;  // workgroups per (tile, step group)
     int u = blockIdx.x, h = 0;
-    if constexpr (NH > 1) {
-        u = (int)(blockIdx.x / (8 * NH)) * 8 + (int)(blockIdx.x % 8);
-        h = (int)(blockIdx.x / 8) % NH;
-        if (u >= nunits) return;  // the grid is padded to whole groups of 8 NH
+    if (NH * nq > 1) {
+        const int sub = (int)(blockIdx.x / 8) % (NH * nq);
+        u = (int)(blockIdx.x / (8 * NH * nq)) * 8 + (int)(blockIdx.x % 8);
+        if (u >= nunits) return;  // the grid is padded to whole groups of 8 NH nq
+        h = sub % NH;
+        const int q = sub / NH;
+        const int64_t col = (int64_t)NR * 4 * npad * L * (L + 2);  // one set of sources, or one partial
+        xin += q * col;
+        part += q * col * (npad / MSTM_SLOTS) * G;
+        if (gate) gate += q;
     }
+    if (gate && !*gate) return;  // the issuing solver has stopped every system of the set
     const int tile = u / G, g = u - tile * G;
     const int s0 = g * (S / G), s1 = s0 + S / G;
     const int2 bt = tiles[tile];
@@ -397,28 +405,29 @@ __global__ __launch_bounds__(64 * NRL) __attribute__((amdgpu_waves_per_eu(tile_w
 
 template <typename T, int L>
 static hipError_t tile_launch(const T *tab, const int2 *tiles, int ntiles, const T *x, T *p, int npad, int nr, int G,
-                              hipStream_t st, const int *gate)
+                              int nq, hipStream_t st, const int *gate)
 {
     constexpr int NRL = tile_cols4(L, sizeof(T));
     const int nu = ntiles * G;
+    auto grid = [&](int per) { return dim3((unsigned)(per == 1 ? nu : (nu + 7) / 8 * 8 * per)); };
     if (nr == 2)
-        hipLaunchKernelGGL((tile_kernel<T, L, 2, 2>), dim3((unsigned)nu), dim3(128), 0, st, tab, tiles, nu, x, p, npad,
-                           G, gate);
+        hipLaunchKernelGGL((tile_kernel<T, L, 2, 2>), grid(nq), dim3(128), 0, st, tab, tiles, nu, x, p, npad, G, nq,
+                           gate);
     else
-        hipLaunchKernelGGL((tile_kernel<T, L, 4, NRL>), dim3((unsigned)(NRL == 4 ? nu : (nu + 7) / 8 * 16)),
-                           dim3(64 * NRL), 0, st, tab, tiles, nu, x, p, npad, G, gate);
+        hipLaunchKernelGGL((tile_kernel<T, L, 4, NRL>), grid(nq * (4 / NRL)), dim3(64 * NRL), 0, st, tab, tiles, nu, x,
+                           p, npad, G, nq, gate);
     return hipGetLastError();
 }
 
 template <typename T>
 static hipError_t tile_dispatch(const T *tab, const int2 *tiles, int ntiles, int L, const T *xin, T *partial, int npad,
-                                int nr, int G, hipStream_t st, const int *gate)
+                                int nr, int G, int nq, hipStream_t st, const int *gate)
 {
-    if (nr != 2 && nr != 4) return hipErrorInvalidValue;
+    if ((nr != 2 && nr != 4) || nq < 1) return hipErrorInvalidValue;
     if (G < 1 || G > MSTM_SLOTS || MSTM_SLOTS % G) return hipErrorInvalidValue;
     switch (L) {
 #define CASE(LL)                                                                                                       \
-    case LL: return tile_launch<T, LL>(tab, tiles, ntiles, xin, partial, npad, nr, G, st, gate);
+    case LL: return tile_launch<T, LL>(tab, tiles, ntiles, xin, partial, npad, nr, G, nq, st, gate);
 #ifdef MSTM_TILE_L_ONLY
         CASE(MSTM_TILE_L_ONLY)
 #else

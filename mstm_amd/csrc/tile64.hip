@@ -4,7 +4,8 @@
 
 template <>
 hipError_t launch_direct_tiles<double>(const double *tab, const int2 *tiles, int ntiles, int L, const double *xin,
-                                    double *partial, int npad, int nr, int G, hipStream_t st, const int *gate)
+                                    double *partial, int npad, int nr, int G, int nq, hipStream_t st,
+                                    const int *gate)
 {
-    return tile_dispatch<double>(tab, tiles, ntiles, L, xin, partial, npad, nr, G, st, gate);
+    return tile_dispatch<double>(tab, tiles, ntiles, L, xin, partial, npad, nr, G, nq, st, gate);
 }

@@ -1,0 +1,39 @@
+"""T-matrix columns solved in blocks (plain solver) against the pair-by-pair
+mixed solver: one sphere, one and several sphere blocks with remainders,
+spheres of unequal order, and a cluster whose degrees take several blocks of
+unequal width.
+
+Both stop at |r|^2/|b|^2 < 1e-14, so each column carries a relative residual of
+1e-7 at most; times a condition below 1e2 that is 1e-5 of the largest element."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _cluster(n, x, spread):
+    from mstm_amd import geometry as G
+
+    c = G.rsa_in_sphere(n, x, 0.12, seed=11, ri=1.5 + 0.01j)
+    radius = c.radius.copy()
+    radius[1::3] *= 1.0 - spread
+    return c.pos, radius, c.ri
+
+
+@pytest.mark.parametrize("n,x,spread", [(1, 1.0, 0.0), (2, 0.3, 0.0), (16, 0.8, 0.5), (17, 1.2, 0.0), (40, 0.6, 0.3),
+                                        (300, 2.2, 0.2)])
+def test_blocks_match_pairs(gpu_ctx, n, x, spread):
+    from mstm_amd.solver import SOLVE_MIXED, SOLVE_PLAIN
+
+    gpu_ctx.set_spheres(*_cluster(n, x, spread), 1.0, 1e-6)
+    r = gpu_ctx.tmatrix_solution(eps=1e-14, niter=2000, conveps=1e-3, solver=SOLVE_PLAIN)
+    m = gpu_ctx.tmatrix_solution(eps=1e-14, niter=2000, conveps=1e-3, solver=SOLVE_MIXED)
+    assert r["istat"] == 0 and r["T"] == m["T"]
+    for k in ("tmat", "sqeff", "qteff"):
+        assert np.abs(r[k] - m[k]).max() <= 1e-5 * np.abs(m[k]).max(), k
+
+
+def test_blocks_iteration_limit(gpu_ctx):
+    gpu_ctx.set_spheres(*_cluster(40, 1.0, 0.0), 1.0, 1e-6)
+    r = gpu_ctx.tmatrix_solution(eps=1e-14, niter=3, conveps=1e-3)
+    assert r["istat"] == 1 and r["maxiter"] == 4 and r["maxerr"] > 1e-14
