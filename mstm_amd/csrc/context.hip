@@ -1777,6 +1777,7 @@ static int lu_setup(mstm_hip_ctx *c)
     HIPCHK(hipMemcpyAsync(&err, c->lu.err, sizeof(int), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     c->lu.factor_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t1).count();
+    if (err & 2) return fail(c, MSTM_HIP_EHIP, "direct solver: the workgroups of a panel did not meet");
     if (err) return fail(c, MSTM_HIP_EARG, "direct solver: lu decomposition failed (a zero row)");
     c->lu.ready = true;
     return 0;

@@ -25,8 +25,6 @@
 
 #define LU_NB 32
 #define LU_GROUP 4  // panels per trailing update
-#define LU_PANEL_THREADS 1024
-#define LU_PANEL_ONE_WG_ROWS 512  // longer panels: pivot/pick/update launches per column
 #define LU_SOLVE_THREADS 1024
 
 namespace {
@@ -78,238 +76,253 @@ __global__ __launch_bounds__(256) void lu_rowscale_kernel(const zc *A, int n, do
     }
 }
 
-// Factor columns c0..c0+nb-1 (rows c0..n-1) with the scaled pivot rule; the
-// row swaps are applied inside the panel only and recorded in piv.
-__global__ __launch_bounds__(LU_PANEL_THREADS) void lu_panel_kernel(zc *A, int n, int c0, int nb, double *vv,
-                                                                    int *piv)
+// ---------------------------------------------------------------------------
+// Panel: columns c0..c0+nb-1 (rows c0..n-1) with the scaled pivot rule, one
+// launch.  A thread keeps one row of the panel, the columns not yet eliminated
+// in registers (x[0] is column j), its multipliers in LDS; a workgroup has 256
+// rows.  Per column the workgroups exchange their candidates for the pivot and
+// every workgroup picks the same one:
+//   each workgroup  its maximum of vv(i)|a(i,j)| (ties to the larger row), and
+//                   the panel row it belongs to; the first one also row j
+//   all             the largest of them; its row is row j of U
+//   the two rows' owners swap them, every row below takes the rank-1 update
+// The exchange needs no fence: a word carries 32 bits of data and the column's
+// number, and a reader polls a word until the number is there.  Two sets of
+// words alternate: a workgroup publishes column j+2 only after all have
+// published j+1, hence read j.  All workgroups (64 at most) are resident, each
+// waiting only for workgroups of its own launch; a wait is bounded.  The rest
+// of a column's update runs while the next column's candidates travel.
+// Bound by latency: 8400 equations, 111 us for 32 columns, 8300 cycles each (two
+// trips through memory 2400, the pivot's row into LDS and the barrier 1500, the
+// update 2500, the pivot's reciprocal and the next column 1500) whatever the
+// number of workgroups; a pick and an update launch per column took 275 us, the
+// panels of the whole factorization 72 ms, now 29 ms.
+// ---------------------------------------------------------------------------
+#define LU_MAX_BLOCKS 64                    // workgroups of a panel
+#define LU_LL_ROW (4 * LU_NB)               // words of a panel row: two per double
+#define LU_LL_HEAD 4                        // a workgroup's candidate: value (2 words), row
+#define LU_LL_SET (LU_MAX_BLOCKS * LU_LL_HEAD + (LU_MAX_BLOCKS + 1) * LU_LL_ROW + 4)
+#define LU_SPIN (1 << 24)                   // polls of a wait (about half a microsecond each)
+typedef unsigned long long lu_word;
+
+__device__ __forceinline__ void ll_put(lu_word *p, unsigned v, unsigned seq)
 {
-    __shared__ double sval[LU_PANEL_THREADS / 64];
-    __shared__ int sidx[LU_PANEL_THREADS / 64];
-    __shared__ int imax_s;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    __hip_atomic_store(p, ((lu_word)v << 32) | seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void ll_put(lu_word *p, double v, unsigned seq)
+{
+    const lu_word b = (lu_word)__double_as_longlong(v);
+    ll_put(p, (unsigned)(b >> 32), seq);
+    ll_put(p + 1, (unsigned)b, seq);
+}
+// a double and, where idx is not null, the index behind it, once they carry
+// seq; act: lanes that wait.  False if the wait ran out.
+__device__ __forceinline__ bool ll_get(const lu_word *p, bool act, unsigned seq, double &v, int *idx)
+{
+    lu_word h = 0, l = 0, x = 0;
+    for (int t = 0; t < LU_SPIN; t++) {
+        bool ok = true;
+        if (act) {
+            h = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            l = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (idx) x = __hip_atomic_load(p + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ok = (unsigned)h == seq && (unsigned)l == seq && (!idx || (unsigned)x == seq);
+        }
+        if (__all(ok)) {
+            v = __longlong_as_double((long long)(((h >> 32) << 32) | (l >> 32)));
+            if (idx) *idx = (int)(x >> 32);
+            return true;
+        }
+    }
+    return false;
+}
+
+__global__ void lu_clear_kernel(lu_word *ll, int n)
+{
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) ll[i] = 0;
+}
+
+// the largest value of a wave's lanes, the same in all (row shifts and row
+// broadcasts; lane 63 has it)
+template <int CTRL, int MASK> __device__ __forceinline__ double dpp_max(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = (int)b, hi = (int)(b >> 32);
+    const unsigned l2 = (unsigned)__builtin_amdgcn_update_dpp(lo, lo, CTRL, MASK, 0xf, false);
+    const unsigned h2 = (unsigned)__builtin_amdgcn_update_dpp(hi, hi, CTRL, MASK, 0xf, false);
+    return fmax(v, __longlong_as_double((long long)(((lu_word)h2 << 32) | l2)));
+}
+__device__ __forceinline__ double wave_max(double v)
+{
+    v = dpp_max<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
+    v = dpp_max<0x112, 0xf>(v);
+    v = dpp_max<0x114, 0xf>(v);
+    v = dpp_max<0x118, 0xf>(v);
+    v = dpp_max<0x142, 0xa>(v);  // row_bcast 15, 31
+    v = dpp_max<0x143, 0xc>(v);
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, 63);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), 63);
+    return __longlong_as_double((long long)(((lu_word)hi << 32) | lo));
+}
+// the last lane that holds the wave's maximum v (-1: no candidate)
+__device__ __forceinline__ int last_lane(double mine, double v)
+{
+    return v < 0.0 ? -1 : 63 - __clzll((long long)__ballot(mine == v));
+}
+
+__global__ __launch_bounds__(256) void lu_panel_kernel(zc *A, int n, int c0, int nb, double *vv, int *piv, lu_word *ll,
+                                                       int *err)
+{
+    __shared__ double sv[4], vvj;
+    __shared__ int si[4], six;
+    // the pivot's row and row j of the panel, zeros behind (two sets: the last
+    // column's are read until its update is complete)
+    __shared__ zc prow2[2][2][2 * LU_NB];
+    __shared__ zc ls[LU_NB][256];  // multipliers of the columns eliminated
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, blk = blockIdx.x, nblk = gridDim.x;
+    const int i = c0 + blk * 256 + tid;
+    const bool mine = i < n;
+    zc x[LU_NB];
+#pragma unroll
+    for (int k = 0; k < LU_NB; k++) x[k] = mine && k < nb ? A[(int64_t)(c0 + k) * n + i] : cmk(0.0, 0.0);
+    double vi = mine ? vv[i] : 0.0;
+    prow2[tid >> 7][(tid >> 6) & 1][lane] = cmk(0.0, 0.0);
+    zc l = cmk(0.0, 0.0);  // the row's multiplier of the last column
+    const zc *plast = nullptr;
     for (int jj = 0; jj < nb; jj++) {
         const int j = c0 + jj;
-        zc *colj = A + (int64_t)j * n;
-        // pivot search: max vv(i)|a(i,j)|, ties to the larger row (as '.ge.')
-        double bv = -1.0;
-        int bi = -1;
-        for (int i = j + tid; i < n; i += LU_PANEL_THREADS) {
-            const double d = vv[i] * zabs(colj[i]);
-            if (d >= bv) {
-                bv = d;
-                bi = i;
-            }
+        zc *crow = prow2[jj & 1][0], *jrow = prow2[jj & 1][1];
+        const unsigned seq = (unsigned)j + 1;
+        lu_word *set = ll + (jj & 1) * LU_LL_SET, *rows = set + LU_MAX_BLOCKS * LU_LL_HEAD,
+                *rowj = rows + LU_MAX_BLOCKS * LU_LL_ROW;
+        double d = -1.0;  // no candidate
+        if (mine && i >= j) {  // (vv|a|)^2: the rows' largest elements are scaled to 1
+            const double dr = vi * x[0].re, di = vi * x[0].im;
+            d = fma(dr, dr, di * di);
         }
-        for (int off = 32; off > 0; off >>= 1) {
-            const double ov = __shfl_down(bv, off, 64);
-            const int oi = __shfl_down(bi, off, 64);
-            if (ov > bv || (ov == bv && oi > bi)) {
-                bv = ov;
-                bi = oi;
-            }
-        }
+        if (!(d >= 0.0)) d = -1.0;
+        double v = wave_max(d);
+        int ix = last_lane(d, v);
+        if (ix >= 0) ix += i - lane;
         if (lane == 0) {
-            sval[wv] = bv;
-            sidx[wv] = bi;
+            sv[w] = v;
+            si[w] = ix;
         }
         __syncthreads();
+        v = sv[0];
+        ix = si[0];
+        for (int q = 1; q < 4; q++)
+            if (si[q] >= 0 && sv[q] >= v) {
+                v = sv[q];
+                ix = si[q];
+            }
+        // the candidate is known from column j alone: its value goes out before
+        // the rest of the last column's update, columns j+2.. taking the place of
+        // j+1.. (the ones behind the panel are zeros)
         if (tid == 0) {
-            double v = sval[0];
-            int ix = sidx[0];
-            for (int w = 1; w < LU_PANEL_THREADS / 64; w++)
-                if (sval[w] > v || (sval[w] == v && sidx[w] > ix)) {
-                    v = sval[w];
-                    ix = sidx[w];
+            ll_put(set + blk * LU_LL_HEAD, v, seq);
+            ll_put(set + blk * LU_LL_HEAD + 2, (unsigned)ix, seq);
+        }
+        if (jj > 0 && mine && i >= j) {
+            auto upd = [&](int k) { x[k - 1] = csub(x[k], cmul(l, plast[k])); };
+#pragma unroll
+            for (int k = 2; k < 8; k++) upd(k);
+            if (jj < LU_NB - 6) {
+#pragma unroll
+                for (int k = 8; k < 16; k++) upd(k);
+            }
+            if (jj < LU_NB - 14) {
+#pragma unroll
+                for (int k = 16; k < 24; k++) upd(k);
+            }
+            if (jj < LU_NB - 22) {
+#pragma unroll
+                for (int k = 24; k < LU_NB; k++) upd(k);
+            }
+            x[LU_NB - 1] = cmk(0.0, 0.0);
+        }
+        const int r0 = c0 + blk * 256;  // the workgroup's rows
+        if (mine && (i == ix || i == j)) {
+            zc *dst = i == ix ? crow : jrow;
+#pragma unroll
+            for (int k = 0; k < LU_NB; k++) dst[jj + k] = x[k];
+            if (i == j) vvj = vi;
+        }
+        if (lane < jj) {
+            if (w == 2 && ix >= 0) crow[lane] = ls[lane][ix - r0];
+            if (w == 3 && blk == 0) jrow[lane] = ls[lane][jj];
+        }
+        const double *cd = reinterpret_cast<const double *>(crow);
+        if (blk == 0 && ix == j) {  // one row, written once; another workgroup's may come to the other place
+            zc *t = crow;
+            crow = jrow;
+            jrow = t;
+        }
+        __syncthreads();
+        const double *jd = reinterpret_cast<const double *>(jrow);
+        if (w == 0) {
+            ll_put(rows + blk * LU_LL_ROW + 2 * lane, cd[lane], seq);
+            bool ok = ll_get(set + lane * LU_LL_HEAD, lane < nblk, seq, d, &ix);
+            if (lane >= nblk || ix < 0) d = -1.0;
+            v = wave_max(d);
+            const int wb = last_lane(d, v);
+            ix = wb < 0 ? j : __builtin_amdgcn_readlane(ix, wb);  // no finite candidate: keep row j
+            if (ok && wb >= 0 && wb != blk) {
+                double c = 0.0;
+                ok = ll_get(rows + wb * LU_LL_ROW + 2 * lane, true, seq, c, nullptr);
+                reinterpret_cast<double *>(crow)[lane] = c;
+            }
+            if (lane == 0) six = ok ? ix : -1;
+        } else if (w == 1) {
+            if (blk == 0) {
+                ll_put(rowj + 2 * lane, jd[lane], seq);
+                if (lane == 0) ll_put(rowj + LU_LL_ROW, vvj, seq);
+            } else {
+                double c = 0.0, vj = 0.0;
+                const bool ok = ll_get(rowj + 2 * lane, true, seq, c, nullptr) &&
+                                ll_get(rowj + LU_LL_ROW, true, seq, vj, nullptr);
+                reinterpret_cast<double *>(jrow)[lane] = c;
+                if (lane == 0) {
+                    vvj = vj;
+                    if (!ok) atomicOr(err, 2);
                 }
-            if (ix < j) ix = j;  // no finite candidate: keep row j
-            imax_s = ix;
-            piv[j] = ix;
-            if (ix != j) vv[ix] = vv[j];
-        }
-        __syncthreads();
-        const int im = imax_s;
-        // swap rows j and im inside the panel
-        if (im != j)
-            for (int k = c0 + tid; k < c0 + nb; k += LU_PANEL_THREADS) {
-                zc *ck = A + (int64_t)k * n;
-                const zc t = ck[im];
-                ck[im] = ck[j];
-                ck[j] = t;
             }
-        __syncthreads();
-        if (tid == 0 && zabs(colj[j]) == 0.0) colj[j] = cmk(1e-20, 0.0);
-        __syncthreads();
-        const zc p = colj[j];
-        const double den = p.re * p.re + p.im * p.im;
-        const zc rcp = cmk(p.re / den, -p.im / den);  // 1 / a(j,j)
-        for (int i = j + 1 + tid; i < n; i += LU_PANEL_THREADS) colj[i] = cmul(colj[i], rcp);
-        __syncthreads();
-        // rank-1 update of the panel's remaining columns
-        for (int k = j + 1; k < c0 + nb; k++) {
-            zc *ck = A + (int64_t)k * n;
-            const zc u = ck[j];
-            for (int i = j + 1 + tid; i < n; i += LU_PANEL_THREADS) ck[i] = csub(ck[i], cmul(colj[i], u));
         }
         __syncthreads();
-    }
-}
-
-// The same panel factorization spread over the chip, per column j: (1) block
-// partial maxima of vv(i)|a(i,j)| over rows >= j (a launch of its own only
-// for a panel's first column: the update of column j-1 leaves them for the
-// others), (2) one wave picks the pivot (ties to the larger row), swaps rows
-// j and imax across the panel and keeps 1/a(j,j), (3) scaling of column j
-// and the rank-1 update of the panel's remaining columns, one thread per row.
-#define LU_PIV_BLOCKS 256
-__global__ __launch_bounds__(256) void lu_pivot_kernel(const zc *A, int n, int j, const double *vv, double *pval,
-                                                       int *pidx)
-{
-    __shared__ double sv[4];
-    __shared__ int si[4];
-    const zc *colj = A + (int64_t)j * n;
-    double bv = -1.0;
-    int bi = -1;
-    for (int i = j + blockIdx.x * 256 + threadIdx.x; i < n; i += 256 * gridDim.x) {
-        const double d = vv[i] * zabs(colj[i]);
-        if (d >= bv) {
-            bv = d;
-            bi = i;
+        ix = six;
+        if (ix < 0) {  // a wait ran out
+            if (tid == 0) atomicOr(err, 2);
+            return;
         }
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        const double ov = __shfl_down(bv, off, 64);
-        const int oi = __shfl_down(bi, off, 64);
-        if (ov > bv || (ov == bv && oi > bi)) {
-            bv = ov;
-            bi = oi;
-        }
-    }
-    if ((threadIdx.x & 63) == 0) {
-        sv[threadIdx.x >> 6] = bv;
-        si[threadIdx.x >> 6] = bi;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 4; w++)
-            if (sv[w] > bv || (sv[w] == bv && si[w] > bi)) {
-                bv = sv[w];
-                bi = si[w];
-            }
-        pval[blockIdx.x] = bv;
-        pidx[blockIdx.x] = bi;
-    }
-}
-
-__global__ __launch_bounds__(64) void lu_pick_kernel(zc *A, int n, int c0, int nb, int j, double *vv, int *piv,
-                                                     const double *pval, const int *pidx, int nblk, zc *rcp)
-{
-    const int t = threadIdx.x;
-    double v = -1.0;
-    int ix = -1;  // no candidate
-    for (int b = t; b < nblk; b += 64) {
-        const double pv = pval[b];
-        const int pi = pidx[b];
-        if (pi >= 0 && (ix < 0 || pv > v || (pv == v && pi > ix))) {
-            v = pv;
-            ix = pi;
-        }
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        const double ov = __shfl_down(v, off, 64);
-        const int oi = __shfl_down(ix, off, 64);
-        if (oi >= 0 && (ix < 0 || ov > v || (ov == v && oi > ix))) {
-            v = ov;
-            ix = oi;
-        }
-    }
-    ix = __shfl(ix, 0, 64);
-    if (ix < j) ix = j;  // no finite candidate: keep row j
-    if (t == 0) {
-        piv[j] = ix;
-        if (ix != j) vv[ix] = vv[j];
-    }
-    // rows j and ix swap across the panel (nb <= 64 columns, one per lane);
-    // the lane of column j keeps the pivot and its reciprocal
-    const int k = c0 + t;
-    if (t < nb) {
-        zc *ck = A + (int64_t)k * n;
-        zc a = ck[ix];
-        if (ix != j) {
-            ck[ix] = ck[j];
-            ck[j] = a;
-        }
-        if (k == j) {
-            if (zabs(a) == 0.0) {
-                a = cmk(1e-20, 0.0);
-                ck[j] = a;
-            }
-            const double den = a.re * a.re + a.im * a.im;
-            rcp[0] = cmk(a.re / den, -a.im / den);
-        }
-    }
-}
-
-// When column j+1 is in the panel, the update also leaves the pivot
-// partials of column j+1 over its rows (one per workgroup, as the pivot
-// kernel would): the search of the next column needs no launch of its own.
-__global__ __launch_bounds__(256) void lu_colupdate_kernel(zc *A, int n, int c0, int nb, int j, const zc *rcp,
-                                                           const double *vv, double *pval, int *pidx)
-{
-    __shared__ double sv[4];
-    __shared__ int si[4];
-    __shared__ zc urow[LU_NB];  // row j of the columns after j in the panel
-    const int i = j + 1 + blockIdx.x * 256 + threadIdx.x, nk = c0 + nb - j - 1;
-    const bool ahead = nk > 0, mine = i < n;
-    // every load of the row goes out before the barrier and before any store
-    // (no thread here writes row j)
-    zc x[LU_NB - 1], l = cmk(0.0, 0.0);
-    if (mine) {
+        const zc *prow = ix == j ? jrow : crow;
+        zc a = prow[jj];
+        if (a.re == 0.0 && a.im == 0.0) a = cmk(1e-20, 0.0);
+        const double den = a.re * a.re + a.im * a.im;
+        const zc rcp = cmk(a.re / den, -a.im / den);
+        if (blk == 0 && w == 2 && lane < nb)  // row j is complete
+            A[(int64_t)(c0 + lane) * n + j] = lane == jj ? a : prow[lane];
+        if (blk == 0 && tid == 192) piv[j] = ix;
+        const int ir = ix - r0;
+        if (w == 3 && ix != j && ir >= 0 && ir < 256 && lane < jj) ls[lane][ir] = jrow[lane];
+        if (mine && i > j) {
+            if (i == ix) {
 #pragma unroll
-        for (int t = 0; t < LU_NB - 1; t++)
-            if (t < nk) x[t] = A[(int64_t)(j + 1 + t) * n + i];
-        l = cmul(A[(int64_t)j * n + i], rcp[0]);
-    }
-    if (threadIdx.x < nk) urow[threadIdx.x] = A[(int64_t)(j + 1 + threadIdx.x) * n + j];
-    __syncthreads();
-    double bv = -1.0;
-    int bi = -1;
-    if (mine) {
-        A[(int64_t)j * n + i] = l;
-#pragma unroll
-        for (int t = 0; t < LU_NB - 1; t++)
-            if (t < nk) {
-                x[t] = csub(x[t], cmul(l, urow[t]));
-                A[(int64_t)(j + 1 + t) * n + i] = x[t];
+                for (int k = 0; k < LU_NB; k++) x[k] = jrow[jj + k];
+                vi = vvj;
             }
-        if (ahead) {
-            bv = vv[i] * zabs(x[0]);
-            bi = i;
+            l = cmul(x[0], rcp);
+            ls[jj][tid] = l;
+            x[0] = csub(x[1], cmul(l, prow[jj + 1]));
         }
+        plast = prow + jj;
     }
-    if (!ahead) return;
-    for (int off = 32; off > 0; off >>= 1) {
-        const double ov = __shfl_down(bv, off, 64);
-        const int oi = __shfl_down(bi, off, 64);
-        if (ov > bv || (ov == bv && oi > bi)) {
-            bv = ov;
-            bi = oi;
-        }
-    }
-    if ((threadIdx.x & 63) == 0) {
-        sv[threadIdx.x >> 6] = bv;
-        si[threadIdx.x >> 6] = bi;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 4; w++)
-            if (sv[w] > bv || (sv[w] == bv && si[w] > bi)) {
-                bv = sv[w];
-                bi = si[w];
-            }
-        pval[blockIdx.x] = bv;
-        pidx[blockIdx.x] = bi;
-    }
+    __syncthreads();  // ls: rows swapped by wave 3
+    if (!mine || i < c0 + nb) return;
+    for (int q = 0; q < nb; q++) A[(int64_t)(c0 + q) * n + i] = ls[q][tid];
+    vv[i] = vi;
 }
+static_assert(LU_NB == 32, "lu_panel_kernel: 64 doubles of a row on a wave, segments of 8 columns");
 
 // the panel's row swaps on columns [k0, k1)
 __global__ void lu_swap_kernel(zc *A, int n, int c0, int nb, const int *piv, int k0, int k1)
@@ -699,39 +712,22 @@ hipError_t launch_lu_store(double *A, int n, int j0, int ncol, const double *th,
     return hipGetLastError();
 }
 
-// scratch: pval[LU_PIV_BLOCKS] doubles, rcp one complex, pidx[LU_PIV_BLOCKS] ints
-size_t lu_factor_scratch_bytes() { return LU_PIV_BLOCKS * (sizeof(double) + sizeof(int)) + 2 * sizeof(double); }
+// scratch: the words of the panels' exchange
+size_t lu_factor_scratch_bytes() { return 2 * LU_LL_SET * sizeof(lu_word); }
 
 hipError_t launch_lu_factor(double *LUm, int n, double *vv, int *piv, int *err, void *scratch, hipStream_t st)
 {
-    if (n < 1 || n > LU_PIV_BLOCKS * 256) return hipErrorInvalidValue;
+    if (n < 1 || n > LU_MAX_BLOCKS * 256) return hipErrorInvalidValue;
     zc *A = reinterpret_cast<zc *>(LUm);
-    double *pval = reinterpret_cast<double *>(scratch);
-    zc *rcp = reinterpret_cast<zc *>(pval + LU_PIV_BLOCKS);
-    int *pidx = reinterpret_cast<int *>(pval + LU_PIV_BLOCKS + 2);
+    lu_word *ll = reinterpret_cast<lu_word *>(scratch);
+    hipLaunchKernelGGL(lu_clear_kernel, dim3(32), dim3(256), 0, st, ll, 2 * LU_LL_SET);
     hipLaunchKernelGGL(lu_rowscale_kernel, dim3((n + 63) / 64), dim3(256), 0, st, A, n, vv, err);
     hipError_t e = hipGetLastError();
     // one panel of nb columns at c0: pivot search, row swaps and elimination
     // inside the panel's own columns
     auto panel = [&](int c0, int nb) {
-        if (n - c0 <= LU_PANEL_ONE_WG_ROWS) {
-            // short panels: one workgroup does all its columns
-            hipLaunchKernelGGL(lu_panel_kernel, dim3(1), dim3(LU_PANEL_THREADS), 0, st, A, n, c0, nb, vv, piv);
-            return;
-        }
-        for (int jj = 0; jj < nb; jj++) {
-            const int j = c0 + jj, rows = n - j;
-            // partials of column j: its own search for the panel's first
-            // column, else those the update of column j-1 left (one per
-            // workgroup of that launch, (rows + 255) / 256 <= LU_PIV_BLOCKS)
-            const int nbk = jj == 0 ? imn(LU_PIV_BLOCKS, (rows + 255) / 256) : (rows + 255) / 256;
-            if (jj == 0) hipLaunchKernelGGL(lu_pivot_kernel, dim3(nbk), dim3(256), 0, st, A, n, j, vv, pval, pidx);
-            hipLaunchKernelGGL(lu_pick_kernel, dim3(1), dim3(64), 0, st, A, n, c0, nb, j, vv, piv, pval, pidx, nbk,
-                               rcp);
-            if (rows > 1)
-                hipLaunchKernelGGL(lu_colupdate_kernel, dim3((rows - 1 + 255) / 256), dim3(256), 0, st, A, n, c0, nb,
-                                   j, rcp, vv, pval, pidx);
-        }
+        hipLaunchKernelGGL(lu_panel_kernel, dim3((n - c0 + 255) / 256), dim3(256), 0, st, A, n, c0, nb, vv, piv, ll,
+                           err);
     };
     auto swap = [&](int p0, int np, int k0, int k1) {  // pivots [p0, p0+np) on columns [k0, k1)
         if (k1 > k0)
