@@ -442,59 +442,90 @@ static hipError_t fft_axis(const cplx<T> *in, cplx<T> *out, int batch, int3 din,
 // The node-kernel spectrum is FP32 (the reference stores complex(4)); the
 // data precision is T.  One thread per (frequency, mode, block of CONTRACT_LC l).
 // ===========================================================================
-#define CONTRACT_LC 4  // output degrees l per thread: each source value read serves LC of them
+// Bound by reading the spectrum.  1000-sphere cylinder (99 degrees, 9216
+// frequencies, 1.45 GB): 258 us, 5.6 TB/s; 2000-sphere aggregate (24, 46080,
+// 425 MB): 126 us.  With the spectrum as [p][l][n][k] and 8 bytes per lane, 319
+// and 137 us: a workgroup hopped 73 KB per n on four streams, and more loads in
+// flight made it slower.  A workgroup's share now lies in one piece.  Degrees per
+// thread 4 / 6 / 8: 263 / 258 / 303 us (130 / 126 / 130); two-wave workgroups 270;
+// four steps in flight instead of two 306.
+#define CONTRACT_LC 6  // output degrees l per thread: each source value read serves LC of them
+#define CONTRACT_NT 64 // threads per workgroup, each with two neighbouring frequencies
+#define CONTRACT_F (2 * CONTRACT_NT)  // frequencies of a workgroup
+// Spectrum element K(p, l, n) at frequency k: what a workgroup reads, CONTRACT_LC
+// degrees l of CONTRACT_F frequencies for n = 0, 1, ..., lies behind each other
+__host__ __device__ inline int64_t spectrum_pos(int p, int l, int n, int k, int M, int nblk)
+{
+    const int64_t X = (M + CONTRACT_F - 1) / CONTRACT_F, Z = (nblk + CONTRACT_LC - 1) / CONTRACT_LC;
+    return ((((p * X + k / CONTRACT_F) * Z + l / CONTRACT_LC) * nblk + n) * CONTRACT_LC + l % CONTRACT_LC) * CONTRACT_F +
+           k % CONTRACT_F;
+}
 // NL (<= CONTRACT_LC) output degrees of one thread: a compile-time count, so
 // that every load of a step has no guard and all of them (and those of the
-// next step) are in flight together
+// next steps) are in flight together
 template <typename T, int NL>
 __device__ __forceinline__ void contract_degrees(const cplx<float> *__restrict__ K, const cplx<T> *__restrict__ a,
                                                  cplx<T> *__restrict__ g, int M, int nblk, int k, int p, int l0)
 {
-    typedef float f2v __attribute__((ext_vector_type(2)));
-    cplx<T> acc[2][NL];
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    struct __attribute__((aligned(16))) two {
+        cplx<T> v[2];
+    };
+    cplx<T> acc[2][NL][2];
 #pragma unroll
-    for (int l = 0; l < NL; l++) acc[0][l] = acc[1][l] = cmk((T)0, (T)0);
-    const int64_t ls = (int64_t)nblk * M;  // K stride between degrees l
-    const cplx<float> *kp = K + ((int64_t)p * nblk + l0) * ls + k;
+    for (int l = 0; l < NL; l++)
+        for (int h = 0; h < 2; h++) acc[0][l][h] = acc[1][l][h] = cmk((T)0, (T)0);
+    const cplx<float> *kp = K + spectrum_pos(p, l0, 0, k, M, nblk);
     const cplx<T> *ap0 = a + (int64_t)p * nblk * M + k, *ap1 = a + (int64_t)(2 + p) * nblk * M + k;
 #pragma unroll 2
     for (int n = 0; n < nblk; n++) {
-        const cplx<T> a0 = ap0[(int64_t)n * M], a1 = ap1[(int64_t)n * M];
+        const two a0 = *reinterpret_cast<const two *>(ap0 + (int64_t)n * M);
+        const two a1 = *reinterpret_cast<const two *>(ap1 + (int64_t)n * M);
 #pragma unroll
         for (int l = 0; l < NL; l++) {
-            const f2v kv = __builtin_nontemporal_load(reinterpret_cast<const f2v *>(kp + l * ls + (int64_t)n * M));
-            const cplx<T> kk = cmk((T)kv[0], (T)kv[1]);
-            cfma(acc[0][l], kk, a0);
-            cfma(acc[1][l], kk, a1);
+            const f4v kv = __builtin_nontemporal_load(reinterpret_cast<const f4v *>(kp + (n * CONTRACT_LC + l) * CONTRACT_F));
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const cplx<T> kk = cmk((T)kv[2 * h], (T)kv[2 * h + 1]);
+                cfma(acc[0][l][h], kk, a0.v[h]);
+                cfma(acc[1][l][h], kk, a1.v[h]);
+            }
         }
     }
 #pragma unroll
-    for (int l = 0; l < NL; l++) {
-        g[((int64_t)(0 * 2 + p) * nblk + l0 + l) * M + k] = acc[0][l];
-        g[((int64_t)(1 * 2 + p) * nblk + l0 + l) * M + k] = acc[1][l];
-    }
+    for (int l = 0; l < NL; l++)
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const two o = {{acc[r][l][0], acc[r][l][1]}};
+            *reinterpret_cast<two *>(g + ((int64_t)(r * 2 + p) * nblk + l0 + l) * M + k) = o;
+        }
 }
 
+// M (8 times the cells) is even, so a thread's two frequencies are 16 bytes of
+// the spectrum at a 16-byte boundary
 template <typename T>
-__global__ void contract_kernel(const cplx<float> *__restrict__ K, const cplx<T> *__restrict__ a,
-                                cplx<T> *__restrict__ g, int M, int nblk, const int *__restrict__ gate)
+__global__ __launch_bounds__(CONTRACT_NT) void contract_kernel(const cplx<float> *__restrict__ K,
+                                                               const cplx<T> *__restrict__ a, cplx<T> *__restrict__ g,
+                                                               int M, int nblk, const int *__restrict__ gate)
 {
     if (gate && !*gate) return;
     constexpr int LC = CONTRACT_LC;
-    static_assert(LC == 4, "the degree-count switch below covers 1..4");
+    static_assert(LC == 6, "the degree-count switch below covers 1..6");
     // workgroup -> (frequency block x, mode p, degree block z): the Z degree
     // blocks of one (x, p) read the same source fields, so they are dealt to
     // one XCD (workgroups go to MI355X's 8 XCDs round robin) one after another
     // and share its L2; the grid holds 8 * ceil(2 X / 8) * Z workgroups
-    const int X = (M + 127) / 128, Z = (nblk + LC - 1) / LC;
+    const int X = (M + CONTRACT_F - 1) / CONTRACT_F, Z = (nblk + LC - 1) / LC;
     const int wg = blockIdx.x, slot = wg >> 3;
     const int c = (wg & 7) + 8 * (slot / Z);  // (x, p) combination
     if (c >= 2 * X) return;
-    const int k = (c >> 1) * blockDim.x + threadIdx.x;
+    const int k = 2 * ((c >> 1) * CONTRACT_NT + threadIdx.x);
     const int p = c & 1;
     const int l0 = (slot % Z) * LC;
     if (k >= M) return;
     switch (imn(LC, nblk - l0)) {  // uniform over the workgroup
+    case 6: contract_degrees<T, 6>(K, a, g, M, nblk, k, p, l0); break;
+    case 5: contract_degrees<T, 5>(K, a, g, M, nblk, k, p, l0); break;
     case 4: contract_degrees<T, 4>(K, a, g, M, nblk, k, p, l0); break;
     case 3: contract_degrees<T, 3>(K, a, g, M, nblk, k, p, l0); break;
     case 2: contract_degrees<T, 2>(K, a, g, M, nblk, k, p, l0); break;
@@ -637,12 +668,17 @@ __global__ void node_kernel_build(double *__restrict__ Ks, int3 N, double dcell,
             }
 }
 
-// complex FP64 chunk -> FP32 spectrum, scaled by 1/M (the /ncells8 of :898)
-__global__ void to_f32_scaled(const cplx<double> *__restrict__ in, cplx<float> *__restrict__ out, int64_t n,
-                              double scale)
+// complex FP64 chunk in[nl][nblk][M] of mode p, degrees l0.. -> FP32 spectrum in
+// the contraction's layout, scaled by 1/M (the /ncells8 of :898)
+__global__ void spectrum_store(const cplx<double> *__restrict__ in, cplx<float> *__restrict__ K, int p, int l0,
+                               int64_t n, int M, int nblk, double scale)
 {
     int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < n) out[q] = cmk((float)(in[q].re * scale), (float)(in[q].im * scale));
+    if (q >= n) return;
+    const int k = (int)(q % M);
+    const int64_t t = q / M;
+    K[spectrum_pos(p, l0 + (int)(t / nblk), (int)(t % nblk), k, M, nblk)] =
+        cmk((float)(in[q].re * scale), (float)(in[q].im * scale));
 }
 
 // ===========================================================================
@@ -1027,7 +1063,7 @@ static int build_kernel(FftOp *f, hipStream_t st)
     FCHK(hipMemcpy(d_kl, kl_of.data(), sizeof(int) * nblk, hipMemcpyHostToDevice));
     FCHK(hipMemcpy(d_mn, mn_of.data(), sizeof(int) * nblk, hipMemcpyHostToDevice));
     if (!hole.empty()) FCHK(hipMemcpy(d_hole, hole.data(), sizeof(int) * hole.size(), hipMemcpyHostToDevice));
-    FCHK(falloc(&f->K, sizeof(cplx<float>) * (size_t)2 * nblk * nblk * M));
+    FCHK(falloc(&f->K, sizeof(cplx<float>) * (size_t)spectrum_pos(2, 0, 0, 0, M, nblk)));
     // chunk over target rows so the FP64 staging stays under ~2 GB
     size_t per_row = (size_t)2 * nblk * M * sizeof(cplx<double>);
     int rows = (int)std::max<size_t>(1, std::min<size_t>(nblk, ((size_t)2 << 30) / per_row));
@@ -1045,12 +1081,11 @@ static int build_kernel(FftOp *f, hipStream_t st)
         FCHK(fft_axis<double>(ks, kt, batch, D2, D2, 2, D2.z, D2.z, D2.z, -1, st));
         FCHK(fft_axis<double>(kt, ks, batch, D2, D2, 1, D2.y, D2.y, D2.y, -1, st));
         FCHK(fft_axis<double>(ks, kt, batch, D2, D2, 0, D2.x, D2.x, D2.x, -1, st));
-        // kt[(p*nl + lr)*nblk + n][M] -> K[p][l0+lr][n][M]
+        // kt[(p*nl + lr)*nblk + n][M] -> K (spectrum_pos)
         for (int p = 0; p < 2; p++) {
             int64_t cnt = (int64_t)nl * nblk * M;
-            hipLaunchKernelGGL(to_f32_scaled, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st,
-                               kt + (int64_t)p * nl * nblk * M, f->K + ((int64_t)p * nblk + l0) * nblk * M, cnt,
-                               1.0 / (double)M);
+            hipLaunchKernelGGL(spectrum_store, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st,
+                               kt + (int64_t)p * nl * nblk * M, f->K, p, l0, cnt, M, nblk, 1.0 / (double)M);
             FCHK(hipGetLastError());
         }
     }
@@ -1211,7 +1246,7 @@ template <typename T> static int matvec_t(FftOp *f, int nrhs, const double *ain,
     FCHK(fft_axis<T>(A, B, batch, d1, d2, 1, 2 * N.y, N.y, 2 * N.y, -1, st, gate));
     FCHK(fft_axis<T>(B, A, batch, d2, d3, 0, 2 * N.x, N.x, 2 * N.x, -1, st, gate));
     // per-frequency contraction with the node kernel spectrum
-    const int cX = (f->M + 127) / 128, cZ = (nblk + CONTRACT_LC - 1) / CONTRACT_LC;
+    const int cX = (f->M + CONTRACT_F - 1) / CONTRACT_F, cZ = (nblk + CONTRACT_LC - 1) / CONTRACT_LC;
     dim3 cg_((unsigned)((2 * cX + 7) / 8 * 8 * cZ));
     if (f->cev_used + 2 > 512) collect_contract(f);
     while (f->cev.size() < f->cev_used + 2) {
@@ -1222,7 +1257,7 @@ template <typename T> static int matvec_t(FftOp *f, int nrhs, const double *ain,
     f->cev_prec.resize(f->cev.size() / 2 + 1);
     f->cev_prec[f->cev_used / 2] = prec;
     FCHK(hipEventRecord(f->cev[f->cev_used], st));
-    hipLaunchKernelGGL(contract_kernel<T>, cg_, dim3(128), 0, st, f->K, A, B, f->M, nblk, gate);
+    hipLaunchKernelGGL(contract_kernel<T>, cg_, dim3(CONTRACT_NT), 0, st, f->K, A, B, f->M, nblk, gate);
     FCHK(hipGetLastError());
     FCHK(hipEventRecord(f->cev[f->cev_used + 1], st));
     f->cev_used += 2;
