@@ -244,10 +244,24 @@ __global__ void sphere_reduce_kernel(const cplx<T> *__restrict__ far, const cplx
     int rp = (int)(t % 4);
     int i = (int)(t / 4);
     cplx<T> s = far[((int64_t)i * 4 + rp) * NBP + e];
-    for (int j = sstart[i]; j < sstart[i + 1]; j++) {
-        int ent = sent[j], pq = ent >> 1;
-        const cplx<T> *src = (ent & 1) ? nr : nf;
-        s = cadd(s, src[((int64_t)pq * 4 + rp) * NBP + e]);
+    // bound by the latency of scattered terms: eight in flight, added in the
+    // list's order (2000 spheres with 75 terms each: 81 us one by one, 25 us)
+    constexpr int U = 8;
+    const int j1 = sstart[i + 1];
+    int j = sstart[i];
+    for (; j + U <= j1; j += U) {
+        cplx<T> v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int ent = sent[j + u];
+            v[u] = ((ent & 1) ? nr : nf)[((int64_t)(ent >> 1) * 4 + rp) * NBP + e];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) s = cadd(s, v[u]);
+    }
+    for (; j < j1; j++) {
+        const int ent = sent[j];
+        s = cadd(s, ((ent & 1) ? nr : nf)[((int64_t)(ent >> 1) * 4 + rp) * NBP + e]);
     }
     int r = rp >> 1, p = rp & 1;
     out[(((int64_t)r * npad + i) * 2 + p) * NBP + e] = s;
