@@ -451,6 +451,267 @@ static hipError_t fft_axis(const cplx<T> *in, cplx<T> *out, int batch, int3 din,
 }
 
 // ===========================================================================
+// The product's transforms: the z axis in one launch (fft_z_kernel), the two
+// axes of every xy plane in another (fft_plane_kernel), both in LDS with the
+// butterflies of the passes above, so the values are the same.
+// An axis at a time moved 21 N values per array and direction, now 13; pieces of
+// 64 bytes along y, divisions and half-empty stages made a pass 23 us on average
+// for a 1000-sphere cylinder (8x8x18 points, 396 arrays) and 36 us for a
+// 2000-sphere aggregate (30x12x16, 96 arrays), six passes a product.  Now z takes
+// 10 and 14 us, the planes 26 and 39 us: 136 -> 71 and 226 -> 107 us a product,
+// bound by the stages' butterflies (full complex products with the roots) and
+// their barriers.  Pencils of the z axis 8 / 16 / 32: 10.0 / 9.6 / 9.3 us; planes of
+// 768 / 1536 / 3072 points: 25 / 26 / 31 us.
+
+// ===========================================================================
+// x / d for x < 65536: exact with m = ceil(2^32 / d)
+struct FftDiv {
+    unsigned m = 0, d = 1;
+};
+static FftDiv fft_div(int d) { return FftDiv{d > 1 ? (unsigned)((((unsigned long long)1 << 32) + d - 1) / d) : 0u, (unsigned)d}; }
+__device__ __forceinline__ int quo(int x, const FftDiv &v) { return v.m ? (int)__umulhi((unsigned)x, v.m) : x; }
+
+struct FftSteps {
+    int n, nstage, radix[16];
+    FftDiv nr[16], Ns[16];  // n / radix, product of the radices before
+};
+static FftSteps make_steps(int n)
+{
+    const FftPlan pl = make_plan(n);
+    FftSteps st{};
+    st.n = pl.n;
+    st.nstage = pl.nstage;
+    int Ns = 1;
+    for (int s = 0; s < pl.nstage; s++) {
+        st.radix[s] = pl.radix[s];
+        st.nr[s] = fft_div(n / pl.radix[s]);
+        st.Ns[s] = fft_div(Ns);
+        Ns *= pl.radix[s];
+    }
+    return st;
+}
+
+template <typename T> __device__ __forceinline__ void fft_roots(cplx<T> *tw, int n, int sign)
+{
+    for (int j = threadIdx.x; j < n; j += blockDim.x) {
+        T sn, cs;
+        if (sizeof(T) == 8) {
+            double sd, cd;
+            sincospi(2.0 * sign * (double)j / (double)n, &sd, &cd);
+            sn = (T)sd;
+            cs = (T)cd;
+        } else {
+            float sf, cf;
+            sincospif(2.0f * sign * (float)j / (float)n, &sf, &cf);
+            sn = (T)sf;
+            cs = (T)cf;
+        }
+        tw[j] = cmk(cs, sn);
+    }
+}
+
+// stage_radix with element j of the pencil at A + j sa (zero from nin on) and
+// at B + j sb
+template <typename T, int R>
+__device__ __forceinline__ void stage_strided(const cplx<T> *__restrict__ A, int sa, int nin, cplx<T> *__restrict__ B,
+                                              int sb, const cplx<T> *__restrict__ tw, int jj, int n, int nr,
+                                              const FftDiv &dNs)
+{
+    const int Ns = (int)dNs.d, jd = quo(jj, dNs), kk = jj - jd * Ns;
+    const int step = quo(nr, dNs);  // n / (Ns R)
+    cplx<T> v[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int j = jj + r * nr;
+        cplx<T> x = j < nin ? A[j * sa] : cmk((T)0, (T)0);
+        if (kk != 0 && r != 0) x = cmul(x, tw[kk * r * step]);
+        v[r] = x;
+    }
+    cplx<T> root[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) root[q] = tw[q * nr];
+    const int idxD = jd * Ns * R + kk;
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        cplx<T> s = cmk((T)0, (T)0);
+#pragma unroll
+        for (int r = 0; r < R; r++) cfma(s, root[(k * r) % R], v[r]);
+        B[(idxD + k * Ns) * sb] = s;
+    }
+}
+
+// one stage of P pencils: pencil p's element j at A + off_a(p) + j sa (zero
+// from nin on), to B + off_b(p) + j sb.  PF: neighbouring lanes take
+// neighbouring pencils, else neighbouring butterflies of one pencil.
+template <typename T, bool PF, typename FA, typename FB>
+__device__ __forceinline__ void fft_stage(const cplx<T> *A, FA off_a, int sa, int nin, cplx<T> *B, FB off_b, int sb,
+                                          const cplx<T> *tw, const FftSteps &st, int s, int P, const FftDiv &dP)
+{
+    const int R = st.radix[s], nr = (int)st.nr[s].d;
+    for (int w = threadIdx.x; w < P * nr; w += blockDim.x) {
+        const int q = quo(w, PF ? dP : st.nr[s]);
+        const int p = PF ? w - q * P : q, jj = PF ? q : w - q * nr;
+        const cplx<T> *a = A + off_a(p);
+        cplx<T> *b = B + off_b(p);
+        switch (R) {
+        case 2: stage_strided<T, 2>(a, sa, nin, b, sb, tw, jj, st.n, nr, st.Ns[s]); break;
+        case 3: stage_strided<T, 3>(a, sa, nin, b, sb, tw, jj, st.n, nr, st.Ns[s]); break;
+        case 4: stage_strided<T, 4>(a, sa, nin, b, sb, tw, jj, st.n, nr, st.Ns[s]); break;
+        default: stage_strided<T, 5>(a, sa, nin, b, sb, tw, jj, st.n, nr, st.Ns[s]); break;
+        }
+    }
+    __syncthreads();
+}
+
+#define FFT_Z_PENCILS 16
+#define FFT_Z_THREADS 128
+// z axis: in[batch][nin][npen] -> out[batch][nout][npen], P neighbouring
+// pencils per workgroup, LDS [z][pencil]
+template <typename T>
+__global__ void fft_z_kernel(const cplx<T> *__restrict__ in, cplx<T> *__restrict__ out, int npen, FftSteps st, int nin,
+                             int nout, int sign, int P, FftDiv dP, const int *__restrict__ gate)
+{
+    if (gate && !*gate) return;
+    extern __shared__ __attribute__((aligned(16))) unsigned char fft_smem[];
+    cplx<T> *A = reinterpret_cast<cplx<T> *>(fft_smem), *B = A + P * st.n, *tw = B + P * st.n;
+    const int pen0 = blockIdx.x * P, np = imn(P, npen - pen0);
+    in += (int64_t)blockIdx.y * nin * npen + pen0;
+    out += (int64_t)blockIdx.y * nout * npen + pen0;
+    fft_roots(tw, st.n, sign);
+    for (int e = threadIdx.x; e < P * nin; e += blockDim.x) {
+        const int j = quo(e, dP), p = e - j * P;
+        if (p < np) A[e] = in[(int64_t)j * npen + p];
+    }
+    __syncthreads();
+    auto off = [](int p) { return p; };
+    for (int s = 0; s < st.nstage; s++) {
+        fft_stage<T, true>(A, off, P, s ? st.n : nin, B, off, P, tw, st, s, P, dP);
+        cplx<T> *t = A;
+        A = B;
+        B = t;
+    }
+    for (int e = threadIdx.x; e < P * nout; e += blockDim.x) {
+        const int j = quo(e, dP), p = e - j * P;
+        if (p < np) out[(int64_t)j * npen + p] = A[e];
+    }
+}
+
+// both axes of Q neighbouring xy planes: forward (FWD) n.x x n.y points, zero
+// padded, y then x, to 2 n.x x 2 n.y; inverse x then y, keeping n.x x n.y.
+// LDS [plane][y][x].
+template <typename T, bool FWD>
+__global__ __launch_bounds__(256) void fft_plane_kernel(const cplx<T> *__restrict__ in, cplx<T> *__restrict__ out,
+                                                        int nx, int ny, int64_t nplanes, FftSteps sx, FftSteps sy,
+                                                        int sign, int Q, FftDiv dx, FftDiv dy2, FftDiv dP,
+                                                        const int *__restrict__ gate)
+{
+    if (gate && !*gate) return;
+    extern __shared__ __attribute__((aligned(16))) unsigned char fft_smem[];
+    const int X = 2 * nx, Y = 2 * ny, full = X * Y;
+    cplx<T> *A = reinterpret_cast<cplx<T> *>(fft_smem), *B = A + Q * full, *tx = B + Q * full, *ty = tx + X;
+    const int64_t q0 = (int64_t)blockIdx.x * Q;
+    const int nq = (int)(nplanes - q0 < Q ? nplanes - q0 : Q);
+    const int vin = FWD ? nx * ny : full, vout = FWD ? full : nx * ny;
+    in += q0 * vin;
+    out += q0 * vout;
+    fft_roots(tx, X, sign);
+    fft_roots(ty, Y, sign);
+    for (int e = threadIdx.x; e < nq * vin; e += blockDim.x) A[e] = in[e];
+    __syncthreads();
+    auto swap = [&]() {
+        cplx<T> *t = A;
+        A = B;
+        B = t;
+    };
+    // the y axis: pencil p = (plane, x), the planes' rows of nx points, ry rows in
+    auto yaxis = [&](int ry) {
+        int rows = ry;
+        for (int s = 0; s < sy.nstage; s++) {
+            const int r0 = rows;
+            auto oa = [&](int p) { const int q = quo(p, dx); return q * r0 * nx + (p - q * nx); };
+            auto ob = [&](int p) { const int q = quo(p, dx); return q * Y * nx + (p - q * nx); };
+            fft_stage<T, true>(A, oa, nx, s ? Y : ry, B, ob, nx, ty, sy, s, nq * nx, dP);
+            rows = Y;
+            swap();
+        }
+    };
+    // the x axis: pencil p = (plane, y) of Y rows
+    auto xaxis = [&](int w) {
+        for (int s = 0; s < sx.nstage; s++) {
+            const int wa = s ? X : w;
+            auto oa = [&](int p) { return p * wa; };
+            auto ob = [&](int p) { return p * X; };
+            fft_stage<T, false>(A, oa, 1, wa, B, ob, 1, tx, sx, s, nq * Y, dP);
+            swap();
+        }
+    };
+    if constexpr (FWD) {
+        yaxis(ny);
+        xaxis(nx);
+        for (int e = threadIdx.x; e < nq * full; e += blockDim.x) out[e] = A[e];
+    } else {
+        xaxis(X);
+        // the first nx points of every row, rows of nx points
+        for (int e = threadIdx.x; e < nq * Y * nx; e += blockDim.x) {
+            const int r = quo(e, dx);
+            B[e] = A[r * X + (e - r * nx)];
+        }
+        __syncthreads();
+        swap();
+        yaxis(Y);
+        for (int e = threadIdx.x; e < nq * vout; e += blockDim.x) {
+            const int r = quo(e, dx), q = quo(r, dy2);  // dy2: rows kept, ny
+            out[e] = A[(q * Y + (r - q * ny)) * nx + (e - r * nx)];
+        }
+    }
+}
+
+// LDS of a workgroup of the two kernels
+#define FFT_LDS 65536
+#define FFT_PLANE_POINTS 1536  // points of a workgroup's planes, at least one plane
+template <typename T> static bool fft_planes_ok(int3 N)
+{
+    const int64_t full = (int64_t)4 * N.x * N.y;
+    return (2 * full + 2 * N.x + 2 * N.y) * (int64_t)sizeof(cplx<T>) <= FFT_LDS && full <= 16384 &&
+           (2 * (int64_t)FFT_Z_PENCILS + 1) * 2 * N.z * (int64_t)sizeof(cplx<T>) <= FFT_LDS &&
+           make_plan(2 * N.x).n > 0 && make_plan(2 * N.y).n > 0 && make_plan(2 * N.z).n > 0;
+}
+
+template <typename T>
+static hipError_t fft_z(const cplx<T> *in, cplx<T> *out, int batch, int npen, int n, int nin, int nout, int sign,
+                        hipStream_t st, const int *gate)
+{
+    const int P = FFT_Z_PENCILS;
+    hipLaunchKernelGGL(fft_z_kernel<T>, dim3((npen + P - 1) / P, batch), dim3(FFT_Z_THREADS),
+                       (2 * (size_t)P + 1) * n * sizeof(cplx<T>), st, in, out, npen, make_steps(n), nin, nout, sign, P,
+                       fft_div(P), gate);
+    return hipGetLastError();
+}
+template <typename T, bool FWD>
+static hipError_t fft_planes(const cplx<T> *in, cplx<T> *out, int batch, int3 N, int sign, hipStream_t st,
+                             const int *gate)
+{
+    const int full = 4 * N.x * N.y;
+    const int64_t planes = (int64_t)batch * 2 * N.z;
+    const int lim = (int)(FFT_LDS / sizeof(cplx<T>)) - 2 * N.x - 2 * N.y;
+    const int Q = std::max(1, std::min(FFT_PLANE_POINTS / full, lim / (2 * full)));
+    const size_t lds = (2 * (size_t)Q * full + 2 * N.x + 2 * N.y) * sizeof(cplx<T>);
+    // the stages along y divide by the pencils of a full workgroup (an incomplete
+    // one's are fewer: its own divisor)
+    for (int part = 0; part < 2; part++) {
+        const int64_t whole = planes / Q, first = part ? whole * Q : 0;
+        const int64_t count = part ? planes - first : whole * Q;
+        if (!count) continue;
+        const int nq = part ? (int)count : Q;
+        hipLaunchKernelGGL((fft_plane_kernel<T, FWD>), dim3((unsigned)(part ? 1 : whole)), dim3(256), lds, st,
+                           in + first * (FWD ? N.x * N.y : full), out + first * (FWD ? full : N.x * N.y), N.x, N.y,
+                           count, make_steps(2 * N.x), make_steps(2 * N.y), sign, Q, fft_div(N.x), fft_div(N.y),
+                           fft_div(nq * N.x), gate);
+    }
+    return hipGetLastError();
+}
+
+// ===========================================================================
 // Per-frequency contraction g(k,l) = sum_n K(p,l,n,k) a(k,n) for both RHS
 // (the pointwise products of fft_node_to_node_translation, :864-872).
 // The node-kernel spectrum is FP32 (the reference stores complex(4)); the
@@ -1256,9 +1517,16 @@ template <typename T> static int matvec_t(FftOp *f, int nrhs, const double *ain,
     const int batch = 4 * nblk;
     int3 d0 = N, d1 = make_int3(N.x, N.y, 2 * N.z), d2 = make_int3(N.x, 2 * N.y, 2 * N.z),
          d3 = make_int3(2 * N.x, 2 * N.y, 2 * N.z);
-    FCHK(fft_axis<T>(B, A, batch, d0, d1, 2, 2 * N.z, N.z, 2 * N.z, -1, st, gate));
-    FCHK(fft_axis<T>(A, B, batch, d1, d2, 1, 2 * N.y, N.y, 2 * N.y, -1, st, gate));
-    FCHK(fft_axis<T>(B, A, batch, d2, d3, 0, 2 * N.x, N.x, 2 * N.x, -1, st, gate));
+    const bool planes = fft_planes_ok<T>(N);
+    if (planes) {
+        FCHK(fft_z<T>(B, A, batch, N.x * N.y, 2 * N.z, N.z, 2 * N.z, -1, st, gate));
+        FCHK((fft_planes<T, true>(A, B, batch, N, -1, st, gate)));
+        std::swap(A, B);
+    } else {
+        FCHK(fft_axis<T>(B, A, batch, d0, d1, 2, 2 * N.z, N.z, 2 * N.z, -1, st, gate));
+        FCHK(fft_axis<T>(A, B, batch, d1, d2, 1, 2 * N.y, N.y, 2 * N.y, -1, st, gate));
+        FCHK(fft_axis<T>(B, A, batch, d2, d3, 0, 2 * N.x, N.x, 2 * N.x, -1, st, gate));
+    }
     // per-frequency contraction with the node kernel spectrum
     const int cX = (f->M + CONTRACT_F - 1) / CONTRACT_F, cZ = (nblk + CONTRACT_LC - 1) / CONTRACT_LC;
     dim3 cg_((unsigned)((2 * cX + 7) / 8 * 8 * cZ));
@@ -1276,9 +1544,15 @@ template <typename T> static int matvec_t(FftOp *f, int nrhs, const double *ain,
     FCHK(hipEventRecord(f->cev[f->cev_used + 1], st));
     f->cev_used += 2;
     // inverse: x, y, z keeping the first N per axis
-    FCHK(fft_axis<T>(B, A, batch, d3, d2, 0, 2 * N.x, 2 * N.x, N.x, 1, st, gate));
-    FCHK(fft_axis<T>(A, B, batch, d2, d1, 1, 2 * N.y, 2 * N.y, N.y, 1, st, gate));
-    FCHK(fft_axis<T>(B, A, batch, d1, d0, 2, 2 * N.z, 2 * N.z, N.z, 1, st, gate));
+    if (planes) {
+        FCHK((fft_planes<T, false>(B, A, batch, N, 1, st, gate)));
+        FCHK(fft_z<T>(A, B, batch, N.x * N.y, 2 * N.z, 2 * N.z, N.z, 1, st, gate));
+        std::swap(A, B);
+    } else {
+        FCHK(fft_axis<T>(B, A, batch, d3, d2, 0, 2 * N.x, 2 * N.x, N.x, 1, st, gate));
+        FCHK(fft_axis<T>(A, B, batch, d2, d1, 1, 2 * N.y, 2 * N.y, N.y, 1, st, gate));
+        FCHK(fft_axis<T>(B, A, batch, d1, d0, 2, 2 * N.z, 2 * N.z, N.z, 1, st, gate));
+    }
     // node -> sphere (reverse J translation) from gnode[r][p][l][cell] in A
     const int64_t nc = f->ncells;
     FCHK((launch_list_translate<T, 1>)(lg, ljb, st, jt, n, LG, Lp, A, f->d_off_node, 2 * nblk * nc, nblk * nc, nc,
