@@ -212,6 +212,170 @@ template <typename T> static size_t list_translate_lds(int LT, int LS)
     return pad_to((int)stages, 16) + sizeof(T) * (size_t)slot_len(LT, LS, 16 / (int)sizeof(T));
 }
 
+// ===========================================================================
+// Near-field pairs: both directions of a pair's translation (one order L), the
+// stages of list_translate_kernel with the same sums.  A thread owns one (n, k)
+// of one direction in every stage and the four columns (r, p) of it, so a table
+// value read from LDS serves four sums, the columns are 32 bytes (FP32) that
+// lanes of one degree read together, and every section offset is a constant.
+// Bound by LDS reads and the stages' latency.  2000-sphere aggregate, 75406 pairs
+// of order 3, FP32: 98 us for both directions against 2 x 154 with a launch per
+// direction (orders taken at run time, 128 threads per pair, the table loaded
+// twice); 1000-sphere cylinder, 8003 pairs of order 6: 63 us against 2 x 64.
+// ===========================================================================
+// Complex products with their roundings spelled out, as list_translate_kernel's
+// come out (a product of the powers of e^{i phi} rounds differently in FP64), so
+// that both kernels give the same bits.
+template <typename T> __device__ __forceinline__ cplx<T> cmul_fixed(cplx<T> a, cplx<T> b)
+{
+    return cmk(fma(a.re, b.re, -(a.im * b.im)), fma(a.re, b.im, a.im * b.re));
+}
+template <typename T> __device__ __forceinline__ cplx<T> cmul_power(cplx<T> r, cplx<T> b)
+{
+    if (sizeof(T) == 8) return cmk(fma(r.re, b.re, -(r.im * b.im)), fma(r.im, b.re, r.re * b.im));
+    return cmul_fixed(r, b);
+}
+
+template <typename T, int L> constexpr int pair_threads() { return (2 * L * (L + 2) + 63) / 64 * 64; }
+
+template <typename T, int L>
+__global__ __launch_bounds__((pair_threads<T, L>())) void pair_translate_kernel(
+    const T *__restrict__ tab, const cplx<T> *__restrict__ src, const int64_t *__restrict__ off_f,
+    const int64_t *__restrict__ off_r, int64_t rs, int64_t ms, cplx<T> *__restrict__ dst_f, cplx<T> *__restrict__ dst_r,
+    const int *__restrict__ gate)
+{
+    if (gate && !*gate) return;
+    constexpr int NB = L * (L + 2), VW = 16 / sizeof(T), SL = slot_len(L, L, VW), NT = pair_threads<T, L>();
+    typedef typename std::conditional<sizeof(T) == 4, float4, double2>::type V;
+    struct __attribute__((aligned(16))) cols {
+        cplx<T> c[4];
+    };
+    __shared__ __attribute__((aligned(16))) T tl[SL];
+    __shared__ cols xs[2 * NB], ys[2 * NB];
+    const int q = blockIdx.x, tid = threadIdx.x;
+    const V *gsrc = reinterpret_cast<const V *>(tab + (int64_t)(q / MSTM_SLOTS) * SL * MSTM_SLOTS + (q % MSTM_SLOTS) * VW);
+    for (int c = tid; c < SL / VW; c += NT) reinterpret_cast<V *>(tl)[c] = gsrc[(int64_t)c * MSTM_SLOTS];
+    const bool act = tid < 2 * NB;
+    const int dir = tid >= NB && act, w = act ? tid - dir * NB : 0;
+    int n = 1;
+#pragma unroll
+    for (int l = 1; l < L; l++) n += w >= l * (l + 2);
+    const int k = w + 1 - n * (n + 1), kk = dir ? -k : k;
+    const T sg = dir && (k & 1) ? (T)-1 : (T)1;
+    // phase-shifted source, m-flipped for the reverse direction
+    cols v;
+    {
+        const cplx<T> *sp = src + (dir ? off_r : off_f)[q] + amn(kk, n, L);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const cplx<T> x = sp[(c >> 1) * rs + (c & 1) * ms];
+            v.c[c] = cmk(sg * x.re, sg * x.im);
+        }
+    }
+    __syncthreads();
+    constexpr int phi = phi_off(L, L, VW);
+    const cplx<T> e1 = cmk(tl[phi], dir ? -tl[phi + 1] : tl[phi + 1]);
+    auto phase = [&](int j) {  // e^{i j phi}
+        cplx<T> r = cmk((T)1, (T)0);
+        const cplx<T> b = j < 0 ? cconj(e1) : e1;
+        for (int u = 0; u < iab(j); u++) r = cmul_power(r, b);
+        return r;
+    };
+    if (act) {
+        const cplx<T> ph = phase(k);
+        cols o;
+#pragma unroll
+        for (int c = 0; c < 4; c++) o.c[c] = cmul_fixed(ph, v.c[c]);
+        xs[tid] = o;
+    }
+    __syncthreads();
+    const int m1 = imx(1, iab(k)), d0 = dir * NB;
+    int bo = 0;  // section of block m = k, its axial matrices
+#pragma unroll
+    for (int m = -L; m <= L; m++)
+        if (m == k) bo = sec_off(m < 0 ? -2 * m - 1 : 2 * m, L, L, VW);
+    const cplx<T> zero = cmk((T)0, (T)0);
+    cols acc;
+    // forward rotation y_k(n)
+    if (act) {
+        acc = cols{{zero, zero, zero, zero}};
+        const T *E = tl + bo + n * n - m1 * m1;
+        const cols *x = xs + d0 + nk(n, -n);
+#pragma unroll
+        for (int i = 0; i <= 2 * L; i++)
+            if (i <= 2 * n) {
+                const T e = E[i];
+                const cols a = x[i];
+#pragma unroll
+                for (int c = 0; c < 4; c++) crfma(acc.c[c], e, a.c[c]);
+            }
+        ys[tid] = acc;
+    }
+    __syncthreads();
+    // axial z_k(t), t = n (transposed matrix for the reverse direction)
+    if (act) {
+        acc = cols{{zero, zero, zero, zero}};
+        const int NR = L - m1 + 1, rl = pad_to((L + 1) * (L + 1) - m1 * m1, VW), al = pad_to(2 * NR * NR, VW);
+        const T *A0 = tl + bo + rl + 2 * (dir ? NR * (n - m1) : n - m1), *A1 = A0 + al;
+        const int st = dir ? 2 : 2 * NR;
+#pragma unroll
+        for (int s = 1; s <= L; s++)
+            if (s >= m1) {
+                const int ex = (s - m1) * st;
+                const cplx<T> a0 = cmk(A0[ex], A0[ex + 1]), a1 = cmk(A1[ex], A1[ex + 1]);
+                const cols y = ys[d0 + nk(s, k)];
+                cfma(acc.c[0], a0, y.c[0]);
+                cfma(acc.c[1], a1, y.c[1]);
+                cfma(acc.c[2], a0, y.c[2]);
+                cfma(acc.c[3], a1, y.c[3]);
+            }
+        xs[tid] = acc;
+    }
+    __syncthreads();
+    if (!act) return;
+    // back rotation with the output phase; m-flip back for the reverse direction
+    acc = cols{{zero, zero, zero, zero}};
+    const T *E = tl + n * n + kk + n;
+    const cols *z = xs + d0 + nk(n, 0);
+#pragma unroll
+    for (int m = -L; m <= L; m++)
+        if (iab(m) <= n) {
+            constexpr auto sec = [](int mm) constexpr {
+                const int mm1 = imx(1, iab(mm));
+                return sec_off(mm < 0 ? -2 * mm - 1 : 2 * mm, L, L, VW) - mm1 * mm1;
+            };
+            const T e = E[sec(m)];
+            const cols a = z[m];
+#pragma unroll
+            for (int c = 0; c < 4; c++) crfma(acc.c[c], e, a.c[c]);
+        }
+    const cplx<T> po = phase(-kk);
+    cplx<T> *out = (dir ? dst_r : dst_f) + (int64_t)q * 4 * NB + amn(k, n, L);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const cplx<T> o = cmul_fixed(po, acc.c[c]);
+        out[c * NB] = cmk(sg * o.re, sg * o.im);
+    }
+}
+
+template <typename T>
+static hipError_t launch_pair_translate(int npairs, int L, hipStream_t st, const T *tab, const cplx<T> *src,
+                                        const int64_t *off_f, const int64_t *off_r, int64_t rs, int64_t ms,
+                                        cplx<T> *dst_f, cplx<T> *dst_r, const int *gate)
+{
+    switch (L) {
+#define CASE(LL) \
+    case LL: \
+        hipLaunchKernelGGL((pair_translate_kernel<T, LL>), dim3(npairs), dim3(pair_threads<T, LL>()), 0, st, tab, src, \
+                           off_f, off_r, rs, ms, dst_f, dst_r, gate); \
+        break;
+        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+#undef CASE
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 // anode[r][p][n][cell] = sum over spheres of the cell of asph[i][r][p][n]
 template <typename T>
 __global__ void node_reduce_kernel(const cplx<T> *__restrict__ asph, const int *__restrict__ cstart,
@@ -974,7 +1138,7 @@ struct FftOp {
     // device structures
     int *d_cstart = nullptr, *d_cmem = nullptr, *d_sstart = nullptr, *d_sent = nullptr;
     int64_t *d_off_sph = nullptr, *d_off_node = nullptr, *d_off_pj = nullptr, *d_off_pi = nullptr;
-    unsigned char *d_ident_j = nullptr, *d_ident_h = nullptr;
+    unsigned char *d_ident_j = nullptr;
     double *d_rt_j = nullptr, *d_rt_h = nullptr;
     void *jtab[2] = {nullptr, nullptr}, *htab[2] = {nullptr, nullptr};
     bool ready[2] = {false, false};
@@ -1259,7 +1423,6 @@ void fft_destroy(FftOp *f)
     ffree(f->d_off_pj);
     ffree(f->d_off_pi);
     ffree(f->d_ident_j);
-    ffree(f->d_ident_h);
     ffree(f->d_rt_j);
     ffree(f->d_rt_h);
     delete f;
@@ -1405,7 +1568,7 @@ int fft_setup(FftOp *f, int prec, hipStream_t st)
             for (int e : ent[i]) sent.push_back(e);
         }
         std::vector<int64_t> off_sph(n), off_node(n), off_pj(f->npairs), off_pi(f->npairs);
-        std::vector<unsigned char> ij(n), ih(std::max(1, f->npairs), 0);
+        std::vector<unsigned char> ij(n);
         std::vector<double> rtj(3 * (size_t)n), rth(3 * (size_t)std::max(1, f->npairs));
         for (int i = 0; i < n; i++) {
             off_sph[i] = (int64_t)i * 2 * NBP;
@@ -1434,7 +1597,6 @@ int fft_setup(FftOp *f, int prec, hipStream_t st)
         FCHK(falloc(&f->d_off_pj, sizeof(int64_t) * std::max(1, f->npairs)));
         FCHK(falloc(&f->d_off_pi, sizeof(int64_t) * std::max(1, f->npairs)));
         FCHK(falloc(&f->d_ident_j, n));
-        FCHK(falloc(&f->d_ident_h, std::max(1, f->npairs)));
         FCHK(falloc(&f->d_rt_j, sizeof(double) * rtj.size()));
         FCHK(falloc(&f->d_rt_h, sizeof(double) * rth.size()));
         FCHK(hipMemcpy(f->d_cstart, cstart.data(), sizeof(int) * cstart.size(), hipMemcpyHostToDevice));
@@ -1446,7 +1608,6 @@ int fft_setup(FftOp *f, int prec, hipStream_t st)
         if (f->npairs) {
             FCHK(hipMemcpy(f->d_off_pj, off_pj.data(), sizeof(int64_t) * f->npairs, hipMemcpyHostToDevice));
             FCHK(hipMemcpy(f->d_off_pi, off_pi.data(), sizeof(int64_t) * f->npairs, hipMemcpyHostToDevice));
-            FCHK(hipMemcpy(f->d_ident_h, ih.data(), f->npairs, hipMemcpyHostToDevice));
         }
         FCHK(hipMemcpy(f->d_ident_j, ij.data(), n, hipMemcpyHostToDevice));
         FCHK(hipMemcpy(f->d_rt_j, rtj.data(), sizeof(double) * rtj.size(), hipMemcpyHostToDevice));
@@ -1506,7 +1667,7 @@ template <typename T> static int matvec_t(FftOp *f, int nrhs, const double *ain,
     const int64_t rs_sph = (int64_t)f->npad * 2 * NBP;
     // sphere -> node (J translation, :573-626)
     dim3 lg(n);
-    const size_t ljb = list_translate_lds<T>(LG, Lp), lhb = list_translate_lds<T>(Lp, Lp);
+    const size_t ljb = list_translate_lds<T>(LG, Lp);
     FCHK((launch_list_translate<T, 0>)(lg, ljb, st, jt, n, LG, Lp, xin, f->d_off_sph, rs_sph, (int64_t)NBP, (int64_t)1,
                                      f->d_ident_j, asph, gate));
     int64_t nn4 = (int64_t)4 * nblk * f->ncells;
@@ -1559,11 +1720,8 @@ template <typename T> static int matvec_t(FftOp *f, int nrhs, const double *ain,
                                      f->d_ident_j, far, gate));
     // near-field pairs, both directions (local_sphere_to_sphere_expansion)
     if (f->npairs) {
-        dim3 pg(f->npairs);
-        FCHK((launch_list_translate<T, 0>)(pg, lhb, st, ht, f->npairs, Lp, Lp, xin, f->d_off_pj, rs_sph, (int64_t)NBP,
-                                         (int64_t)1, f->d_ident_h, nf, gate));
-        FCHK((launch_list_translate<T, 1>)(pg, lhb, st, ht, f->npairs, Lp, Lp, xin, f->d_off_pi, rs_sph, (int64_t)NBP,
-                                         (int64_t)1, f->d_ident_h, nr, gate));
+        FCHK(launch_pair_translate<T>(f->npairs, Lp, st, ht, xin, f->d_off_pj, f->d_off_pi, rs_sph, (int64_t)NBP, nf, nr,
+                                      gate));
     }
     int64_t ns4 = (int64_t)n * 4 * NBP;
     hipLaunchKernelGGL(sphere_reduce_kernel<T>, dim3((unsigned)((ns4 + 255) / 256)), dim3(256), 0, st, far, nf, nr,
