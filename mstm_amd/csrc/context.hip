@@ -122,7 +122,7 @@ struct mstm_hip_ctx {
     size_t kv_n = 0;
     double *d_partials = nullptr;
     std::vector<double> h_partials;
-    BicgScal *d_bscal = nullptr;  // device-resident BiCG scalars of two systems
+    BicgScal *d_bscal = nullptr;  // device-resident BiCG scalars of two systems, twice
     BicgScal *h_bscal = nullptr;  // their pinned host copy
     bool graphs = true;           // replay lazily read BiCG iterations from HIP graphs
     int *d_gate = nullptr;        // 1 while any of those systems is active
@@ -414,7 +414,7 @@ int mstm_hip_create(mstm_hip_ctx **ctx, int device)
     HIPCHK(hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking));
     HIPCHK(dalloc(&c->d_partials, sizeof(double) * 16 * krylov_grid()));  // 8 regions of one value per block
     c->h_partials.resize(16 * krylov_grid());
-    HIPCHK(dalloc(&c->d_bscal, sizeof(BicgScal) * 2));
+    HIPCHK(dalloc(&c->d_bscal, sizeof(BicgScal) * 4));
     HIPCHK(dalloc(&c->d_gate, sizeof(int)));
     HIPCHK(hipHostMalloc((void **)&c->h_bscal, sizeof(BicgScal) * 2, hipHostMallocDefault));
     *ctx = c;
@@ -860,7 +860,7 @@ static inline int pregion_off(int s) { return 2 * krylov_grid() * s; }
 // of an iteration are identical every time (iteration numbers, scalars and
 // the stop test live on the device; flags and pointers are fixed), so a
 // graph captured once per pattern of active systems and set of buffers
-// replaces 8 K launches by one.  Tile timing events are left out of the
+// replaces 6 K launches by one.  Tile timing events are left out of the
 // graph; the product count is kept.
 template <typename F>
 static int bicg_graph_steps(mstm_hip_ctx *c, int ns, int prec, const bool act[2], const double *x0, int K, F &&step)
@@ -1010,12 +1010,12 @@ static int bicg2_dev(mstm_hip_ctx *c, int ns, int niter, const double *eps, cons
         if (act[0] && act[1]) rc_ = matvec(c, 4, P[0], AP[0], f4, prec, use_fft);
         else rc_ = matvec(c, 2, act[0] ? P[0] : P[1], act[0] ? AP[0] : AP[1], f4, prec, use_fft);
         if (rc_) return rc_;
-        HIPCHK(launch_bicg_a_dev(AP[0], AW[0], P[0], W[0], 2 * (int64_t)V, n, pregion(c, 0), region, S, ns, c->st));
-        HIPCHK(launch_bicg_scal(2, c->d_partials, region, S, ns, n, c->st, gate));
-        HIPCHK(launch_bicg_b_dev(X[0], Rr[0], Q[0], P[0], AP[0], AW[0], (int64_t)V, 2 * (int64_t)V, S, n, pregion(c, 0),
-                                 region, ns, c->st));
-        HIPCHK(launch_bicg_scal(3, c->d_partials, region, S, ns, n, c->st, gate));
-        HIPCHK(launch_bicg_c_dev(P[0], W[0], Rr[0], Q[0], (int64_t)V, 2 * (int64_t)V, S, n, ns, c->st));
+        double *den = pregion(c, 2);  // partial sums of step a, those of step b in regions 0 and 1
+        HIPCHK(launch_bicg_a_dev(AP[0], AW[0], P[0], W[0], 2 * (int64_t)V, n, den, region, S, ns, c->st));
+        HIPCHK(launch_bicg_b_dev(X[0], Rr[0], Q[0], P[0], AP[0], AW[0], (int64_t)V, 2 * (int64_t)V, S, S + 2, n, den,
+                                 pregion(c, 0), region, ns, c->st));
+        HIPCHK(launch_bicg_c_dev(P[0], W[0], Rr[0], Q[0], (int64_t)V, 2 * (int64_t)V, S + 2, S, n, pregion(c, 0), region,
+                                 ns, c->st, gate));
         return 0;
     };
     int iter = 1, synced = 0;
@@ -1065,7 +1065,7 @@ static int bicg2_dev(mstm_hip_ctx *c, int ns, int niter, const double *eps, cons
 // ---------------------------------------------------------------------------
 struct BicgBlock {
     int np = 0, G = 1;  // pairs, workgroups per tile of the product
-    double *x, *b, *pw, *cap, *r, *q, *partials, *xin, *part;
+    double *x, *b, *pw, *cap, *r, *q, *partials, *den, *xin, *part;
     BicgScal *sc;
     int *gate;
 };
@@ -1087,9 +1087,10 @@ static size_t bicg_block_layout(const mstm_hip_ctx *c, unsigned char *base, Bicg
     put(k.r, 2 * V * np);
     put(k.q, 2 * V * np);
     put(k.partials, sizeof(double) * 4 * (size_t)krylov_grid() * 2 * np);
+    put(k.den, sizeof(double) * 4 * (size_t)krylov_grid() * 2 * np);
     put(k.xin, col * np);
     put(k.part, col * np * c->nblocks * k.G);
-    put(k.sc, sizeof(BicgScal) * 2 * np);
+    put(k.sc, sizeof(BicgScal) * 4 * np);
     put(k.gate, sizeof(int) * np);
     return o;
 }
@@ -1145,12 +1146,11 @@ static int bicg_block(mstm_hip_ctx *c, const BicgBlock &k, int niter, double eps
         const int nst = std::min(K, niter - iter);
         for (int q = 0; q < nst; q++) {
             if (int rc = product(4, k.pw, k.cap, f4, k.gate)) return rc;
-            HIPCHK(launch_bicg_a_dev(k.cap, k.cap + V, k.pw, k.pw + V, 2 * V, n, k.partials, region, k.sc, ns, c->st));
-            HIPCHK(launch_bicg_scal(2, k.partials, region, k.sc, ns, n, c->st, k.gate));
-            HIPCHK(launch_bicg_b_dev(k.x, k.r, k.q, k.pw, k.cap, k.cap + V, V, 2 * V, k.sc, n, k.partials, region, ns,
-                                     c->st));
-            HIPCHK(launch_bicg_scal(3, k.partials, region, k.sc, ns, n, c->st, k.gate));
-            HIPCHK(launch_bicg_c_dev(k.pw, k.pw + V, k.r, k.q, V, 2 * V, k.sc, n, ns, c->st));
+            HIPCHK(launch_bicg_a_dev(k.cap, k.cap + V, k.pw, k.pw + V, 2 * V, n, k.den, region, k.sc, ns, c->st));
+            HIPCHK(launch_bicg_b_dev(k.x, k.r, k.q, k.pw, k.cap, k.cap + V, V, 2 * V, k.sc, k.sc + ns, n, k.den,
+                                     k.partials, region, ns, c->st));
+            HIPCHK(launch_bicg_c_dev(k.pw, k.pw + V, k.r, k.q, V, 2 * V, k.sc + ns, k.sc, n, k.partials, region, ns,
+                                     c->st, k.gate));
         }
         iter += nst;
         HIPCHK(hipMemcpyAsync(hS, k.sc, sizeof(BicgScal) * ns, hipMemcpyDeviceToHost, c->st));

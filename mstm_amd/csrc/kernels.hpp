@@ -75,14 +75,15 @@ struct BicgScal {
     int active, it, brk;
     int cur;  // iterations begun while active (the loop's iteration number)
 };
-// step 0: enorm = |b|^2 (active = enorm != 0); 1: csk = r.r (inactive if 0);
-// 2: a new iteration (cur + 1), den = <w, A p>, cak = csk / den (breakdown:
-// inactive, it = cur, brk = 1); 3: <q, r>, <r, r>: err, stop test (it = cur),
-// cbk, csk.  The iteration number is counted on the device, so the launches
-// of an iteration are the same every time (they can be replayed from a
-// graph).  partials: region s of the system s at partials + s * region
-// (complex), one or two values per block of a vector of n elements.  gate
-// (optional): gate[q] set to 1 while system 2 q or 2 q + 1 is active, else 0.
+// Start-up: step 0, enorm = |b|^2 (active = enorm != 0); 1, csk = r.r (inactive
+// if 0).  Step b begins an iteration (cur + 1; den = <w, A p>, cak = csk / den;
+// breakdown: inactive, it = cur, brk = 1), step c ends it (<q, r>, <r, r>: err,
+// stop test, it = cur, cbk, csk); both read the states sc and write sn.  The
+// iteration number is counted on the device, so the launches of an iteration
+// are the same every time (they can be replayed from a graph).  Partial sums:
+// system s's at partials + s * region (complex), one or two values per block of
+// a vector of n elements.  gate (optional): gate[q] set to 1 while system 2 q or
+// 2 q + 1 is active, else 0.
 hipError_t launch_bicg_scal(int step, const double *partials, int64_t region, BicgScal *st, int ns, int n,
                             hipStream_t st_, int *gate = nullptr);
 // the vector steps of ns systems in one launch: system s's vectors at the
@@ -95,10 +96,11 @@ hipError_t launch_bicg_init(double *cr, double *cq, double *cw, double *cp, cons
 hipError_t launch_bicg_a_dev(double *cap, double *caw, const double *cp, const double *cw, int64_t sp, int n,
                              double *partials, int64_t region, const BicgScal *sc, int ns, hipStream_t st);
 hipError_t launch_bicg_b_dev(double *anp, double *cr, double *cq, const double *cp, const double *cap,
-                             const double *caw, int64_t sv, int64_t sp, const BicgScal *sc, int n, double *partials,
-                             int64_t region, int ns, hipStream_t st);
+                             const double *caw, int64_t sv, int64_t sp, const BicgScal *sc, BicgScal *sn, int n,
+                             const double *den, double *partials, int64_t region, int ns, hipStream_t st);
 hipError_t launch_bicg_c_dev(double *cp, double *cw, const double *cr, const double *cq, int64_t sv, int64_t sp,
-                             const BicgScal *sc, int n, int ns, hipStream_t st);
+                             const BicgScal *sc, BicgScal *sn, int n, const double *partials, int64_t region, int ns,
+                             hipStream_t st, int *gate);
 hipError_t launch_zdot(const double *a, const double *b, int n, int conj_a, double *partials, double *result,
                        hipStream_t st);
 hipError_t launch_zaxpby(double ar, double ai, const double *x, double br, double bi, double *y, int n, hipStream_t st);

@@ -63,33 +63,73 @@ static int bicg_grid(int n) { return imn(KGRID, (n + KB - 1) / KB); }
 // kernels of a system whose state is inactive return at once, so the host
 // may launch one iteration for both systems and learn only afterwards which
 // of them stopped.
+// An iteration's two reductions need no launch of their own: every workgroup
+// of the vector step that follows adds the partial sums (at most 512, in one
+// order) and works out the new scalars for itself; its first workgroup writes
+// them to the other of two state arrays, so none reads what another writes.
+// 20 spheres of order 5: 43 us per iteration with a 4.4 us launch after each
+// reduction, now 34 us.
 // ---------------------------------------------------------------------------
-// one workgroup per pair of systems
+// the sums of nv values per block over nb blocks, in all threads
+__device__ __forceinline__ void sum_blocks(const cplx<double> *__restrict__ p, int nv, int nb, cplx<double> *v)
+{
+    __shared__ cplx<double> red[2][KB];
+    for (int q = 0; q < nv; q++) {
+        cplx<double> s = cmk(0.0, 0.0);
+        for (int b = threadIdx.x; b < nb; b += KB) s = cadd(s, p[(int64_t)nv * b + q]);
+        red[q][threadIdx.x] = s;
+    }
+    __syncthreads();
+    for (int h = KB / 2; h > 0; h >>= 1) {
+        if (threadIdx.x < h)
+            for (int q = 0; q < nv; q++) red[q][threadIdx.x] = cadd(red[q][threadIdx.x], red[q][threadIdx.x + h]);
+        __syncthreads();
+    }
+    for (int q = 0; q < nv; q++) v[q] = red[q][0];
+    __syncthreads();
+}
+
+// a new iteration: den = v0 = <w, A p>
+__device__ __forceinline__ void bicg_alpha(BicgScal &S, cplx<double> v0)
+{
+    S.cur++;
+    if (v0.re == 0.0 && v0.im == 0.0) {  // breakdown: the Fortran loop exits here
+        S.active = 0;
+        S.it = S.cur;
+        S.brk = 1;
+        S.cak = cmk(0.0, 0.0);
+    } else {
+        S.cak = cdiv(S.csk, v0);
+    }
+}
+// its end: v0 = <q, r>, v1 = <r, r>
+__device__ __forceinline__ void bicg_beta(BicgScal &S, cplx<double> v0, cplx<double> v1)
+{
+    S.err = v1.re / S.enorm;
+    if (S.err < S.eps || (S.csk.re == 0.0 && S.csk.im == 0.0)) {
+        S.active = 0;
+        S.it = S.cur;
+        S.cbk = cmk(0.0, 0.0);
+    } else {
+        S.cbk = cdiv(v0, S.csk);
+        S.csk = v0;
+    }
+}
+
+// start-up, one workgroup per pair of systems: step 0, enorm = |b|^2; step 1,
+// csk = r.r
 __global__ __launch_bounds__(KB) void bicg_scal_kernel(int step, const cplx<double> *__restrict__ partials,
                                                        int64_t region, BicgScal *__restrict__ sc, int ns,
                                                        int nb, int *__restrict__ gate)
 {
-    __shared__ cplx<double> red[2][KB];
-    const int nv = step == 3 ? 2 : 1, sa = 2 * blockIdx.x, se = imn(ns, sa + 2);
+    const int sa = 2 * blockIdx.x, se = imn(ns, sa + 2);
+    int any = 0;
     for (int s = sa; s < se; s++) {
         BicgScal &S = sc[s];
         const bool skip = step >= 1 && !S.active;  // uniform: read by all threads
-        if (!skip) {
-            const cplx<double> *p = partials + region * s;
-            for (int q = 0; q < nv; q++) {
-                cplx<double> v = cmk(0.0, 0.0);
-                for (int b = threadIdx.x; b < nb; b += KB) v = cadd(v, p[(int64_t)nv * b + q]);
-                red[q][threadIdx.x] = v;
-            }
-            __syncthreads();
-            for (int h = KB / 2; h > 0; h >>= 1) {
-                if (threadIdx.x < h)
-                    for (int q = 0; q < nv; q++) red[q][threadIdx.x] = cadd(red[q][threadIdx.x], red[q][threadIdx.x + h]);
-                __syncthreads();
-            }
-        }
+        cplx<double> v0 = cmk(0.0, 0.0);
+        if (!skip) sum_blocks(partials + region * s, 1, nb, &v0);
         if (threadIdx.x == 0) {
-            const cplx<double> v0 = red[0][0], v1 = red[1][0];
             const cplx<double> zero = cmk(0.0, 0.0);
             if (step == 0) {
                 S.enorm = v0.re;
@@ -101,38 +141,14 @@ __global__ __launch_bounds__(KB) void bicg_scal_kernel(int step, const cplx<doub
                 S.cak = S.cbk = zero;
             } else if (skip) {
                 S.cak = S.cbk = zero;
-            } else if (step == 1) {
+            } else {
                 S.csk = v0;
                 if (v0.re == 0.0 && v0.im == 0.0) S.active = 0;  // it stays 0
-            } else if (step == 2) {
-                S.cur++;
-                if (v0.re == 0.0 && v0.im == 0.0) {  // breakdown: the Fortran loop exits here
-                    S.active = 0;
-                    S.it = S.cur;
-                    S.brk = 1;
-                    S.cak = zero;
-                } else {
-                    S.cak = cdiv(S.csk, v0);
-                }
-            } else {
-                S.err = v1.re / S.enorm;
-                if (S.err < S.eps || (S.csk.re == 0.0 && S.csk.im == 0.0)) {
-                    S.active = 0;
-                    S.it = S.cur;
-                    S.cbk = zero;
-                } else {
-                    S.cbk = cdiv(v0, S.csk);
-                    S.csk = v0;
-                }
             }
+            any |= S.active != 0;
         }
-        __syncthreads();
     }
-    if (gate && threadIdx.x == 0) {
-        int any = 0;
-        for (int s = sa; s < se; s++) any |= sc[s].active != 0;
-        gate[blockIdx.x] = any;
-    }
+    if (gate && threadIdx.x == 0) gate[blockIdx.x] = any;
 }
 
 // The vector steps of ns systems in one launch: system s = blockIdx.y has
@@ -200,11 +216,22 @@ __global__ void bicg_a_dev_kernel(cplx<double> *__restrict__ cap, cplx<double> *
 __global__ void bicg_b_dev_kernel(cplx<double> *__restrict__ anp, cplx<double> *__restrict__ cr,
                                   cplx<double> *__restrict__ cq, const cplx<double> *__restrict__ cp,
                                   const cplx<double> *__restrict__ cap, const cplx<double> *__restrict__ caw,
-                                  int64_t sv, int64_t sp, const BicgScal *__restrict__ sc, int n,
+                                  int64_t sv, int64_t sp, const BicgScal *__restrict__ sc,
+                                  BicgScal *__restrict__ sn, int n, const cplx<double> *__restrict__ den,
                                   cplx<double> *__restrict__ partials, int64_t region)
 {
     const int64_t y = blockIdx.y;
-    if (!sc[y].active) return;
+    BicgScal S = sc[y];
+    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+    if (S.active) {
+        cplx<double> v0;
+        sum_blocks(den + y * region, 1, gridDim.x, &v0);
+        bicg_alpha(S, v0);
+    } else {
+        S.cak = S.cbk = cmk(0.0, 0.0);
+    }
+    if (first) sn[y] = S;
+    if (!S.active) return;
     anp += y * sv;
     cr += y * sv;
     cq += y * sv;
@@ -212,7 +239,7 @@ __global__ void bicg_b_dev_kernel(cplx<double> *__restrict__ anp, cplx<double> *
     cap += y * sp;
     caw += y * sp;
     partials += y * region;
-    const cplx<double> cak = sc[y].cak, cakc = cconj(cak);
+    const cplx<double> cak = S.cak, cakc = cconj(cak);
     cplx<double> s[2] = {cmk(0.0, 0.0), cmk(0.0, 0.0)};
     for (int i = blockIdx.x * KB + threadIdx.x; i < n; i += gridDim.x * KB) {
         cplx<double> a = anp[i];
@@ -237,15 +264,35 @@ __global__ void bicg_b_dev_kernel(cplx<double> *__restrict__ anp, cplx<double> *
 // cp = cr + cbk cp ; cw = cq + conj(cbk) cw   (:928-929)
 __global__ void bicg_c_dev_kernel(cplx<double> *__restrict__ cp, cplx<double> *__restrict__ cw,
                                   const cplx<double> *__restrict__ cr, const cplx<double> *__restrict__ cq, int64_t sv,
-                                  int64_t sp, const BicgScal *__restrict__ sc, int n)
+                                  int64_t sp, const BicgScal *__restrict__ sc, BicgScal *__restrict__ sn, int n,
+                                  const cplx<double> *__restrict__ partials, int64_t region, int *__restrict__ gate)
 {
     const int64_t y = blockIdx.y;
-    if (!sc[y].active) return;
+    auto next = [&](int64_t s) {
+        BicgScal S = sc[s];
+        if (S.active) {
+            cplx<double> v[2];
+            sum_blocks(partials + s * region, 2, gridDim.x, v);
+            bicg_beta(S, v[0], v[1]);
+        } else {
+            S.cak = S.cbk = cmk(0.0, 0.0);
+        }
+        return S;
+    };
+    const BicgScal S = next(y);
+    if (blockIdx.x == 0) {
+        if (threadIdx.x == 0) sn[y] = S;
+        if (gate && y % 2 == 0) {  // the pair's gate: the other system's state too
+            const bool any = S.active || (y + 1 < gridDim.y && next(y + 1).active);
+            if (threadIdx.x == 0) gate[y / 2] = any;
+        }
+    }
+    if (!S.active) return;
     cp += y * sp;
     cw += y * sp;
     cr += y * sv;
     cq += y * sv;
-    const cplx<double> cbk = sc[y].cbk, cbkc = cconj(cbk);
+    const cplx<double> cbk = S.cbk, cbkc = cconj(cbk);
     for (int i = blockIdx.x * KB + threadIdx.x; i < n; i += gridDim.x * KB) {
         cplx<double> p = cr[i];
         cfma(p, cbk, cp[i]);
@@ -259,7 +306,7 @@ __global__ void bicg_c_dev_kernel(cplx<double> *__restrict__ cp, cplx<double> *_
 hipError_t launch_bicg_scal(int step, const double *partials, int64_t region, BicgScal *sc, int ns, int n,
                             hipStream_t st, int *gate)
 {
-    if (ns < 1 || step < 0 || step > 3) return hipErrorInvalidValue;
+    if (ns < 1 || step < 0 || step > 1) return hipErrorInvalidValue;
     hipLaunchKernelGGL(bicg_scal_kernel, dim3((ns + 1) / 2), dim3(KB), 0, st, step,
                        reinterpret_cast<const cplx<double> *>(partials), region, sc, ns, bicg_grid(n), gate);
     return hipGetLastError();
@@ -289,20 +336,21 @@ hipError_t launch_bicg_a_dev(double *cap, double *caw, const double *cp, const d
     return hipGetLastError();
 }
 hipError_t launch_bicg_b_dev(double *anp, double *cr, double *cq, const double *cp, const double *cap,
-                             const double *caw, int64_t sv, int64_t sp, const BicgScal *sc, int n, double *partials,
-                             int64_t region, int ns, hipStream_t st)
+                             const double *caw, int64_t sv, int64_t sp, const BicgScal *sc, BicgScal *sn, int n,
+                             const double *den, double *partials, int64_t region, int ns, hipStream_t st)
 {
     typedef cplx<double> Z;
     hipLaunchKernelGGL(bicg_b_dev_kernel, dim3(bicg_grid(n), ns), dim3(KB), 0, st, (Z *)anp, (Z *)cr, (Z *)cq, (const Z *)cp,
-                       (const Z *)cap, (const Z *)caw, sv / 2, sp / 2, sc, n, (Z *)partials, region);
+                       (const Z *)cap, (const Z *)caw, sv / 2, sp / 2, sc, sn, n, (const Z *)den, (Z *)partials, region);
     return hipGetLastError();
 }
 hipError_t launch_bicg_c_dev(double *cp, double *cw, const double *cr, const double *cq, int64_t sv, int64_t sp,
-                             const BicgScal *sc, int n, int ns, hipStream_t st)
+                             const BicgScal *sc, BicgScal *sn, int n, const double *partials, int64_t region, int ns,
+                             hipStream_t st, int *gate)
 {
     typedef cplx<double> Z;
     hipLaunchKernelGGL(bicg_c_dev_kernel, dim3(bicg_grid(n), ns), dim3(KB), 0, st, (Z *)cp, (Z *)cw, (const Z *)cr,
-                       (const Z *)cq, sv / 2, sp / 2, sc, n);
+                       (const Z *)cq, sv / 2, sp / 2, sc, sn, n, (const Z *)partials, region, gate);
     return hipGetLastError();
 }
 hipError_t launch_zaxpby(double ar, double ai, const double *x, double br, double bi, double *y, int n, hipStream_t st)
