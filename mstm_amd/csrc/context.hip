@@ -1232,9 +1232,11 @@ static int oos2_dev(mstm_hip_ctx *c, int ns, int nord, const double *eps, const 
 // GMRES(m) (Saad & Schultz, SIAM J. Sci. Stat. Comput. 7, 856 (1986)) for
 // ns = 1 or 2 systems A d_s = b_s at once, from d_s = 0.  Arnoldi vectors
 // are FP64 and orthogonalised by classical Gram-Schmidt applied twice; the
-// products run at precision prec, one column per system (both systems in one launch) -- half the columns of a BiCG step.  A
-// system stops when its residual estimate |g_{j+1}|^2/|b|^2 < eps[s];
-// restarts every m steps from the residual b - A d.  it[s]: Arnoldi steps.
+// products run at precision prec, one column per system (both systems in one
+// launch) -- half the columns of a BiCG step.  A system stops when its residual
+// estimate |g_{j+1}|^2/|b|^2 < eps[s], or for good at a step or a residual that
+// is not finite, with the correction of the steps before and err[s] >= eps[s];
+// it restarts every m steps from the residual b - A d.  it[s]: Arnoldi steps.
 // Projections, rotations and the stop test stay on the device (launch_gm_step);
 // the host enqueues one step ahead of the state it has read, and a step of
 // systems that have all stopped returns at once (gate).
@@ -1278,8 +1280,8 @@ static int gmres2_dev(mstm_hip_ctx *c, int ns, int niter, const double *eps, con
         double v[2];
         reduce_region(c, pregion_off(q), 1, v);
         bb[q] = v[0];
-        open[q] = bb[q] > 0.0;
-        err[q] = open[q] ? 1.0 : 0.0;
+        open[q] = gm_opens(bb[q], bb[q], 0.0, 0, 1);
+        err[q] = bb[q] == 0.0 ? 0.0 : 1.0;
     }
     int f2[2] = {2, 2};
     for (int cycle = 0; open[0] || (ns == 2 && open[1]); cycle++) {
@@ -1311,13 +1313,12 @@ static int gmres2_dev(mstm_hip_ctx *c, int ns, int niter, const double *eps, con
                 if (!open[q]) continue;
                 double v[2];
                 reduce_region(c, pregion_off(q), 1, v);
-                beta[q] = std::sqrt(std::max(v[0], 0.0));
-                err[q] = v[0] / bb[q];
-                if (err[q] < eps[q] || it[q] >= niter || beta[q] == 0.0) {
+                if (gm_finite(v[0])) err[q] = v[0] / bb[q];
+                if (!gm_opens(v[0], bb[q], eps[q], it[q], niter)) {
                     open[q] = false;
-                    beta[q] = 0.0;
                     continue;
                 }
+                beta[q] = std::sqrt(v[0]);
                 HIPCHK(hipMemcpyAsync(basis(0, q), T + V * q, sizeof(double) * V, hipMemcpyDeviceToDevice, c->st));
             }
             if (!open[0] && !(ns == 2 && open[1])) break;

@@ -3,6 +3,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "gmres.hpp"
 
 // context.hip: vector-coupling constants of axialtrancoefinit for orders <= LM
 void vcc_table(int LM, std::vector<double> &h);
@@ -106,19 +107,6 @@ hipError_t launch_zdot(const double *a, const double *b, int n, int conj_a, doub
 hipError_t launch_zaxpby(double ar, double ai, const double *x, double br, double bi, double *y, int n, hipStream_t st);
 // GMRES (restart length GM_M at most) with its small quantities on the device,
 // one or two systems; see krylov.hip
-#define GM_M 120
-struct GmSys {
-    double bb, eps, err, scale;  // |b|^2, stop test |g|^2 / bb < eps, its last value; 1 / norm of the next vector
-    int active, done;            // iterating; stopped on eps or niter
-    int k, it0, niter, m;        // steps of this cycle, steps before it, step limits
-    double cs[GM_M];
-    cplx<double> sn[GM_M], g[GM_M + 1], h[2][GM_M + 1];
-    cplx<double> R[GM_M * (GM_M + 1) / 2];  // columns of the triangular factor
-};
-struct GmStart {
-    double bb, eps, beta;  // beta = |v_0| as given, 0: not in this cycle
-    int it0, niter, m;
-};
 struct GmStat {  // what the host reads after a step
     double err;
     int active, done, k;

@@ -525,32 +525,7 @@ __global__ __launch_bounds__(KB) void gm_final_kernel(int nv, int nb, GmSys *__r
         if (threadIdx.x == 0) {
             double ww = 0.0;
             for (int b = 0; b < nb; b++) ww += sq[b];
-            const double hn = sqrt(ww > 0.0 ? ww : 0.0);
-            Z *R = S.R + (j * (j + 1)) / 2;
-            Z cur = col[0];
-            for (int r = 0; r < j; r++) {  // earlier rotations on column j
-                const Z b = col[r + 1];
-                R[r] = cadd(cscale(cur, cs[r]), cmul(sn[r], b));
-                cur = csub(cscale(b, cs[r]), cmul(cconj(sn[r]), cur));
-            }
-            const double ca = sqrt(cur.re * cur.re + cur.im * cur.im), nu = sqrt(ca * ca + hn * hn);
-            double c = 0.0;
-            Z s = cmk(1.0, 0.0);
-            if (ca != 0.0) {
-                c = ca / nu;
-                s = cscale(cur, hn / (ca * nu));
-            }
-            R[j] = cadd(cscale(cur, c), cscale(s, hn));
-            S.cs[j] = c;
-            S.sn[j] = s;
-            const Z gj = S.g[j], gn = cmul(cmk(-s.re, s.im), gj);
-            S.g[j + 1] = gn;
-            S.g[j] = cscale(gj, c);
-            S.k = nv;
-            S.scale = 1.0 / hn;
-            S.err = (gn.re * gn.re + gn.im * gn.im) / S.bb;
-            S.done = S.err < S.eps || S.it0 + nv >= S.niter;
-            if (S.done || hn == 0.0 || nu == 0.0 || nv == S.m) S.active = 0;
+            gm_column(S, col, cs, sn, nv, ww);
         }
         __syncthreads();
         any |= S.active;
@@ -573,8 +548,7 @@ __global__ __launch_bounds__(128) void gm_solve_kernel(GmSys *__restrict__ sys)
     for (int r = k - 1; r >= 0; r--) {
         const Z *R = S.R + (r * (r + 1)) / 2;
         if (t == r) {
-            const Z d = R[r];
-            piv = d.re != 0.0 || d.im != 0.0 ? cdiv(g, d) : cmk(0.0, 0.0);
+            piv = gm_pivot(g, R[r]);
             S.h[0][r] = piv;
         }
         __syncthreads();
@@ -609,19 +583,7 @@ __global__ void gm_begin_kernel(GmSys *__restrict__ sys, int ns, GmStart a, GmSt
     const int q = threadIdx.x;
     if (q == 0) *gate = 1;
     if (q >= ns) return;
-    const GmStart &st = q ? b : a;
-    GmSys &S = sys[q];
-    S.bb = st.bb;
-    S.eps = st.eps;
-    S.err = 0.0;
-    S.active = st.beta > 0.0;
-    S.done = 0;
-    S.k = 0;
-    S.it0 = st.it0;
-    S.niter = st.niter;
-    S.m = st.m;
-    S.scale = 1.0 / st.beta;
-    S.g[0] = cmk(st.beta, 0.0);
+    gm_begin(sys[q], q ? b : a);
 }
 
 static int gm_chunks(int n) { return imn(KGRID, (n + KB - 1) / KB); }

@@ -50,3 +50,21 @@ def test_mixed_gmres_iteration_limit(gpu_ctx):
     st = gpu_ctx.stats()
     assert r["istat"] == 1 and r["iterations"] >= 5
     assert st["matvecs_fp32"] == 5 and st["iters_fp32"] == 10
+
+
+def test_mixed_falls_back_when_fp32_overflows(gpu_ctx):
+    """Two touching grains beside a sphere of order 8: at the common order their
+    table holds h_16(0.04), about 1e41, above the FP32 range, so every FP32
+    product is not finite.  The mixed solver ends its inner solves and answers
+    with FP64 BiCG."""
+    from mstm_amd.solver import SOLVE_MIXED, SOLVE_PLAIN
+
+    pos = np.array([[0.0, 0.0, 0.0], [4.65, 0.0, 0.0], [4.65, 0.04, 0.0], [0.0, 0.0, 12.0]])
+    gpu_ctx.set_spheres(pos, np.array([4.6, 0.02, 0.02, 4.0]), np.full(4, 1.4 + 0.01j), 1.0, 1e-6)
+    assert gpu_ctx.orders()[0].max() == 8
+    ref = gpu_ctx.fixedorsoln(alpha=0.3, sinc=0.5, solver=SOLVE_PLAIN, eps=1e-14)
+    gpu_ctx.clear(clear_tables=False)
+    r = gpu_ctx.fixedorsoln(alpha=0.3, sinc=0.5, solver=SOLVE_MIXED, eps=1e-14)
+    st = gpu_ctx.stats()
+    assert r["istat"] == 0 and r["maxerr"] < 1e-14 and st["lig_fallbacks"] == 2
+    assert np.abs(r["amnp"] - ref["amnp"]).max() <= 1e-5 * np.abs(ref["amnp"]).max()
