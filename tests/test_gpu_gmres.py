@@ -53,15 +53,17 @@ def test_mixed_gmres_iteration_limit(gpu_ctx):
 
 
 def test_mixed_falls_back_when_fp32_overflows(gpu_ctx):
-    """Two touching grains beside a sphere of order 8: at the common order their
-    table holds h_16(0.04), about 1e41, above the FP32 range, so every FP32
-    product is not finite.  The mixed solver ends its inner solves and answers
-    with FP64 BiCG."""
-    from mstm_amd.solver import SOLVE_MIXED, SOLVE_PLAIN
+    """Two touching grains of x = 1e-4 beside a sphere of order 8: at the common
+    order their table's row of degree 1 holds h_9(2e-4), about 3e44, above the
+    FP32 range, and its product with the grains' zero padding is NaN.  The mixed
+    solver ends its inner solves and answers with FP64 BiCG."""
+    from mstm_amd.solver import FP32, SOLVE_MIXED, SOLVE_PLAIN
 
-    pos = np.array([[0.0, 0.0, 0.0], [4.65, 0.0, 0.0], [4.65, 0.04, 0.0], [0.0, 0.0, 12.0]])
-    gpu_ctx.set_spheres(pos, np.array([4.6, 0.02, 0.02, 4.0]), np.full(4, 1.4 + 0.01j), 1.0, 1e-6)
+    pos = np.array([[0.0, 0.0, 0.0], [4.65, 0.0, 0.0], [4.65, 2e-4, 0.0], [0.0, 0.0, 12.0]])
+    gpu_ctx.set_spheres(pos, np.array([4.6, 1e-4, 1e-4, 4.0]), np.full(4, 1.4 + 0.01j), 1.0, 1e-6)
     assert gpu_ctx.orders()[0].max() == 8
+    one = np.ones((1, gpu_ctx.number_eqns), complex)
+    assert np.isnan(gpu_ctx.sphereinteraction(one, [False], [True], precision=FP32)).any()
     ref = gpu_ctx.fixedorsoln(alpha=0.3, sinc=0.5, solver=SOLVE_PLAIN, eps=1e-14)
     gpu_ctx.clear(clear_tables=False)
     r = gpu_ctx.fixedorsoln(alpha=0.3, sinc=0.5, solver=SOLVE_MIXED, eps=1e-14)
