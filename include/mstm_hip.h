@@ -178,6 +178,12 @@ int mstm_hip_set_refinement_cycles(mstm_hip_ctx *ctx, int cycles);
  * a context whose stream cannot be captured switches to 0 by itself. */
 int mstm_hip_set_graphs(mstm_hip_ctx *ctx, int on);
 
+/* Direct solver: how often a workgroup of a factorization panel looks for the
+ * others' pivots, about half a microsecond each, before it gives up (no
+ * counterpart in MSTM; default 2097152, about a second).  A wait that runs out
+ * ends the factorization with MSTM_HIP_EHIP. */
+int mstm_hip_set_lu_wait(mstm_hip_ctx *ctx, int polls);
+
 /* ---------------------------------------------------------------------------
  * Post-solve observables of a single-origin expansion (a cluster without
  * plane boundaries, single_origin_expansion = .true., the reference default;

@@ -182,6 +182,7 @@ struct mstm_hip_ctx {
         int *piv = nullptr, *err = nullptr;
         void *scr = nullptr;
         int n = 0;
+        int polls = 1 << 21;  // looks of a panel's workgroups for each other, about a second
         bool ready = false;
         double build_ms = 0, factor_ms = 0, solve_ms = 0;
     } lu;
@@ -1773,7 +1774,8 @@ static int lu_setup(mstm_hip_ctx *c)
     c->lu.build_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
     HIPCHK(hipMemcpyAsync(c->lu.LU, c->lu.A, sizeof(double) * 2 * (size_t)n * n, hipMemcpyDeviceToDevice, c->st));
     HIPCHK(hipMemsetAsync(c->lu.err, 0, sizeof(int), c->st));
-    HIPCHK(launch_lu_factor(c->lu.LU, n, c->lu.vv, c->lu.piv, c->lu.err, c->lu.scr, c->st));
+    HIPCHK(launch_lu_factor(c->lu.LU, n, c->lu.vv, c->lu.piv, c->lu.err, c->lu.scr, c->lu.polls,
+                            c->st));
     int err = 0;
     HIPCHK(hipMemcpyAsync(&err, c->lu.err, sizeof(int), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
@@ -2239,6 +2241,14 @@ int mstm_hip_set_refinement_cycles(mstm_hip_ctx *c, int cycles)
     if (!c) return MSTM_HIP_EARG;
     if (cycles < 0 || cycles > 100) return fail(c, MSTM_HIP_EARG, "set_refinement_cycles: %d outside 0..100", cycles);
     c->max_ref = cycles;
+    return 0;
+}
+
+int mstm_hip_set_lu_wait(mstm_hip_ctx *c, int polls)
+{
+    if (!c) return MSTM_HIP_EARG;
+    if (polls < 0) return fail(c, MSTM_HIP_EARG, "set_lu_wait: %d polls", polls);
+    c->lu.polls = polls;
     return 0;
 }
 

@@ -143,7 +143,10 @@ hipError_t launch_lu_expand(const double *tab, int slot_elems, const int2 *pairs
 hipError_t launch_lu_identity(double *A, int n, hipStream_t st);
 hipError_t launch_lu_store(double *A, int n, int j0, int ncol, const double *th, int64_t ld, hipStream_t st);
 size_t lu_factor_scratch_bytes();
-hipError_t launch_lu_factor(double *LUm, int n, double *vv, int *piv, int *err, void *scratch, hipStream_t st);
+// *err |= 1 for a zero row, 2 where the workgroups of a panel did not meet
+// within `polls` looks (half a microsecond each); the factors are then unusable
+hipError_t launch_lu_factor(double *LUm, int n, double *vv, int *piv, int *err, void *scratch, int polls,
+                            hipStream_t st);
 hipError_t launch_lu_solve(const double *LUm, int n, const int *piv, double *b, int64_t ld, int nrhs, hipStream_t st);
 hipError_t launch_lu_resid(const double *A, int n, const double *x, const double *p, double *r, hipStream_t st);
 hipError_t launch_s00_moments(const double *a0, int T, const double *cgm, const double *cg1, double *out,

@@ -89,9 +89,10 @@ __global__ __launch_bounds__(256) void lu_rowscale_kernel(const zc *A, int n, do
 // The exchange needs no fence: a word carries 32 bits of data and the column's
 // number, and a reader polls a word until the number is there.  Two sets of
 // words alternate: a workgroup publishes column j+2 only after all have
-// published j+1, hence read j.  All workgroups (64 at most) are resident, each
-// waiting only for workgroups of its own launch; a wait is bounded.  The rest
-// of a column's update runs while the next column's candidates travel.
+// published j+1, hence read j.  A workgroup waits only for workgroups of its own
+// launch, and a wait is bounded: one that runs out sets *err, ends its
+// workgroup, hence the others' waits too, and the panels after it return at once.
+// The rest of a column's update runs while the next column's candidates travel.
 // Bound by latency: 8400 equations, 111 us for 32 columns, 8300 cycles each (two
 // trips through memory 2400, the pivot's row into LDS and the barrier 1500, the
 // update 2500, the pivot's reciprocal and the next column 1500) whatever the
@@ -102,7 +103,6 @@ __global__ __launch_bounds__(256) void lu_rowscale_kernel(const zc *A, int n, do
 #define LU_LL_ROW (4 * LU_NB)               // words of a panel row: two per double
 #define LU_LL_HEAD 4                        // a workgroup's candidate: value (2 words), row
 #define LU_LL_SET (LU_MAX_BLOCKS * LU_LL_HEAD + (LU_MAX_BLOCKS + 1) * LU_LL_ROW + 4)
-#define LU_SPIN (1 << 24)                   // polls of a wait (about half a microsecond each)
 typedef unsigned long long lu_word;
 
 __device__ __forceinline__ void ll_put(lu_word *p, unsigned v, unsigned seq)
@@ -116,11 +116,11 @@ __device__ __forceinline__ void ll_put(lu_word *p, double v, unsigned seq)
     ll_put(p + 1, (unsigned)b, seq);
 }
 // a double and, where idx is not null, the index behind it, once they carry
-// seq; act: lanes that wait.  False if the wait ran out.
-__device__ __forceinline__ bool ll_get(const lu_word *p, bool act, unsigned seq, double &v, int *idx)
+// seq; act: lanes that wait.  False if the wait ran out after `polls` looks.
+__device__ __forceinline__ bool ll_get(const lu_word *p, bool act, unsigned seq, int polls, double &v, int *idx)
 {
     lu_word h = 0, l = 0, x = 0;
-    for (int t = 0; t < LU_SPIN; t++) {
+    for (int t = 0; t < polls; t++) {
         bool ok = true;
         if (act) {
             h = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -137,9 +137,12 @@ __device__ __forceinline__ bool ll_get(const lu_word *p, bool act, unsigned seq,
     return false;
 }
 
-__global__ void lu_clear_kernel(lu_word *ll, int n)
+// no word has been published, and no row has been swapped: columns that a panel
+// gives up keep these pivots, which the later launches use as row numbers
+__global__ void lu_clear_kernel(lu_word *ll, int nll, int *piv, int n)
 {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) ll[i] = 0;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nll; i += gridDim.x * blockDim.x) ll[i] = 0;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) piv[i] = i;
 }
 
 // the largest value of a wave's lanes, the same in all (row shifts and row
@@ -172,10 +175,10 @@ __device__ __forceinline__ int last_lane(double mine, double v)
 }
 
 __global__ __launch_bounds__(256) void lu_panel_kernel(zc *A, int n, int c0, int nb, double *vv, int *piv, lu_word *ll,
-                                                       int *err)
+                                                       int *err, int polls)
 {
     __shared__ double sv[4], vvj;
-    __shared__ int si[4], six;
+    __shared__ int si[4], six, lost;
     // the pivot's row and row j of the panel, zeros behind (two sets: the last
     // column's are read until its update is complete)
     __shared__ zc prow2[2][2][2 * LU_NB];
@@ -183,6 +186,9 @@ __global__ __launch_bounds__(256) void lu_panel_kernel(zc *A, int n, int c0, int
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, blk = blockIdx.x, nblk = gridDim.x;
     const int i = c0 + blk * 256 + tid;
     const bool mine = i < n;
+    if (tid == 0) lost = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 2;
+    __syncthreads();
+    if (lost) return;  // a wait of an earlier panel ran out: the factorization has failed
     zc x[LU_NB];
 #pragma unroll
     for (int k = 0; k < LU_NB; k++) x[k] = mine && k < nb ? A[(int64_t)(c0 + k) * n + i] : cmk(0.0, 0.0);
@@ -263,14 +269,14 @@ __global__ __launch_bounds__(256) void lu_panel_kernel(zc *A, int n, int c0, int
         const double *jd = reinterpret_cast<const double *>(jrow);
         if (w == 0) {
             ll_put(rows + blk * LU_LL_ROW + 2 * lane, cd[lane], seq);
-            bool ok = ll_get(set + lane * LU_LL_HEAD, lane < nblk, seq, d, &ix);
+            bool ok = ll_get(set + lane * LU_LL_HEAD, lane < nblk, seq, polls, d, &ix);
             if (lane >= nblk || ix < 0) d = -1.0;
             v = wave_max(d);
             const int wb = last_lane(d, v);
             ix = wb < 0 ? j : __builtin_amdgcn_readlane(ix, wb);  // no finite candidate: keep row j
             if (ok && wb >= 0 && wb != blk) {
                 double c = 0.0;
-                ok = ll_get(rows + wb * LU_LL_ROW + 2 * lane, true, seq, c, nullptr);
+                ok = ll_get(rows + wb * LU_LL_ROW + 2 * lane, true, seq, polls, c, nullptr);
                 reinterpret_cast<double *>(crow)[lane] = c;
             }
             if (lane == 0) six = ok ? ix : -1;
@@ -280,18 +286,18 @@ __global__ __launch_bounds__(256) void lu_panel_kernel(zc *A, int n, int c0, int
                 if (lane == 0) ll_put(rowj + LU_LL_ROW, vvj, seq);
             } else {
                 double c = 0.0, vj = 0.0;
-                const bool ok = ll_get(rowj + 2 * lane, true, seq, c, nullptr) &&
-                                ll_get(rowj + LU_LL_ROW, true, seq, vj, nullptr);
+                const bool ok = ll_get(rowj + 2 * lane, true, seq, polls, c, nullptr) &&
+                                ll_get(rowj + LU_LL_ROW, true, seq, polls, vj, nullptr);
                 reinterpret_cast<double *>(jrow)[lane] = c;
                 if (lane == 0) {
                     vvj = vj;
-                    if (!ok) atomicOr(err, 2);
+                    if (!ok) lost = 1;
                 }
             }
         }
         __syncthreads();
         ix = six;
-        if (ix < 0) {  // a wait ran out
+        if (ix < 0 || lost) {  // a wait ran out
             if (tid == 0) atomicOr(err, 2);
             return;
         }
@@ -715,19 +721,20 @@ hipError_t launch_lu_store(double *A, int n, int j0, int ncol, const double *th,
 // scratch: the words of the panels' exchange
 size_t lu_factor_scratch_bytes() { return 2 * LU_LL_SET * sizeof(lu_word); }
 
-hipError_t launch_lu_factor(double *LUm, int n, double *vv, int *piv, int *err, void *scratch, hipStream_t st)
+hipError_t launch_lu_factor(double *LUm, int n, double *vv, int *piv, int *err, void *scratch, int polls,
+                            hipStream_t st)
 {
     if (n < 1 || n > LU_MAX_BLOCKS * 256) return hipErrorInvalidValue;
     zc *A = reinterpret_cast<zc *>(LUm);
     lu_word *ll = reinterpret_cast<lu_word *>(scratch);
-    hipLaunchKernelGGL(lu_clear_kernel, dim3(32), dim3(256), 0, st, ll, 2 * LU_LL_SET);
+    hipLaunchKernelGGL(lu_clear_kernel, dim3(32), dim3(256), 0, st, ll, 2 * LU_LL_SET, piv, n);
     hipLaunchKernelGGL(lu_rowscale_kernel, dim3((n + 63) / 64), dim3(256), 0, st, A, n, vv, err);
     hipError_t e = hipGetLastError();
     // one panel of nb columns at c0: pivot search, row swaps and elimination
     // inside the panel's own columns
     auto panel = [&](int c0, int nb) {
         hipLaunchKernelGGL(lu_panel_kernel, dim3((n - c0 + 255) / 256), dim3(256), 0, st, A, n, c0, nb, vv, piv, ll,
-                           err);
+                           err, polls);
     };
     auto swap = [&](int p0, int np, int k0, int k1) {  // pivots [p0, p0+np) on columns [k0, k1)
         if (k1 > k0)

@@ -370,6 +370,11 @@ class HipContext:
         issue the same launches one by one (same results)."""
         self._chk(self.L.mstm_hip_set_graphs(self.h, int(bool(on))), "set_graphs")
 
+    def set_lu_wait(self, polls: int = 1 << 21):
+        """Looks of a workgroup of the direct solver's panels for the others,
+        about half a microsecond each, before it gives up."""
+        self._chk(self.L.mstm_hip_set_lu_wait(self.h, int(polls)), "set_lu_wait")
+
     def clear(self, clear_tables=True):
         self._chk(self.L.mstm_hip_clear(self.h, int(bool(clear_tables))), "clear")
 

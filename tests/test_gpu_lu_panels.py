@@ -25,3 +25,28 @@ def test_lu_matches_bicg(gpu_ctx, n, x, spread, neq):
     r = gpu_ctx.fixedorsoln(alpha=0.4, sinc=0.3, solver=SOLVE_LU)
     t = gpu_ctx.fixedorsoln(alpha=0.4, sinc=0.3, solver=SOLVE_PLAIN, eps=1e-20, niter=1000)
     assert np.abs(r["amnp"] - t["amnp"]).max() <= 1e-7 * np.abs(t["amnp"]).max()
+
+
+def test_waits_that_run_out_end_the_factorization():
+    """No look at the other workgroups: every wait of the first panel runs out.
+    The factorization ends with an error, and the context solves again."""
+    import time
+
+    from mstm_amd import geometry as G
+    from mstm_amd.solver import SOLVE_LU, SOLVE_PLAIN, HipContext, MstmHipError
+
+    c = G.rsa_in_sphere(100, 2.0, 0.15, seed=3, ri=1.31 + 0.01j)
+    ctx = HipContext(0)
+    try:
+        ctx.set_spheres(c.pos, c.radius, c.ri, 1.0, 1e-6)
+        ctx.set_lu_wait(0)
+        t0 = time.perf_counter()
+        with pytest.raises(MstmHipError, match="did not meet"):
+            ctx.fixedorsoln(alpha=0.4, sinc=0.3, solver=SOLVE_LU)
+        assert time.perf_counter() - t0 < 5.0
+        ctx.set_lu_wait()
+        r = ctx.fixedorsoln(alpha=0.4, sinc=0.3, solver=SOLVE_LU)
+        t = ctx.fixedorsoln(alpha=0.4, sinc=0.3, solver=SOLVE_PLAIN, eps=1e-20, niter=1000)
+        assert np.abs(r["amnp"] - t["amnp"]).max() <= 1e-7 * np.abs(t["amnp"]).max()
+    finally:
+        ctx.close()
