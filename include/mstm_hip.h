@@ -180,8 +180,8 @@ int mstm_hip_set_graphs(mstm_hip_ctx *ctx, int on);
 
 /* Direct solver: how often a workgroup of a factorization panel looks for the
  * others' pivots, about half a microsecond each, before it gives up (no
- * counterpart in MSTM; default 2097152, about a second).  A wait that runs out
- * ends the factorization with MSTM_HIP_EHIP. */
+ * counterpart in MSTM; default 2097152, about a second).  The factorization is
+ * then done again without an exchange between workgroups. */
 int mstm_hip_set_lu_wait(mstm_hip_ctx *ctx, int polls);
 
 /* ---------------------------------------------------------------------------

@@ -1772,15 +1772,18 @@ static int lu_setup(mstm_hip_ctx *c)
     HIPCHK(hipStreamSynchronize(c->st));
     auto t1 = std::chrono::steady_clock::now();
     c->lu.build_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
-    HIPCHK(hipMemcpyAsync(c->lu.LU, c->lu.A, sizeof(double) * 2 * (size_t)n * n, hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemsetAsync(c->lu.err, 0, sizeof(int), c->st));
-    HIPCHK(launch_lu_factor(c->lu.LU, n, c->lu.vv, c->lu.piv, c->lu.err, c->lu.scr, c->lu.polls,
-                            c->st));
+    // where the workgroups of a panel did not meet (their CUs were held by other
+    // work), the factorization is done again without an exchange between them
     int err = 0;
-    HIPCHK(hipMemcpyAsync(&err, c->lu.err, sizeof(int), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
+    for (int capacity = lu_panel_capacity(c->device);; capacity = 0) {
+        HIPCHK(hipMemcpyAsync(c->lu.LU, c->lu.A, sizeof(double) * 2 * (size_t)n * n, hipMemcpyDeviceToDevice, c->st));
+        HIPCHK(hipMemsetAsync(c->lu.err, 0, sizeof(int), c->st));
+        HIPCHK(launch_lu_factor(c->lu.LU, n, c->lu.vv, c->lu.piv, c->lu.err, c->lu.scr, capacity, c->lu.polls, c->st));
+        HIPCHK(hipMemcpyAsync(&err, c->lu.err, sizeof(int), hipMemcpyDeviceToHost, c->st));
+        HIPCHK(hipStreamSynchronize(c->st));
+        if (!(err & 2) || !capacity) break;
+    }
     c->lu.factor_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t1).count();
-    if (err & 2) return fail(c, MSTM_HIP_EHIP, "direct solver: the workgroups of a panel did not meet");
     if (err) return fail(c, MSTM_HIP_EARG, "direct solver: lu decomposition failed (a zero row)");
     c->lu.ready = true;
     return 0;

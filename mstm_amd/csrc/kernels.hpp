@@ -143,10 +143,17 @@ hipError_t launch_lu_expand(const double *tab, int slot_elems, const int2 *pairs
 hipError_t launch_lu_identity(double *A, int n, hipStream_t st);
 hipError_t launch_lu_store(double *A, int n, int j0, int ncol, const double *th, int64_t ld, hipStream_t st);
 size_t lu_factor_scratch_bytes();
+// Workgroups of the panel kernel that a device holds at once, 0 if it cannot be
+// told; a panel of that many (at most LU_MAX_BLOCKS) exchanges pivots between
+// them, a longer one takes a launch per step.
+#define LU_MAX_BLOCKS 64
+int lu_panel_capacity(int device);
+inline bool lu_panel_exchanges(int rows, int capacity) { return (rows + 255) / 256 <= imn(LU_MAX_BLOCKS, capacity); }
 // *err |= 1 for a zero row, 2 where the workgroups of a panel did not meet
-// within `polls` looks (half a microsecond each); the factors are then unusable
-hipError_t launch_lu_factor(double *LUm, int n, double *vv, int *piv, int *err, void *scratch, int polls,
-                            hipStream_t st);
+// within `polls` looks (half a microsecond each); the factors are then unusable.
+// capacity 0: no panel exchanges.
+hipError_t launch_lu_factor(double *LUm, int n, double *vv, int *piv, int *err, void *scratch, int capacity,
+                            int polls, hipStream_t st);
 hipError_t launch_lu_solve(const double *LUm, int n, const int *piv, double *b, int64_t ld, int nrhs, hipStream_t st);
 hipError_t launch_lu_resid(const double *A, int n, const double *x, const double *p, double *r, hipStream_t st);
 hipError_t launch_s00_moments(const double *a0, int T, const double *cgm, const double *cg1, double *out,

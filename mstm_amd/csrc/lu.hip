@@ -89,9 +89,15 @@ __global__ __launch_bounds__(256) void lu_rowscale_kernel(const zc *A, int n, do
 // The exchange needs no fence: a word carries 32 bits of data and the column's
 // number, and a reader polls a word until the number is there.  Two sets of
 // words alternate: a workgroup publishes column j+2 only after all have
-// published j+1, hence read j.  A workgroup waits only for workgroups of its own
-// launch, and a wait is bounded: one that runs out sets *err, ends its
-// workgroup, hence the others' waits too, and the panels after it return at once.
+// published j+1, hence read j.  A workgroup takes a whole CU (135 KB of LDS) and
+// waits for the other workgroups of its launch, so all of them have to be
+// resident at once: a panel with more workgroups than the device holds takes
+// the route without an exchange (lu_pick_kernel).  Below that, other work on the
+// device that ends only delays them; several factorizations at once (contexts on
+// more than four queues, other processes) can hold each other's CUs, which is
+// why a wait is bounded.  One that runs out sets *err and ends its workgroup,
+// hence the others' waits too, and the panels after it return at once; the host
+// then factors again without an exchange.
 // The rest of a column's update runs while the next column's candidates travel.
 // Bound by latency: 8400 equations, 111 us for 32 columns, 8300 cycles each (two
 // trips through memory 2400, the pivot's row into LDS and the barrier 1500, the
@@ -99,7 +105,6 @@ __global__ __launch_bounds__(256) void lu_rowscale_kernel(const zc *A, int n, do
 // number of workgroups; a pick and an update launch per column took 275 us, the
 // panels of the whole factorization 72 ms, now 29 ms.
 // ---------------------------------------------------------------------------
-#define LU_MAX_BLOCKS 64                    // workgroups of a panel
 #define LU_LL_ROW (4 * LU_NB)               // words of a panel row: two per double
 #define LU_LL_HEAD 4                        // a workgroup's candidate: value (2 words), row
 #define LU_LL_SET (LU_MAX_BLOCKS * LU_LL_HEAD + (LU_MAX_BLOCKS + 1) * LU_LL_ROW + 4)
@@ -329,6 +334,76 @@ __global__ __launch_bounds__(256) void lu_panel_kernel(zc *A, int n, int c0, int
     vv[i] = vi;
 }
 static_assert(LU_NB == 32, "lu_panel_kernel: 64 doubles of a row on a wave, segments of 8 columns");
+
+// The route without an exchange, two launches per column, the same pivots and
+// operations: one workgroup picks the pivot of column j, swaps the panel's rows j
+// and piv[j] and leaves the pivot's reciprocal; then a thread per row takes the
+// rank-1 update.  8400 equations: 400 us for 32 columns on average, against 111.
+__global__ __launch_bounds__(1024) void lu_pick_kernel(zc *A, int n, int c0, int nb, int j, double *vv, int *piv,
+                                                       zc *rcp)
+{
+    __shared__ double sv[16];
+    __shared__ int si[16];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const zc *cj = A + (int64_t)j * n;
+    double v = -1.0;  // no candidate
+    int ix = -1;
+    for (int i = j + tid; i < n; i += 1024) {
+        const double vi = vv[i], dr = vi * cj[i].re, di = vi * cj[i].im, d = fma(dr, dr, di * di);
+        if (d >= 0.0 && d >= v) {
+            v = d;
+            ix = i;
+        }
+    }
+    auto take = [&](double ov, int oi) {  // ties to the larger row
+        if (oi >= 0 && (ix < 0 || ov > v || (ov == v && oi > ix))) {
+            v = ov;
+            ix = oi;
+        }
+    };
+    for (int off = 32; off > 0; off >>= 1) {
+        const double ov = __shfl_down(v, off, 64);
+        const int oi = __shfl_down(ix, off, 64);
+        take(ov, oi);
+    }
+    if (lane == 0) {
+        sv[w] = v;
+        si[w] = ix;
+    }
+    __syncthreads();
+    if (w) return;
+    v = sv[0];
+    ix = si[0];
+    for (int q = 1; q < 16; q++) take(sv[q], si[q]);
+    if (ix < 0) ix = j;  // no finite candidate: keep row j
+    if (lane == 0) {
+        piv[j] = ix;
+        if (ix != j) vv[ix] = vv[j];
+    }
+    if (lane < nb) {
+        zc *ck = A + (int64_t)(c0 + lane) * n;
+        zc a = ck[ix];
+        if (ix != j) {
+            ck[ix] = ck[j];
+            ck[j] = a;
+        }
+        if (c0 + lane == j) {
+            if (a.re == 0.0 && a.im == 0.0) ck[j] = a = cmk(1e-20, 0.0);
+            const double den = a.re * a.re + a.im * a.im;
+            rcp[0] = cmk(a.re / den, -a.im / den);
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void lu_column_kernel(zc *A, int n, int ce, int j, const zc *rcp)
+{
+    const int i = j + 1 + blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const zc l = cmul(A[(int64_t)j * n + i], rcp[0]);
+    A[(int64_t)j * n + i] = l;
+    for (int k = j + 1; k < ce; k++)  // no thread here writes row j
+        A[(int64_t)k * n + i] = csub(A[(int64_t)k * n + i], cmul(l, A[(int64_t)k * n + j]));
+}
 
 // the panel's row swaps on columns [k0, k1)
 __global__ void lu_swap_kernel(zc *A, int n, int c0, int nb, const int *piv, int k0, int k1)
@@ -718,23 +793,45 @@ hipError_t launch_lu_store(double *A, int n, int j0, int ncol, const double *th,
     return hipGetLastError();
 }
 
-// scratch: the words of the panels' exchange
-size_t lu_factor_scratch_bytes() { return 2 * LU_LL_SET * sizeof(lu_word); }
+// scratch: the words of the panels' exchange, a pivot's reciprocal
+size_t lu_factor_scratch_bytes() { return 2 * LU_LL_SET * sizeof(lu_word) + sizeof(zc); }
 
-hipError_t launch_lu_factor(double *LUm, int n, double *vv, int *piv, int *err, void *scratch, int polls,
-                            hipStream_t st)
+int lu_panel_capacity(int device)
+{
+    int cus = 0, per_cu = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lu_panel_kernel, 256, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return cus * per_cu;
+}
+
+hipError_t launch_lu_factor(double *LUm, int n, double *vv, int *piv, int *err, void *scratch, int capacity,
+                            int polls, hipStream_t st)
 {
     if (n < 1 || n > LU_MAX_BLOCKS * 256) return hipErrorInvalidValue;
     zc *A = reinterpret_cast<zc *>(LUm);
     lu_word *ll = reinterpret_cast<lu_word *>(scratch);
+    zc *rcp = reinterpret_cast<zc *>(ll + 2 * LU_LL_SET);
     hipLaunchKernelGGL(lu_clear_kernel, dim3(32), dim3(256), 0, st, ll, 2 * LU_LL_SET, piv, n);
     hipLaunchKernelGGL(lu_rowscale_kernel, dim3((n + 63) / 64), dim3(256), 0, st, A, n, vv, err);
     hipError_t e = hipGetLastError();
     // one panel of nb columns at c0: pivot search, row swaps and elimination
     // inside the panel's own columns
     auto panel = [&](int c0, int nb) {
-        hipLaunchKernelGGL(lu_panel_kernel, dim3((n - c0 + 255) / 256), dim3(256), 0, st, A, n, c0, nb, vv, piv, ll,
-                           err, polls);
+        const int rows = n - c0;
+        if (lu_panel_exchanges(rows, capacity)) {
+            hipLaunchKernelGGL(lu_panel_kernel, dim3((rows + 255) / 256), dim3(256), 0, st, A, n, c0, nb, vv, piv, ll,
+                               err, polls);
+            return;
+        }
+        for (int j = c0; j < c0 + nb; j++) {
+            hipLaunchKernelGGL(lu_pick_kernel, dim3(1), dim3(1024), 0, st, A, n, c0, nb, j, vv, piv, rcp);
+            if (j + 1 < n)
+                hipLaunchKernelGGL(lu_column_kernel, dim3((n - j - 1 + 255) / 256), dim3(256), 0, st, A, n, c0 + nb, j,
+                                   rcp);
+        }
     };
     auto swap = [&](int p0, int np, int k0, int k1) {  // pivots [p0, p0+np) on columns [k0, k1)
         if (k1 > k0)

@@ -372,7 +372,8 @@ class HipContext:
 
     def set_lu_wait(self, polls: int = 1 << 21):
         """Looks of a workgroup of the direct solver's panels for the others,
-        about half a microsecond each, before it gives up."""
+        about half a microsecond each, before the factorization is done
+        again without an exchange between workgroups."""
         self._chk(self.L.mstm_hip_set_lu_wait(self.h, int(polls)), "set_lu_wait")
 
     def clear(self, clear_tables=True):

@@ -27,26 +27,26 @@ def test_lu_matches_bicg(gpu_ctx, n, x, spread, neq):
     assert np.abs(r["amnp"] - t["amnp"]).max() <= 1e-7 * np.abs(t["amnp"]).max()
 
 
-def test_waits_that_run_out_end_the_factorization():
-    """No look at the other workgroups: every wait of the first panel runs out.
-    The factorization ends with an error, and the context solves again."""
-    import time
-
+@pytest.mark.parametrize("n,x,spread", [(1, 0.05, 0.0), (17, 0.3, 0.0), (33, 0.9, 0.7), (100, 2.0, 0.0)])
+def test_waits_that_run_out(n, x, spread):
+    """No look at the other workgroups: every wait of the first panel runs out,
+    and the factorization is done again without an exchange, on the context's
+    first matrix.  Both routes take the same operations; their factors differ
+    by rounding, times the condition (below 1e2) 1e-11."""
     from mstm_amd import geometry as G
-    from mstm_amd.solver import SOLVE_LU, SOLVE_PLAIN, HipContext, MstmHipError
+    from mstm_amd.solver import SOLVE_LU, HipContext
 
-    c = G.rsa_in_sphere(100, 2.0, 0.15, seed=3, ri=1.31 + 0.01j)
+    c = G.rsa_in_sphere(n, x, 0.15, seed=3, ri=1.31 + 0.01j)
+    radius = c.radius.copy()
+    radius[1::3] *= 1.0 - spread
     ctx = HipContext(0)
     try:
-        ctx.set_spheres(c.pos, c.radius, c.ri, 1.0, 1e-6)
+        ctx.set_spheres(c.pos, radius, c.ri, 1.0, 1e-6)
         ctx.set_lu_wait(0)
-        t0 = time.perf_counter()
-        with pytest.raises(MstmHipError, match="did not meet"):
-            ctx.fixedorsoln(alpha=0.4, sinc=0.3, solver=SOLVE_LU)
-        assert time.perf_counter() - t0 < 5.0
-        ctx.set_lu_wait()
         r = ctx.fixedorsoln(alpha=0.4, sinc=0.3, solver=SOLVE_LU)
-        t = ctx.fixedorsoln(alpha=0.4, sinc=0.3, solver=SOLVE_PLAIN, eps=1e-20, niter=1000)
-        assert np.abs(r["amnp"] - t["amnp"]).max() <= 1e-7 * np.abs(t["amnp"]).max()
+        ctx.set_lu_wait()
+        ctx.clear()
+        t = ctx.fixedorsoln(alpha=0.4, sinc=0.3, solver=SOLVE_LU)
+        assert np.abs(r["amnp"] - t["amnp"]).max() <= 1e-11 * np.abs(t["amnp"]).max()
     finally:
         ctx.close()
