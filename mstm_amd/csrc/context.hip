@@ -1124,11 +1124,20 @@ static int bicg_block(mstm_hip_ctx *c, const BicgBlock &k, int niter, double eps
     auto product = [&](int ncol, const double *in, double *out, const int *f, const int *gate) -> int {
         HIPCHK(launch_prep_quad<double>(in, (int)V, k.xin, ncol, f, c->nsph, c->npad, L, c->d_order, c->d_offset,
                                         c->d_an, np, c->st, gate));
+        hipEvent_t e0 = nullptr, e1 = nullptr;
+        if (c->timing) {
+            e0 = next_event(c);
+            e1 = next_event(c);
+            hipEventRecord(e0, c->st);
+        }
         HIPCHK(launch_direct_tiles<double>((const double *)d.tab, c->d_tiles, c->ntiles, L, k.xin, k.part, c->npad,
                                            ncol, k.G, np, c->st, gate));
+        if (e1) {
+            hipEventRecord(e1, c->st);
+            c->ev_prec.push_back(MSTM_HIP_FP64 + 2 * (ncol == 4));
+        }
         HIPCHK(launch_reduce_quad<double>(k.part, c->nblocks * k.G, out, (int)V, ncol, f, c->nsph, c->npad, L,
                                           c->d_order, c->d_offset, c->d_an, np, c->st, gate));
-        c->stats.matvecs[MSTM_HIP_FP64] += np;
         return 0;
     };
     for (int s = 0; s < ns; s++) {
@@ -1164,6 +1173,9 @@ static int bicg_block(mstm_hip_ctx *c, const BicgBlock &k, int niter, double eps
         err[s] = hS[s].err;
         c->stats.iters_fp64 += hS[s].active ? niter : hS[s].it - hS[s].brk;
     }
+    for (int s = 0; s < ns; s += 2)  // a pair's products: the start, and one per iteration of either system
+        if (hS[s].enorm != 0.0 || hS[s + 1].enorm != 0.0)
+            c->stats.matvecs[MSTM_HIP_FP64] += 1 + std::max(hS[s].cur, hS[s + 1].cur);
     return 0;
 }
 

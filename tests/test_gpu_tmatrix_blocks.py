@@ -37,3 +37,18 @@ def test_blocks_iteration_limit(gpu_ctx):
     gpu_ctx.set_spheres(*_cluster(40, 1.0, 0.0), 1.0, 1e-6)
     r = gpu_ctx.tmatrix_solution(eps=1e-14, niter=3, conveps=1e-3)
     assert r["istat"] == 1 and r["maxiter"] == 4 and r["maxerr"] > 1e-14
+
+
+def test_blocks_are_in_the_statistics(gpu_ctx):
+    """Tile times and products of the blocks, above the 500 spheres up to which
+    single systems are replayed from graphs: one start per column pair, one
+    four-column product per iteration of a pair."""
+    gpu_ctx.set_spheres(*_cluster(520, 0.2, 0.0), 1.0, 1e-3)
+    gpu_ctx.clear()
+    r = gpu_ctx.tmatrix_solution(eps=1e-6, conveps=1e-3)
+    st = gpu_ctx.stats()
+    assert st["tile_launches_fp64"] > 0 and st["tile4_launches_fp64"] > 0
+    assert 0.0 < st["tile_ms_fp64"] + st["tile4_ms_fp64"] < st["tmatrix_ms"]
+    pairs = st["tmatrix_solves"] // 2
+    assert pairs == sum(2 * l + 1 for l in range(1, r["T"] + 1))
+    assert pairs + st["iters_fp64"] / 2 <= st["matvecs_fp64"] <= pairs + st["iters_fp64"]
