@@ -2745,35 +2745,47 @@ int mstm_hip_tmatrix_solution(mstm_hip_ctx *c, double eps, int niter, double con
     if (int rc = ensure_vccd(c, T, c->Lmax)) return rc;
     if (int rc = grow(c, &c->obs.d_dist, c->obs.dist_bytes, sizeof(double) * V * 2 * (2 * T + 1))) return rc;
     const size_t per_group = sizeof(double) * 8 * (size_t)bT;
+    int G = std::min(nsph, 1024);
+    G = (int)std::max<size_t>(1, std::min<size_t>((size_t)G, ((size_t)1 << 30) / per_group));
+    if (int rc = grow(c, &c->obs.d_part, c->obs.part_bytes, per_group * G)) return rc;
+    if (int rc = grow(c, &c->obs.d_a0, c->obs.a0_bytes, per_group)) return rc;
+    if (int rc = grow(c, &c->obs.d_dq, c->obs.dq_bytes, sizeof(double) * 9 * nsph)) return rc;
     // Column pairs solved together (plain solver): the widest block of any
-    // degree; without room for it the pairs go one by one.
-    int np = 1;
+    // degree.  One allocation holds all that a block needs beyond a single
+    // pair's (systems, efficiencies, merge of npm pairs at once), after
+    // everything a single pair needs: without room for it the pairs go one by one.
+    int np = 1, npm = 1;
+    double *dq = c->obs.d_dq, *da0 = c->obs.d_a0, *dpart = c->obs.d_part;
     if (solver == MSTM_HIP_SOLVE_PLAIN) {
+        if (!c->dop[MSTM_HIP_FP64].ready)
+            if (int rc = mstm_hip_setup_direct(c, MSTM_HIP_FP64)) return rc;
         size_t need_blk = 0;
         for (int l = 1; l <= T; l++) {
             BicgBlock k = bicg_block_plan(c, 2 * l + 1);
             need_blk = std::max(need_blk, bicg_block_layout(c, nullptr, k));
             np = std::max(np, k.np);
         }
-        if (np > 1 && (!c->obs.d_blk || c->obs.blk_bytes < need_blk)) {
+        npm = (int)std::max<size_t>(1, std::min<size_t>((size_t)np, ((size_t)1 << 28) / (per_group * G)));
+        size_t o[4] = {(need_blk + 255) / 256 * 256};  // the block's systems, then efficiencies, merged columns, partials
+        o[1] = o[0] + (sizeof(double) * 9 * nsph * np + 255) / 256 * 256;
+        o[2] = o[1] + (per_group * np + 255) / 256 * 256;
+        o[3] = o[2] + per_group * G * npm;
+        if (np > 1 && (!c->obs.d_blk || c->obs.blk_bytes < o[3])) {
             dfree(c->obs.d_blk);
             c->obs.blk_bytes = 0;
-            if (dalloc(&c->obs.d_blk, need_blk) == hipSuccess) c->obs.blk_bytes = need_blk;
+            if (dalloc(&c->obs.d_blk, o[3]) == hipSuccess) c->obs.blk_bytes = o[3];
             else {
                 (void)hipGetLastError();
                 c->obs.d_blk = nullptr;
-                np = 1;
+                np = npm = 1;
             }
         }
-        if (np > 1 && !c->dop[MSTM_HIP_FP64].ready)
-            if (int rc = mstm_hip_setup_direct(c, MSTM_HIP_FP64)) return rc;
+        if (np > 1) {
+            dq = reinterpret_cast<double *>(c->obs.d_blk + o[0]);
+            da0 = reinterpret_cast<double *>(c->obs.d_blk + o[1]);
+            dpart = reinterpret_cast<double *>(c->obs.d_blk + o[2]);
+        }
     }
-    int G = std::min(nsph, 1024);
-    G = (int)std::max<size_t>(1, std::min<size_t>((size_t)G, ((size_t)1 << 30) / per_group));
-    const int npm = (int)std::max<size_t>(1, std::min<size_t>((size_t)np, ((size_t)1 << 28) / (per_group * G)));  // merged together
-    if (int rc = grow(c, &c->obs.d_part, c->obs.part_bytes, per_group * G * npm)) return rc;
-    if (int rc = grow(c, &c->obs.d_a0, c->obs.a0_bytes, per_group * np)) return rc;
-    if (int rc = grow(c, &c->obs.d_dq, c->obs.dq_bytes, sizeof(double) * 9 * nsph * np)) return rc;
     // vol_radius (mstm-input-37.f90:1205-1211): real(4) exponent .333333
     double vr = 0.0;
     for (int i = 0; i < nsph; i++) vr += c->radius[i] * c->radius[i] * c->radius[i];
@@ -2856,14 +2868,14 @@ int mstm_hip_tmatrix_solution(mstm_hip_ctx *c, double eps, int niter, double con
             }
             // per-sphere efficiencies of each column (qefficiencyfactors, npol = 1)
             HIPCHK(launch_qeff(xs, dp, 2 * n, nsph, c->d_radius, c->d_order, c->d_offset, c->d_mieoff, c->d_an,
-                               c->rimed, c->obs.d_dq, c->st, nk));
-            HIPCHK(hipMemcpyAsync(hq, c->obs.d_dq, sizeof(double) * 9 * nsph * nk, hipMemcpyDeviceToHost, c->st));
+                               c->rimed, dq, c->st, nk));
+            HIPCHK(hipMemcpyAsync(hq, dq, sizeof(double) * 9 * nsph * nk, hipMemcpyDeviceToHost, c->st));
             // the columns merged to the origin at order l (target orders min(l, torder_i))
             for (int p = 0; p < nk; p += npm)
                 HIPCHK(launch_merge(xs + 2 * V * p, n, c->d_order, c->d_offset, c->obs.d_torder, c->d_pos, nsph, l,
-                                    c->Lmax, c->obs.r0, c->rimed, c->obs.d_vccm, c->obs.d_part, G,
-                                    c->obs.d_a0 + (size_t)8 * b0 * p, c->st, std::min(npm, nk - p)));
-            HIPCHK(hipMemcpyAsync(ha0, c->obs.d_a0, sizeof(double) * 8 * b0 * nk, hipMemcpyDeviceToHost, c->st));
+                                    c->Lmax, c->obs.r0, c->rimed, c->obs.d_vccm, dpart, G,
+                                    da0 + (size_t)8 * b0 * p, c->st, std::min(npm, nk - p)));
+            HIPCHK(hipMemcpyAsync(ha0, da0, sizeof(double) * 8 * b0 * nk, hipMemcpyDeviceToHost, c->st));
             HIPCHK(hipStreamSynchronize(c->st));
             for (int p = 0; p < nk; p++, k0++)
                 for (int q = 0; q < 2; q++) {
