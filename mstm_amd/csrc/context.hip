@@ -368,6 +368,8 @@ static void release_spheres(mstm_hip_ctx *c)
     c->obs.a0_T = 0;
     c->obs.torder.clear();
     dfree(c->obs.d_torder);
+    dfree(c->obs.d_blk);
+    c->obs.blk_bytes = 0;
 }
 
 static void release_observables(mstm_hip_ctx *c)
@@ -387,8 +389,6 @@ static void release_observables(mstm_hip_ctx *c)
     dfree(c->obs.d_vccd);
     dfree(c->obs.d_dist);
     dfree(c->obs.d_dq);
-    dfree(c->obs.d_blk);
-    c->obs.blk_bytes = 0;
     if (c->obs.h_pin) hipHostFree(c->obs.h_pin);
     c->obs.h_pin = nullptr;
     c->obs.pin_bytes = 0;

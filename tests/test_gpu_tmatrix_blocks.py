@@ -52,3 +52,32 @@ def test_blocks_are_in_the_statistics(gpu_ctx):
     pairs = st["tmatrix_solves"] // 2
     assert pairs == sum(2 * l + 1 for l in range(1, r["T"] + 1))
     assert pairs + st["iters_fp64"] / 2 <= st["matvecs_fp64"] <= pairs + st["iters_fp64"]
+
+
+def test_blocks_give_their_work_space_back():
+    """The block work space (300 MB here) goes with the spheres it was for, so
+    that the next cluster has the room; what stays is a single pair's."""
+    import ctypes as C
+
+    from mstm_amd.solver import HipContext
+
+    ctx = HipContext(0)
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert C.CDLL(ctx.L._name).hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    try:
+        one = (np.zeros((1, 3)), np.ones(1), np.full(1, 1.5 + 0.01j), 1.0, 1e-6)
+        ctx.set_spheres(*one)
+        free0 = free()
+        ctx.set_spheres(*_cluster(200, 0.6, 0.0), 1.0, 1e-6)
+        ctx.tmatrix_solution(conveps=1e-3)
+        held = free0 - free()
+        ctx.set_spheres(*one)
+        left = free0 - free()
+        print(f"held {held >> 20} MB with the T-matrix, {left >> 20} MB after")
+        assert left < (128 << 20)
+    finally:
+        ctx.close()
