@@ -1,6 +1,6 @@
 """LU solutions whose panels end at the edges of the factorization's blocks: one
 short panel, full workgroups and panels, remainders of 256 rows and 32 columns,
-spheres of unequal order, 28 workgroups.
+spheres of unequal order, 28 and all 64 workgroups.
 
 The BiCG solution at |r|^2/|b|^2 < 1e-20 carries a relative residual of 1e-10;
 times a condition below 1e2 that is 1e-8, taken ten times wider."""
@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,x,spread,neq", [(1, 0.05, 0.0, None), (16, 1.0, 0.0, 768), (17, 0.3, 0.0, 510),
-                                            (9, 0.3, 0.0, 270), (33, 0.9, 0.7, None), (100, 2.0, 0.0, 7000)])
+                                            (9, 0.3, 0.0, 270), (33, 0.9, 0.7, None), (100, 2.0, 0.0, 7000),
+                                            (234, 2.0, 0.0, 16380)])
 def test_lu_matches_bicg(gpu_ctx, n, x, spread, neq):
     from mstm_amd import geometry as G
     from mstm_amd.solver import SOLVE_LU, SOLVE_PLAIN
