@@ -610,21 +610,29 @@ def main():
     # algorithmic bytes of one product: the minimal per-pair table (rotation
     # rows sum_n (2n+1)^2 reals + both modes' axial blocks) at the stored
     # precision for every unordered pair, plus the vectors; the tiles store
-    # and read the symmetric half of it (stored_bytes)
+    # and read triangles of it (stored_bytes)
     alg32 = npairs * full_table_bytes_per_pair(L, 4) + vec_bytes
     st32 = npairs * table_bytes_per_pair(L, 4) + vec_bytes
     cols64 = plain["tile_columns"] if plain else 2
-    alg64 = npairs * full_table_bytes_per_pair(L, 8) + cols64 * 2 * ne * 16
     if ncol == 4:
         t32 = st_lig["tile4_ms_fp32"] / st_lig["tile4_launches_fp32"]
     else:
         t32 = st_lig["tile_ms_fp32"] / max(1, st_lig["tile_launches_fp32"])
     ach32 = alg32 / (t32 * 1e-3) / 1e9
-    traffic = None
-    pmc = os.path.join(HERE, "profiles", "tile_fp32_cfg5_pmc.json")
-    if os.path.exists(pmc):
-        rec = json.load(open(pmc)).get("by_columns", {}).get(str(ncol))
-        traffic = rec["hbm_bytes_per_launch"] if rec else None
+    pmc = os.path.join(HERE, "profiles", "tile_cfg5_pmc.json")
+    pmc = json.load(open(pmc)) if os.path.exists(pmc) else {}
+
+    def counted(prec, cols):
+        """HBM bytes of a tile launch by hardware counters, for the cluster they were taken on."""
+        rec = pmc.get(prec, {}).get(str(cols)) if pmc.get("nsphere") == cl.n else None
+        return rec["hbm_bytes_per_launch"] if rec else None
+
+    def hbm_rate(prec, elem, cols, ms):
+        """GB/s of the counted bytes, or of the stored tables and the vectors where none are counted."""
+        b = counted(prec, cols) or npairs * table_bytes_per_pair(L, elem) + cols * 2 * ne * 2 * elem
+        return round(b / (ms * 1e-3) / 1e9, 1)
+
+    traffic = counted("fp32", ncol)
     fl32 = npairs * full_tile_flops_per_pair(L, ncol)
     ex32 = npairs * tile_flops_per_pair(L, ncol)
     etf = ex32 / (t32 * 1e-3) / 1e12
@@ -641,18 +649,19 @@ def main():
                       "vectors; the kernel stores and reads triangles of symmetric matrices (stored_bytes: blocks "
                       "m >= 0, half-sum/half-difference Wigner matrices, one axial block per mode), staged in LDS "
                       "once per tile step, and executes executed_flops, the achieved rate; it is bound by vector "
-                      "instruction issue (93% of a step's cycles); traffic is the measured HBM bytes; "
+                      "instruction issue (89% of the launch's cycles at four per instruction); traffic is the "
+                      "counted HBM bytes; "
                       "packed FP32 is disabled, so the FP32 vector peak is 78.6 TF/s"))
-    matvec = dict(fp32_tile_ms=round(t32, 4), fp32_columns=ncol, fp32_hbm_GBps=round(ach32, 1))
+    matvec = dict(fp32_tile_ms=round(t32, 4), fp32_columns=ncol, fp32_hbm_GBps=hbm_rate("fp32", 4, ncol, t32))
     if st_lig.get("tile_launches_fp32", 0) > 0:
         t2 = st_lig["tile_ms_fp32"] / st_lig["tile_launches_fp32"]
-        a2 = npairs * full_table_bytes_per_pair(L, 4) + 2 * 2 * ne * 8
-        matvec.update(fp32_2col_tile_ms=round(t2, 4), fp32_2col_hbm_GBps=round(a2 / (t2 * 1e-3) / 1e9, 1))
+        matvec.update(fp32_2col_tile_ms=round(t2, 4), fp32_2col_hbm_GBps=hbm_rate("fp32", 4, 2, t2))
     if plain is not None:
         t64 = plain["tile_ms_avg"]
-        matvec.update(fp64_tile_ms=round(t64, 4), fp64_columns=cols64,
-                      fp64_hbm_GBps=round(alg64 / (t64 * 1e-3) / 1e9, 1),
-                      fp64_frac=round(alg64 / (t64 * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4))
+        r64 = hbm_rate("fp64", 8, cols64, t64)
+        matvec.update(fp64_tile_ms=round(t64, 4), fp64_columns=cols64, fp64_hbm_GBps=r64,
+                      fp64_frac=round(r64 / HBM_PEAK_GBPS, 4))
+    matvec["hbm_note"] = "bytes counted by the hardware where profiles/tile_cfg5_pmc.json has them, else as stored"
 
     small = small_cluster_solve()
     print(f"[bench] 20-sphere solve: {small['s_per_solve'] * 1e3:.3f} ms", file=sys.stderr, flush=True)

@@ -1121,11 +1121,14 @@ static int bicg_block(mstm_hip_ctx *c, const BicgBlock &k, int niter, double eps
     const int n = c->neqns, np = k.np, ns = 2 * np, L = c->Lmax, K = 4;
     const int64_t V = 2 * (int64_t)c->kv_n, region = 2 * (int64_t)krylov_grid();
     const DirectOp &d = c->dop[MSTM_HIP_FP64];
+    // tile times as bicg2_dev has them: not for small clusters (200 spheres: the
+    // events cost 1.2 of 97 ms)
+    const bool timed = c->timing && c->nsph > 500;
     auto product = [&](int ncol, const double *in, double *out, const int *f, const int *gate) -> int {
         HIPCHK(launch_prep_quad<double>(in, (int)V, k.xin, ncol, f, c->nsph, c->npad, L, c->d_order, c->d_offset,
                                         c->d_an, np, c->st, gate));
         hipEvent_t e0 = nullptr, e1 = nullptr;
-        if (c->timing) {
+        if (timed) {
             e0 = next_event(c);
             e1 = next_event(c);
             hipEventRecord(e0, c->st);
