@@ -330,8 +330,10 @@ hipError_t launch_reduce_quad(const T *partial, int nparts, double *aout, int ld
     const int KS = imx(1, imn(threads / (SP * U), (nparts + 3) / 4));
     const dim3 g((nsph + SP - 1) / SP, nr / 2, nq);
     const size_t lds = sizeof(double) * (size_t)KS * SP * 8 * NB;
-#define RQ(V) \
-    hipLaunchKernelGGL((reduce_quad_kernel<T, V>), g, dim3(threads), lds, st, partial, nparts,                                                    reinterpret_cast<cplx<double> *>(aout), ldaout / 2, nrhs, flags4(flags, nrhs), nr, nsph, npad,                         Lp, SP, KS, order, offset, reinterpret_cast<const cplx<double> *>(an), gate)
+#define RQ(V)                                                                                                          \
+    hipLaunchKernelGGL((reduce_quad_kernel<T, V>), g, dim3(threads), lds, st, partial, nparts,                         \
+                       reinterpret_cast<cplx<double> *>(aout), ldaout / 2, nrhs, flags4(flags, nrhs), nr, nsph, npad,  \
+                       Lp, SP, KS, order, offset, reinterpret_cast<const cplx<double> *>(an), gate)
     if (VC == 2) RQ(2);
     else RQ((sizeof(T) == 8 ? 2 : 4));
 #undef RQ

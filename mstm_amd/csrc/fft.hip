@@ -626,7 +626,6 @@ static hipError_t fft_axis(const cplx<T> *in, cplx<T> *out, int batch, int3 din,
 // bound by the stages' butterflies (full complex products with the roots) and
 // their barriers.  Pencils of the z axis 8 / 16 / 32: 10.0 / 9.6 / 9.3 us; planes of
 // 768 / 1536 / 3072 points: 25 / 26 / 31 us.
-
 // ===========================================================================
 // x / d for x < 65536: exact with m = ceil(2^32 / d)
 struct FftDiv {

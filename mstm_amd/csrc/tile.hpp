@@ -343,18 +343,18 @@ __device__ __forceinline__ void tile_wave(int2 bt, int tile, const T *__restrict
 }
 
 // What bounds the tiles (MI355X, 5000 spheres of order 4, 12.5 M pairs):
-//   FP32, two columns: 2.77 ms.  A step is about 940 vector instructions at
-//   4.3 cycles (measured for independent FMAs at two waves per SIMD), 93% of
-//   the 4330 cycles it takes; HBM delivers 7.9 GB of tables, a third of what it
-//   could.  With the half tables of the former layout (992 bytes per pair,
+//   FP32, two columns: 2.77 ms.  A step is about 960 vector instructions: at
+//   four cycles each and 2.4 GHz they issue during 89% of the launch (counted,
+//   profiles/direct_tile_cfg5_sq_counters.txt); HBM moves 9.7 GB, 3.5 TB/s.
+//   With the half tables of the former layout (992 bytes per pair,
 //   now 624; phases applied to every coefficient) it was 3.68 ms.  The same
 //   step on v_mfma_f32_4x4x1 (one small matrix per slot) ran 3.71 ms: those
 //   MFMAs take 8.2 cycles, do not overlap with vector work and cost 8 more at
 //   every switch.
-//   FP64, two / four columns: 6.3 / 12.2 ms (8.8 / 16.0 before): one wave per
-//   SIMD, its register file and 71 KB of LDS per workgroup being full, so LDS
-//   latency shows (vector unit 50% busy, LDS 37%, a third of the cycles
-//   waiting).  Sources read from L2 with two waves per SIMD instead: 14% slower.
+//   FP64, two / four columns: 6.3 / 11.8 ms (8.8 / 16.0 before): one wave per
+//   SIMD (71 KB of LDS per workgroup of two waves), so latency shows: vector
+//   instructions issue during 41-44% of the launch, LDS is active 31-33% of it.
+//   Sources read from L2 with two waves per SIMD instead: 14% slower.
 //   FP64 orders 5..8 spill less without the register prefetch (order 6,
 //   801 spheres, four columns: 2.32 -> 1.61 ms; 20.3 ms with the full tables of
 //   the former layout).
